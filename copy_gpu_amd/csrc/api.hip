@@ -131,14 +131,20 @@ static void free_all(Engine& E)
     if (E.order_event) hipEventDestroy(E.order_event);
 }
 
-// The list build keeps the tile's reference stage and one hit buffer of cap
-// slots per wave in LDS: shrink the stage until both fit a workgroup (larger
-// tiles take the global-memory path).  False if even the smallest stage does not.
+// The list build keeps the tile's reference stage and its masks (half rows: one hit
+// buffer of cap slots per wave) in LDS: shrink the stage until both fit a workgroup
+// (larger tiles take the global-memory path).  False if even the smallest stage does
+// not.
 static bool fit_stage(Engine& E)
 {
     const size_t lim = (size_t)E.lds_max - 4096;
-    while (E.stage_cap > 64 && list_lds_bytes(E.stage_cap, E.cap, E.rbl) > lim) E.stage_cap -= 64;
-    return list_lds_bytes(E.stage_cap, E.cap, E.rbl) <= lim;
+    auto bytes = [&]() {
+        return E.half ? half_list_lds_bytes(E.stage_cap, E.cap)
+                      : list_lds_bytes(E.stage_cap, E.cap, 32, E.rbl);
+    };
+    while (E.stage_cap > 64 && bytes() > lim) E.stage_cap -= 64;
+    // rows longer than the smallest stage's hit buffers hold stay refused in both modes
+    return bytes() <= lim && half_list_lds_bytes(64, E.cap) + (E.rbl ? 1024 : 0) <= lim;
 }
 
 static int alloc_list(Engine& E, int cap)
@@ -235,7 +241,7 @@ static void half_geometry(Engine& E, int64_t n)
         return (int64_t)E.stage_cap * per + (int64_t)E.acc_cap * 24;
     };
     while (E.stage_cap > 64 && (bytes() > budget ||
-                                (int64_t)list_lds_bytes(E.stage_cap, E.cap) > budget))
+                                (int64_t)half_list_lds_bytes(E.stage_cap, E.cap) > budget))
         E.stage_cap -= 64;
     E.split = 1;
 }

@@ -118,10 +118,52 @@ __device__ inline double4 half_ref(const HalfHdr& h, const double4* __restrict__
     return make_double4(p.x - h.sx[st], p.y - h.sy[st], p.z - h.sz[st], p.w);
 }
 
+// Reference-position stage of the half rows' build: (x, y) of candidate u at xy[u], z at
+// zz[u], for u below the stage size rounded up to the sweep's kSweepLen candidates
+// (entries past the tile hold its dummy position, so the sweep needs no bounds
+// test).  The per-wave hit buffers follow (hit_buffer).
+constexpr int kSweep = 4;  // 64-candidate chunks per sweep iteration (independent chains)
+constexpr int kSweepLen = 64 * kSweep;
+__host__ __device__ inline int ref_stage_len(int stage_cap)
+{
+    return (stage_cap + kSweepLen - 1) / kSweepLen * kSweepLen;
+}
+
+struct RefStage {
+    double2* xy;
+    double* zz;
+    __device__ RefStage(double4* lds, int stage_cap)
+        : xy((double2*)lds), zz((double*)lds + 2 * (size_t)ref_stage_len(stage_cap))
+    {
+    }
+    __device__ void put(int u, const double4& p) const
+    {
+        xy[u] = make_double2(p.x, p.y);
+        zz[u] = p.z;
+    }
+    __device__ double3 get(int u) const
+    {
+        const double2 a = xy[u];
+        return make_double3(a.x, a.y, zz[u]);
+    }
+};
+
+// LDS bytes of the half rows' build: the reference stage plus one hit buffer of cap
+// uint16 per wave.
+inline size_t half_list_lds_bytes(int stage_cap, int cap)
+{
+    return 24 * (size_t)ref_stage_len(stage_cap) +
+           (size_t)kTileWaves * (size_t)cap * sizeof(uint16_t);
+}
+
+__device__ inline uint16_t* hit_buffer(double4* lds, int stage_cap, int cap, int wv)
+{
+    return (uint16_t*)((double*)lds + 3 * (size_t)ref_stage_len(stage_cap)) + (size_t)wv * cap;
+}
+
 // Half rows of the home atoms of a half tile: for the home atom at tile index ui,
 // the candidates u in (ui, total) -- the later home atoms and every forward atom --
-// with the criterion and distance convention of list_wave (tile.h); rows in the same
-// layout (LJ-range entries, the rest, the sentinel `total`).  Staged: the reference
+// with the criterion, distance convention and row layout of the full rows (tile.h).  Staged: the reference
 // stage holds the tile and its dummy up to index total.
 template <bool STAGED>
 __device__ inline void list_wave_half(const HalfHdr& h, const RefStage& rs,

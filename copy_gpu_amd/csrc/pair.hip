@@ -14,6 +14,8 @@
 // Pair displacements are FP64 differences of the staged positions (no per-pair
 // minimum image), the force maths runs in T (float or double), and cutoff
 // decisions use the FP64 squared distance.
+#include <stddef.h>
+
 #include "half.h"
 #include "kspace.h"
 #include "state.h"
@@ -482,7 +484,7 @@ __device__ inline void block_fsum(const double* fs, int lane, int wv, double* __
 }
 
 // Tile pass: one workgroup per (cell tile, part).  On a rebuild step it first
-// builds the Verlet rows of its home atoms (list_wave over the tile's reference
+// builds the Verlet rows of its home atoms (list_tile over the tile's reference
 // positions), then the pair pass: the tile's current positions are staged in
 // LDS shifted to the home cell's image, with the charge (rec_q) and the types
 // when there are several;
@@ -494,9 +496,18 @@ __device__ inline void block_fsum(const double* fs, int lane, int wv, double* __
 // the workgroup finally bins its home atoms for the next rebuild; that comes
 // last so its atomics' latency overlaps the other workgroups' pair work rather
 // than delaying this one's.
+// The FP32 pass keeps to 80 registers: three workgroups of eight waves share a CU with
+// the stage of a 5-sigma tile.
+template <typename T, bool EV>
+constexpr int tile_min_waves()
+{
+    return sizeof(T) == 4 && !EV ? 6 : 1;
+}
+
 template <typename T, bool EV, bool MULTI, bool RBL = false>
 struct TilePass {
     static constexpr int kThreads = kTileThreads;
+    static constexpr int kMinWaves = tile_min_waves<T, EV>();
     struct Args {
         PairArgs a;
         const double4* xs_ref;
@@ -506,6 +517,8 @@ struct TilePass {
         Box box;
         int stage_cap;
         double rl2, rin2;
+        float margin;   // list_margin of the cells
+        int list_rows;  // rows per mask group of the build
         PairScalars ps;
         const PairParams* pp;
         T *fx, *fy, *fz;
@@ -521,7 +534,8 @@ struct TilePass {
         const int32_t* order;  // workgroup -> cell * split + part (null: identity)
         RblArgs rbl;           // random batch list (RBL instantiation)
     };
-    __device__ static void run(const Args& A, int blk, int)
+    // self: the address of A, in constant memory
+    __device__ __forceinline__ static void run(const Args& A, int blk, int, uintptr_t self)
     {
         const PairArgs& a = A.a;
         extern __shared__ double4 lds[];
@@ -548,27 +562,22 @@ struct TilePass {
         // kernels before this one have counted the current build
         const uint32_t epoch = RBL ? (uint32_t)A.stats[0] : 0u;
         if (rebuild) {
-            if (!staged && part == 0 && threadIdx.x == 0) atomicAdd(&A.stats[6], 1ull);
-            const RefStage rs(lds, A.stage_cap);
-            int32_t* ids = RBL && staged ? stage_ids(lds, A.stage_cap, a.cap) : nullptr;
-            if (staged) {
-                for (int u = threadIdx.x; u < total; u += kTileThreads) {
-                    rs.put(u, stage_ref(h, A.xs_ref, u));
-                    if (RBL) ids[u] = tile_atom_id(h, a.perm, u);
-                }
-                const int pad = ref_stage_len(total);  // the sweep reads whole chunks
-                for (int u = total + (int)threadIdx.x; u < pad; u += kTileThreads)
-                    rs.put(u, h.dummy);
-            }
-            __syncthreads();
-            uint16_t* hb = hit_buffer(lds, A.stage_cap, a.cap, wv);
-            const RblBuild rb{A.rbl.near2, A.rbl.seed, epoch, A.rbl.pice, a.perm, ids};
-            if (staged)
-                list_wave<true, RBL>(h, rs, A.xs_ref, a0 + wv, a1, h0, lane, A.rl2, A.rin2,
-                                     a.cap, hb, A.nlist, A.ncount, A.stats, rb);
-            else
-                list_wave<false, RBL>(h, rs, A.xs_ref, a0 + wv, a1, h0, lane, A.rl2, A.rin2,
-                                      a.cap, hb, A.nlist, A.ncount, A.stats, rb);
+            const Args& R = reload<Args>(self);
+            if (!staged && part == 0 && threadIdx.x == 0) atomicAdd(&R.stats[6], 1ull);
+            const int cc = opaque(c);  // its divisions stay off the steps without a rebuild
+            const ListArgs la{R.xs_ref,
+                              R.rl2,
+                              RBL ? R.rbl.near2 : R.rin2,
+                              R.margin,
+                              {R.box.lo[0] + (cc % R.dims.x + 0.5) * R.cell.x,
+                               R.box.lo[1] + ((cc / R.dims.x) % R.dims.y + 0.5) * R.cell.y,
+                               R.box.lo[2] + (cc / (R.dims.x * R.dims.y) + 0.5) * R.cell.z},
+                              R.a.cap,
+                              R.nlist,
+                              R.ncount,
+                              R.stats};
+            const RblBuild rb{R.rbl.seed, epoch, R.rbl.pice, R.a.perm};
+            list_tile<RBL>(h, la, lds, R.stage_cap, R.list_rows, staged, a0, a1, h0, wv, lane, rb);
             __syncthreads();  // rows and LDS are reused below
         }
         if (staged) {
@@ -837,7 +846,7 @@ struct TilePassHalf {
         HalfPlanes planes;
         int acc_cap;
     };
-    __device__ static void run(const Args& AH, int blk, int)
+    __device__ __forceinline__ static void run(const Args& AH, int blk, int)
     {
         const auto& A = AH.t;
         const PairArgs& a = A.a;
@@ -1025,20 +1034,21 @@ struct TileRhoHalf {
 template <typename T, bool EV, bool M, bool RBL = false>
 struct TileRho {
     static constexpr int kThreads = kTileThreads;
+    static constexpr int kMinWaves = tile_min_waves<T, EV>();
     struct Args {
         typename RhoFinalT<T, kTileThreads>::Args fin;
         int nfin, ntile;
         int fin_first;
         typename TilePass<T, EV, M, RBL>::Args tile;
     };
-    __device__ static void run(const Args& A, int blk, int)
+    __device__ __forceinline__ static void run(const Args& A, int blk, int, uintptr_t self)
     {
         const int t = A.fin_first ? blk - A.nfin : blk;
         if (t < 0 || t >= A.ntile) {
             RhoFinalT<T, kTileThreads>::run(A.fin, A.fin_first ? blk : blk - A.ntile, A.nfin);
             return;
         }
-        TilePass<T, EV, M, RBL>::run(A.tile, t, A.ntile);
+        TilePass<T, EV, M, RBL>::run(A.tile, t, A.ntile, self + offsetof(Args, tile));
     }
 };
 
@@ -1129,6 +1139,16 @@ PairScalars pair_scalars(const Engine& e)
     return ps;
 }
 
+// LDS of the pair pass's stage, and the rows of a list-build mask group beside it.
+size_t pair_stage_bytes(const Engine& e)
+{
+    return (size_t)e.stage_cap * (sizeof(double4) + (e.pp.ntypes > 1 ? 4 : 0));
+}
+int pair_list_rows(const Engine& e)
+{
+    return list_rows(e.stage_cap, e.cap, pair_stage_bytes(e), e.rbl);
+}
+
 template <typename T, bool EV, bool M, bool RBL = false>
 typename TilePass<T, EV, M, RBL>::Args tile_args(Engine& e, void* fx, void* fy, void* fz,
                                                  bool md)
@@ -1145,7 +1165,7 @@ typename TilePass<T, EV, M, RBL>::Args tile_args(Engine& e, void* fx, void* fy, 
     return typename TilePass<T, EV, M, RBL>::Args{
         PairArgs{e.xs, e.ts, e.perm, e.nlist, e.ncount, e.cap},
         e.xs_ref, e.cell_start, e.split, make_int3(e.dims[0], e.dims[1], e.dims[2]), e.box,
-        e.stage_cap, e.r_list * e.r_list, e.r_in * e.r_in, pair_scalars(e), e.d_pp, (T*)fx,
+        e.stage_cap, e.r_list * e.r_list, e.r_in * e.r_in, list_margin(e.cell), pair_list_rows(e), pair_scalars(e), e.d_pp, (T*)fx,
         (T*)fy, (T*)fz, e.ev_part, e.flags, e.stats, e.nlist, e.ncount, e.cell_count,
         md ? 1 : 0, make_double3(e.cell[0], e.cell[1], e.cell[2]), md_bins(e),
         tile_order_ncu(e.ncell, e.split, e.num_cu) > 0 ? e.tile_order : nullptr, rbl};
@@ -1153,8 +1173,8 @@ typename TilePass<T, EV, M, RBL>::Args tile_args(Engine& e, void* fx, void* fy, 
 
 size_t pair_lds(const Engine& e)
 {
-    const size_t stage = (size_t)e.stage_cap * (sizeof(double4) + (e.pp.ntypes > 1 ? 4 : 0));
-    const size_t build = list_lds_bytes(e.stage_cap, e.cap, e.rbl);
+    const size_t stage = pair_stage_bytes(e);
+    const size_t build = list_lds_bytes(e.stage_cap, e.cap, pair_list_rows(e), e.rbl);
     return stage > build ? stage : build;
 }
 
@@ -1164,7 +1184,7 @@ size_t half_lds(const Engine& e)
 {
     const size_t pass = (size_t)e.stage_cap * sizeof(double4) + (size_t)e.acc_cap * 24 +
                         (e.pp.ntypes > 1 ? (size_t)e.stage_cap * 4 : 0);
-    const size_t build = list_lds_bytes(e.stage_cap, e.cap);
+    const size_t build = half_list_lds_bytes(e.stage_cap, e.cap);
     return pass > build ? pass : build;
 }
 

@@ -9,6 +9,8 @@
 // Each stencil cell carries the periodic image shift s (k L, k in {-1,0,1})
 // such that x_j - s is the image of x_j next to the home cell.
 #pragma once
+#include <type_traits>
+
 #include "engine.h"
 
 namespace rbmd {
@@ -250,16 +252,38 @@ __device__ inline int tile_seg(const TileHdr& h, int u)
     return lo;
 }
 // ---------------------------------------------------------------- Verlet list
-// One workgroup per (home cell, part): the tile's reference positions are
-// staged in LDS already moved to the home cell's image, x_j - s (s the image
-// shift of j's stencil cell), then one wave per home atom i sweeps the whole
-// tile, kSweep chunks of 64 candidates per iteration.  A candidate is kept iff
-// (r_list^2 - d2 > 1e-4) && (d2 > 1e-4) with dx = (x_j - s) - x_i and
+// One workgroup per (home cell, part) builds the rows of its home atoms.  A
+// candidate j of home atom i is kept iff (r_list^2 - d2 > 1e-4) && (d2 > 1e-4) with
+// dx = (x_j - s) - x_i (s the image shift of j's stencil cell) and
 // d2 = fma(dz,dz, fma(dy,dy, dx*dx)) -- the reference's operation order
-// (RunWorklet.cpp:77-83) and the exact bits the CPU oracle uses.  The stage is
-// two arrays, (x, y) pairs then z, so the sweep's consecutive reads are
-// bank-conflict-free.  Tiles larger than the LDS stage read candidates from
-// global memory; tiles beyond the 15-bit index range mark their rows overflowed.
+// (RunWorklet.cpp:77-83) and the exact bits the CPU oracle uses.
+//
+// Testing every candidate of every home atom that way costs about 25 VALU
+// instructions per 64 pairs, and 85% of the pairs miss.  So the squared distances are
+// formed on the matrix cores in FP32, |j|^2 - 2 i.j + (|i|^2 - t) for 16 home atoms x
+// 16 candidates per v_mfma_f32_16x16x4_f32 (positions relative to the home cell's
+// centre): the sign bits are the hits, and those of the same values moved to the
+// LJ range are its entries.  Rows with a value within rounding (list_margin) of a
+// threshold (about 1% of them) are built by the exact criterion instead, so the rows
+// hold exactly the pairs that it accepts.
+//
+// Steps, per block of up to 4096 candidates staged in LDS (float4: position and
+// |j|^2):
+//   near_masks  the 8 waves share the 16-candidate chunks (wave w: chunks w T ..
+//               w T + T - 1); each lane keeps one bit per chunk for its four rows of
+//               every 16-row tile and stores them to LDS: 64 words per row and mask
+//   row_hits    one wave per row: lane (g, column) holds the column's bits of waves 2g
+//               and 2g + 1, and the wave writes one hit of every lane per trip
+// A row's consecutive entries then come from different columns (u mod 16), and the
+// pair pass, which gathers 16 consecutive entries at a time, reads different LDS banks.
+// Tiles larger than the LDS stage are staged block by block.  Tiles beyond the 15-bit
+// index range mark their rows overflowed.
+//
+// Bound by VALU issue: at 100,000 ions (1,229 candidates a tile, 45 rows) staging takes
+// 6 us, the masks 28 us and the rows 49 us of a rebuild's tile pass.  Against one wave per
+// row testing every candidate in FP64: 150 -> 134 us (the whole pass, the pair part 46 of
+// it), 2,574 -> 2,136 us at 1,048,576 ions, and 6.6 -> 2.0 ms where the tile is staged in
+// blocks (1,000 ions in a box of one cell, 27,000 candidates).
 //
 // Row layout (uint16 tile-local indices, cap slots per home atom): the LJ-range
 // entries (d2 < r_in^2) first, then the others, then one sentinel slot holding
@@ -267,10 +291,6 @@ __device__ inline int tile_seg(const TileHdr& h, int u)
 // clamp its slot to the row length instead of testing it.  A row of n entries
 // needs n + 1 <= cap slots; ncount = (LJ-range, other) entries, or (n, 0) with
 // n >= cap for a row that did not fit.
-//
-// The sweep compacts hits with one ballot + mbcnt into this wave's LDS hit
-// buffer (cap entries, LJ-range hits tagged with kInnerFlag), then one pass
-// over the buffer writes the row in its final order.
 constexpr int kInnerFlag = 0x8000;
 constexpr int kMaxTile = 0x7fff;  // tile-local indices and the sentinel fit in 15 bits
 
@@ -282,54 +302,59 @@ __device__ inline double4 stage_ref(const TileHdr& h, const double4* __restrict_
     return make_double4(p.x - h.sx[st], p.y - h.sy[st], p.z - h.sz[st], p.w);
 }
 
-// Reference-position stage of list_wave: (x, y) of candidate u at xy[u], z at
-// zz[u], for u below the stage size rounded up to the sweep's kSweepLen candidates
-// (entries past the tile hold its dummy position, so the sweep needs no bounds
-// test).  The per-wave hit buffers follow (hit_buffer).
-constexpr int kSweep = 4;  // 64-candidate chunks per sweep iteration (independent chains)
-constexpr int kSweepLen = 64 * kSweep;
-__host__ __device__ inline int ref_stage_len(int stage_cap)
+constexpr int kListBlock = 4096;  // most candidates of one block (32 chunks per wave)
+constexpr int kMaskRow = 256;     // bytes of a row's mask (64 uint32 words)
+
+// Staged candidates of a build: whole 16-candidate chunks.
+__host__ __device__ inline int list_len(int stage_cap) { return (stage_cap + 15) / 16 * 16; }
+
+// Rows of one mask group (a multiple of 16): as many as fit beside the candidates in
+// the LDS that the pair pass's stage takes anyway (pass_bytes), between 32 and 64.
+inline size_t list_fixed_bytes(int stage_cap, int cap, bool rbl)
 {
-    return (stage_cap + kSweepLen - 1) / kSweepLen * kSweepLen;
+    return (size_t)(rbl ? 20 : 16) * (size_t)list_len(stage_cap) +
+           (size_t)kTileWaves * (size_t)cap * sizeof(uint16_t);
+}
+inline int list_rows(int stage_cap, int cap, size_t pass_bytes, bool rbl)
+{
+    const size_t c = list_fixed_bytes(stage_cap, cap, rbl);
+    const size_t fit = pass_bytes > c ? (pass_bytes - c) / (2 * kMaskRow) : 0;
+    return fit >= 64 ? 64 : fit < 48 ? 32 : 48;
 }
 
-struct RefStage {
-    double2* xy;
-    double* zz;
-    __device__ RefStage(double4* lds, int stage_cap)
-        : xy((double2*)lds), zz((double*)lds + 2 * (size_t)ref_stage_len(stage_cap))
+// LDS bytes of the list build: the candidates (and, for a random batch list, their atom
+// ids), a row buffer of cap entries per wave and two masks of `rows` rows.
+inline size_t list_lds_bytes(int stage_cap, int cap, int rows = 32, bool rbl = false)
+{
+    return list_fixed_bytes(stage_cap, cap, rbl) + 2 * kMaskRow * (size_t)rows;
+}
+
+struct ListLds {
+    float4* cand;    // [list_len]
+    char* mask;      // two masks, mask_bytes apart: hits, then their LJ-range ones
+    int mask_bytes;
+    uint16_t* buf;   // this wave's row buffer [cap]
+    int32_t* ids;    // random batch list: [list_len] atom ids
+    __device__ ListLds(double4* lds, int stage_cap, int cap, int rows, int wv)
     {
-    }
-    __device__ void put(int u, const double4& p) const
-    {
-        xy[u] = make_double2(p.x, p.y);
-        zz[u] = p.z;
-    }
-    __device__ double3 get(int u) const
-    {
-        const double2 a = xy[u];
-        return make_double3(a.x, a.y, zz[u]);
+        cand = (float4*)lds;
+        mask = (char*)(cand + list_len(stage_cap));
+        mask_bytes = kMaskRow * rows;
+        uint16_t* b = (uint16_t*)(mask + 2 * mask_bytes);
+        buf = b + (size_t)wv * cap;
+        ids = (int32_t*)(b + (size_t)kTileWaves * cap);
     }
 };
 
-// LDS bytes of the list build: the reference stage plus one hit buffer of cap
-// uint16 per wave (and, for a random batch list, the candidates' atom ids).
-inline size_t list_lds_bytes(int stage_cap, int cap, bool rbl = false)
+// Bound of the rounding of near_masks' squared distances: candidates lie within 1.5
+// cells per axis of the centre (R^2 the square of that corner), and with u = 2^-24 the
+// rounded positions, products and five-term sums add up to less than 27 u R^2;
+// 2^-19 R^2 = 32 u R^2.
+inline float list_margin(const double cell[3])
 {
-    return 24 * (size_t)ref_stage_len(stage_cap) +
-           (size_t)kTileWaves * (size_t)cap * sizeof(uint16_t) +
-           (rbl ? 4 * (size_t)ref_stage_len(stage_cap) : 0);
-}
-
-__device__ inline uint16_t* hit_buffer(double4* lds, int stage_cap, int cap, int wv)
-{
-    return (uint16_t*)((double*)lds + 3 * (size_t)ref_stage_len(stage_cap)) + (size_t)wv * cap;
-}
-
-// Atom ids of the staged candidates (random batch list builds), after the hit buffers.
-__device__ inline int32_t* stage_ids(double4* lds, int stage_cap, int cap)
-{
-    return (int32_t*)(hit_buffer(lds, stage_cap, cap, kTileWaves));
+    double r2 = 0.0;
+    for (int d = 0; d < 3; ++d) r2 += 2.25 * cell[d] * cell[d];
+    return (float)(r2 * 1.9073486328125e-6);
 }
 
 // Random batch list of a build: rows keep every pair closer than r_near = r_core +
@@ -337,12 +362,10 @@ __device__ inline int32_t* stage_ids(double4* lds, int stage_cap, int cap)
 // rbl_select keeps, tagged with kRblSel so the pair pass weights them.
 constexpr int kRblSel = 0x8000;
 struct RblBuild {
-    double near2;      // (r_core + skin)^2
     uint64_t seed;
     uint32_t epoch;    // list build number
     uint32_t pice;
     const int32_t* perm;  // sorted slot -> atom id
-    const int32_t* ids;   // LDS: atom id of each staged candidate (null: from perm)
 };
 
 // Atom id of tile-local candidate u (random batch list builds and their fallback).
@@ -352,125 +375,406 @@ __device__ inline int32_t tile_atom_id(const TileHdr& h, const int32_t* __restri
     return perm[h.gstart[st] + (u - h.off[st])];
 }
 
-template <bool STAGED, bool RBL = false>
-__device__ inline void list_wave(const TileHdr& h, const RefStage& rs,
-                                 const double4* __restrict__ xs_ref, int first, int a1, int h0,
-                                 int lane, double rl2, double rin2, int cap, uint16_t* hb,
-                                 uint16_t* __restrict__ nlist, int2* __restrict__ ncount,
-                                 unsigned long long* __restrict__ stats,
-                                 const RblBuild& rb = RblBuild{})
+// The same value, unknown to the compiler: keeps what is computed from it inside the
+// phase that uses it, where hoisting it over the whole build would cost registers that the
+// pair pass's occupancy does not have.
+__device__ inline int opaque(int v)
 {
-#pragma clang fp contract(off)
-    const int total = h.off[27];
-    for (int s = first; s < a1; s += kTileWaves) {
-        if (total >= kMaxTile) {
-            if (lane == 0) {
-                ncount[s] = make_int2(cap + 1, 0);
-                atomicAdd(&stats[2], 1ull);
-                atomicMax(&stats[4], (unsigned long long)(cap + 1));
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+struct ListArgs {
+    const double4* xs_ref;
+    double rl2, tag2;  // r_list^2; LJ range (full list) or the always-kept near band (RBL)
+    float margin;      // list_margin
+    double ctr[3];     // centre of the home cell
+    int cap;
+    uint16_t* nlist;
+    int2* ncount;
+    unsigned long long* stats;
+};
+
+typedef float list_f4 __attribute__((ext_vector_type(4)));
+
+// FP32 position relative to the home cell's centre, its square in w.
+__device__ inline float4 list_pos(const ListArgs& A, double x, double y, double z)
+{
+    const float a = (float)(x - A.ctr[0]), b = (float)(y - A.ctr[1]), c = (float)(z - A.ctr[2]);
+    return make_float4(a, b, c, fmaf(c, c, fmaf(b, b, a * a)));
+}
+
+// The home rows of one near_masks call: NMT 16-row tiles, rows [0, nrow) being home
+// atoms s0 + row, tile index u0 + row relative to the staged block.
+struct MaskRows {
+    const float4* home;  // staged positions of the rows, or null: from xs_ref
+    int s0, u0, nrow;
+};
+
+// Masks of NMT x 16 rows against the nch chunks of the staged block.  Word of (row,
+// wave pair, column): the pair's 2T chunks, the first in bit 2T - 1 (W: uint32 for
+// T <= 16, else uint64, built in two halves).  slow: bit per row.  Per 256 pairs 32 cycles
+// of a SIMD's matrix core and 18 VALU instructions (two sign bits, the LJ-range shift
+// and the smallest distances from the thresholds).
+template <int NMT, typename H>
+__device__ inline void near_masks(const ListArgs& a, const float4* cand, const MaskRows& R,
+                                  const ListLds& L, unsigned long long* slow, int row0, int nch,
+                                  int T, int wv, int lane_in)
+{
+    const int lane = opaque(lane_in), col = lane & 15, q = lane >> 4;
+    const int tw = min(T, nch - wv * T);
+    const float t0 = (float)(a.rl2 - 1e-4);         // d = d2 - t0
+    const float tin = (float)(a.rl2 - 1e-4 - a.tag2);  // d + tin = d2 - tag2
+    float av[NMT], near[NMT], dmin = 3.0e38f;
+    list_f4 c[NMT];
+    uint32_t hit[NMT][4], in[NMT][4];
+#pragma unroll
+    for (int m = 0; m < NMT; ++m) {
+        const int ra = min(16 * m + col, R.nrow - 1);
+        float4 f;
+        if (R.home) {
+            f = R.home[ra];
+        } else {
+            const double4 p = a.xs_ref[R.s0 + ra];
+            f = list_pos(a, p.x, p.y, p.z);
+        }
+        const float fq = q == 0 ? f.x : q == 1 ? f.y : f.z;
+        av[m] = q == 3 ? 1.0f : -2.0f * fq;
+        // rows past the last: far from everything
+        const float w = 16 * m + col < R.nrow ? f.w - t0 : 1.0e30f;
+        near[m] = 3.0e38f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            c[m][r] = __shfl(w, 4 * q + r, 64);
+            hit[m][r] = in[m][r] = 0u;
+        }
+    }
+    const float* b0 = (const float*)cand + 4 * (16 * wv * T + col) + q;
+    float bn = tw > 0 ? b0[0] : 0.0f;
+    for (int t = 0; t < tw; ++t) {
+        const float bv = bn;
+        bn = b0[64 * min(t + 1, tw - 1)];
+        list_f4 d[NMT];
+#pragma unroll
+        for (int m = 0; m < NMT; ++m)
+            d[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[m], bv, c[m], 0, 0, 0);
+        const int uc = 16 * (wv * T + t);
+        if (uc + 15 >= R.u0 && uc < R.u0 + R.nrow) {
+            // the rows themselves: not their own neighbours
+#pragma unroll
+            for (int m = 0; m < NMT; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (uc + col == R.u0 + 16 * m + 4 * q + r) d[m][r] = 1.0e30f;
+        }
+#pragma unroll
+        for (int m = 0; m < NMT; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float x = d[m][r], y = x + tin;
+                hit[m][r] = __builtin_amdgcn_alignbit(hit[m][r], __float_as_uint(x), 31);
+                in[m][r] = __builtin_amdgcn_alignbit(in[m][r], __float_as_uint(y), 31);
+                near[m] = fminf(fminf(near[m], fabsf(x)), fabsf(y));
+                dmin = fminf(dmin, x);
             }
+    }
+    const int sh = T - (tw > 0 ? tw : 0);
+    const bool tiny = dmin < 2e-4f - t0 + a.margin;  // d2 within rounding of 1e-4
+#pragma unroll
+    for (int m = 0; m < NMT; ++m) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = row0 + 16 * m + 4 * q + r;
+            // a word's two halves: waves 2g (high) and 2g + 1 (low)
+            H* w = (H*)L.mask + (((row * 4 + (wv >> 1)) * 16 + col) * 2 + (1 - (wv & 1)));
+            w[0] = tw > 0 ? (H)(hit[m][r] << sh) : (H)0;
+            w[L.mask_bytes / (int)sizeof(H)] = tw > 0 ? (H)(in[m][r] << sh) : (H)0;
+        }
+        if (near[m] < a.margin || tiny) {
+            const int row = row0 + 16 * m + 4 * q;
+            atomicOr(slow, 0xfull << row);
+        }
+    }
+}
+
+// Wave sum of an int, uniform.
+__device__ inline int wave_sum_int(int v)
+{
+    v += dpp_i<0xB1>(v);
+    v += dpp_i<0x4E>(v);
+    v += dpp_i<0x141>(v);
+    v += dpp_i<0x140>(v);
+    v += dpp_i<0x142, 0xa>(v);
+    v += dpp_i<0x143, 0xc>(v);
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Number of leading zero bits of a non-zero word.
+__device__ inline int lead0(uint32_t v) { return __clz((int)v); }
+__device__ inline int lead0(uint64_t v) { return __clzll((long long)v); }
+
+// One wave: the hits of row `row` (home atom s, tile index ui) in the staged block,
+// whose first candidate is tile index cb.  SINGLE: the block is the whole tile and the
+// row collects in the wave's LDS buffer; else over the blocks in its slots in global
+// memory.  It collects from both ends, the LJ-range entries at the front and the others
+// at the back, unless their counts are known first.  have: entries that earlier blocks
+// gave the row.  The last block writes the row.
+template <bool RBL, typename W, bool SINGLE>
+__device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListLds& L, int row,
+                                int s, int ui, const float4* cand, const float4* home, int cb,
+                                int cn, const int32_t* ids, int T, int lane_in, bool last,
+                                bool slow, int2 have, const RblBuild& rb)
+{
+    const int lane = opaque(lane_in);
+    const int cap = a.cap, total = h.off[27];
+    const int g = lane >> 4, col = lane & 15;
+    uint16_t* __restrict__ rowp = a.nlist + (size_t)s * cap;
+    const int32_t id_i = RBL ? rb.perm[s] : 0;
+    int ci = have.x, co = have.y;
+    auto put1 = [&](int k, int u) {
+        if (SINGLE) L.buf[k] = (uint16_t)u;
+        else rowp[k] = (uint16_t)u;
+    };
+    // one entry per lane with `keep`: LJ range (and, for a random batch list, every
+    // kept pair) at the front, else at the back
+    auto put = [&](bool keep, bool front, int u, int base) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(keep);
+        const int k = base + (int)mbcnt64(m);
+        if (keep && k < cap) put1(front ? k : cap - 1 - k, u);
+        return __popcll(m);
+    };
+    bool ordered = RBL;  // the others already stand behind the LJ range
+    if (!slow) {
+        constexpr int kBits = 8 * sizeof(W);
+        const int wo = (row * 4 + g) * 16 + col;
+        W m, mi;
+        {
+            // the halves T bits wide, joined; the first chunk in the top bit
+            using H = typename std::conditional<sizeof(W) == 4, uint16_t, uint32_t>::type;
+            const H* p = (const H*)L.mask + 2 * wo;
+            const H* pi = p + L.mask_bytes / (int)sizeof(H);
+            m = (((W)p[1] << T) | (W)p[0]) << (kBits - 2 * T);
+            mi = (((W)pi[1] << T) | (W)pi[0]) << (kBits - 2 * T);
+        }
+        W mo = m & ~mi;
+        mi &= m;
+        const int ub = cb + 32 * g * T + col;
+        const W top = (W)1 << (kBits - 1);
+        if (RBL) {
+            // every hit draws its selection: a near-band entry kept for being near counts
+            // only if selected should it lie in the shell when evaluated
+            while (__builtin_amdgcn_ballot_w64(m != 0) != 0ull) {
+                const bool act = m != 0;
+                const int z = act ? lead0(m) : 0;
+                const W bit = top >> z;
+                const int u = ub + 16 * z;
+                bool sel = false;
+                if (act) sel = rbl_select(rb.seed, rb.epoch, id_i, ids[u - cb], rb.pice);
+                ci += put(act && ((mi & bit) != 0 || sel), true, sel ? (u | kRblSel) : u, ci);
+                m &= ~bit;
+            }
+        } else {
+            // the row's counts first: a row that fits is written without tests, one that
+            // does not is only counted
+            int pc = sizeof(W) == 4 ? __popc((uint32_t)mi) | (__popc((uint32_t)mo) << 16)
+                                    : __popcll(mi) | (__popcll(mo) << 16);
+            pc = wave_sum_int(pc);
+            const int ni = pc & 0xffff, no = pc >> 16;
+            if (ci + co + ni + no < cap) {
+                // each trip writes the next hit of every lane that has one
+                auto expand = [&](W w, int k0, bool back) {
+                    while (w != 0) {
+                        const uint64_t act = __builtin_amdgcn_ballot_w64(true);
+                        const int k = (int)__builtin_amdgcn_mbcnt_hi(
+                            (uint32_t)(act >> 32),
+                            __builtin_amdgcn_mbcnt_lo((uint32_t)act, (uint32_t)k0));
+                        const int z = lead0(w);
+                        put1(back ? cap - 1 - k : k, ub + 16 * z);
+                        w ^= top >> z;
+                        k0 += __popcll(act);
+                    }
+                };
+                expand(mi, ci, false);
+                expand(mo, SINGLE ? ni : co, !SINGLE);
+                ordered = SINGLE;
+            }
+            ci += ni;
+            co += no;
+        }
+    } else {
+        // some candidate within rounding of a threshold: every candidate's FP32 distance
+        // (as differences, off by at most 13 u R^2) and the exact criterion for those near
+        // a threshold
+        float4 pi;
+        if (home) {
+            pi = home[row];
+        } else {
+            const double4 p = a.xs_ref[s];
+            pi = list_pos(a, p.x, p.y, p.z);
+        }
+        const float thr = (float)(a.rl2 - 1e-4), tag = (float)a.tag2;
+        for (int k0 = 0; k0 < cn; k0 += 64) {
+            const int k = min(k0 + lane, cn - 1), u = cb + k;
+            const float4 pj = cand[k];
+            const float fx = pj.x - pi.x, fy = pj.y - pi.y, fz = pj.z - pi.z;
+            const float f2 = fmaf(fz, fz, fmaf(fy, fy, fx * fx));
+            const bool live = k0 + lane < cn && u != ui;
+            bool hit = live && f2 < thr, in = f2 < tag;
+            const bool near = live && (fabsf(f2 - thr) < a.margin || fabsf(f2 - tag) < a.margin ||
+                                       f2 < 1e-4f + a.margin);
+            if (near) {
+#pragma clang fp contract(off)
+                const double4 e = stage_ref(h, a.xs_ref, u), pd = a.xs_ref[s];
+                const double dx = e.x - pd.x, dy = e.y - pd.y, dz = e.z - pd.z;
+                const double d2 = fma(dz, dz, fma(dy, dy, dx * dx));
+                hit = (a.rl2 - d2) > 1e-4 && d2 > 1e-4;
+                in = d2 < a.tag2;
+            }
+            if (RBL) {
+                bool sel = false;
+                if (hit) sel = rbl_select(rb.seed, rb.epoch, id_i, ids[u - cb], rb.pice);
+                ci += put(hit && (in || sel), true, sel ? (u | kRblSel) : u, ci);
+            } else {
+                ci += put(hit && in, true, u, ci);
+                co += put(hit && !in, false, u, co);
+            }
+        }
+    }
+    if (!last) return make_int2(ci, co);
+    const int n = ci + co;
+    if (n < cap) {
+        __syncwarp();
+        if (!SINGLE) {
+            // the row from global memory into the buffer, in order
+            __threadfence_block();
+            for (int k = lane; k < n; k += 64)
+                L.buf[k] = rowp[k < ci || ordered ? k : cap - 1 - (k - ci)];
+        } else if (!ordered) {
+            // close the gap between the LJ range and the others: the last of them move
+            // into it (the source starts at or behind the gap's end)
+            const int cnt = min(co, cap - n);
+            for (int k = lane; k < cnt; k += 64) L.buf[ci + k] = L.buf[cap - cnt + k];
+        }
+        __syncwarp();
+        // two entries per 32-bit word (rows start at multiples of 64 entries)
+        if (lane == 0) L.buf[n] = (uint16_t)total;
+        __syncwarp();
+        for (int k = lane; 2 * k <= n; k += 64)
+            ((uint32_t*)rowp)[k] = ((const uint32_t*)L.buf)[k];
+        __syncwarp();  // the buffer is reused for the wave's next row
+    }
+    if (lane == 0) {
+        a.ncount[s] = n < cap ? make_int2(ci, co) : make_int2(n, 0);
+        if (n >= cap) {
+            atomicAdd(&a.stats[2], 1ull);
+            atomicMax(&a.stats[4], (unsigned long long)(n + 1));
+        }
+    }
+    return make_int2(ci, co);
+}
+
+// LDS of the build besides the stage: entries per row over the blocks of one tile,
+// and the rows to build by the exact criterion.
+struct ListRows {
+    int2 cnt[64];
+    unsigned long long slow;
+};
+
+// One block of the build: masks, then rows, for the row group [0, nrow) of home atoms
+// s0.. (tile index u0..).
+template <bool RBL, typename W>
+__device__ inline void list_block(const TileHdr& h, const ListArgs& a, const ListLds& L,
+                                  ListRows& lr, const float4* cand, const float4* home,
+                                  const int32_t* ids, int cb, int cn, int s0, int u0, int nrow,
+                                  bool single, bool last, int wv, int lane, const RblBuild& rb)
+{
+    using H = typename std::conditional<sizeof(W) == 4, uint16_t, uint32_t>::type;
+    const int nch = (cn + 15) / 16, T = (nch + kTileWaves - 1) / kTileWaves;
+    // A row or two per wave of a small tile: the wave sweeps the candidates itself.  The
+    // sweep takes about cn / 2 VALU instructions a row; the masks about cn / 3 + 100 a wave,
+    // 185 a row and a barrier.
+    const bool sweep = nrow <= kTileWaves ? cn < 2048 : nrow <= 2 * kTileWaves && cn < 704;
+    // 32 rows at a time: more row tiles would take the tile pass past the registers
+    // that its LDS stage's occupancy allows
+    for (int r0 = 0; r0 < nrow && !sweep; r0 += 32) {
+        const MaskRows R{home ? home + r0 : nullptr, s0 + r0, u0 + r0 - cb, min(32, nrow - r0)};
+        if (R.nrow > 16) near_masks<2, H>(a, cand, R, L, &lr.slow, r0, nch, T, wv, lane);
+        else near_masks<1, H>(a, cand, R, L, &lr.slow, r0, nch, T, wv, lane);
+    }
+    if (!sweep) __syncthreads();
+    const uint32_t slow[2] = {sweep ? ~0u : (uint32_t)uniform((int)(uint32_t)lr.slow),
+                              sweep ? ~0u : (uint32_t)uniform((int)(uint32_t)(lr.slow >> 32))};
+    for (int row = wv; row < nrow; row += kTileWaves) {
+        const bool sl = ((row < 32 ? slow[0] : slow[1]) >> (row & 31)) & 1u;
+        if (single) {
+            row_hits<RBL, W, true>(h, a, L, row, s0 + row, u0 + row, cand, home, cb, cn, ids, T,
+                                   lane, true, sl, make_int2(0, 0), rb);
             continue;
         }
-        const int ui = h.off[kHomeSeg] + (s - h0);
-        double3 pi;
-        if (STAGED) {
-            pi = rs.get(ui);
-        } else {
-            const double4 p = xs_ref[s];
-            pi = make_double3(p.x, p.y, p.z);
+        const int2 n = row_hits<RBL, W, false>(h, a, L, row, s0 + row, u0 + row, cand, home, cb, cn,
+                                               ids, T, lane, last, sl,
+                                               cb > 0 ? lr.cnt[row] : make_int2(0, 0), rb);
+        if (!last && lane == 0) lr.cnt[row] = n;
+    }
+    __syncthreads();
+}
+
+// Rows of the home atoms [a0, a1) of a tile (every thread of the workgroup).  staged:
+// the whole tile fits the LDS stage.
+template <bool RBL>
+__device__ inline void list_tile(const TileHdr& h, const ListArgs& a, double4* lds, int stage_cap,
+                                 int rows, bool staged, int a0, int a1, int h0, int wv, int lane,
+                                 const RblBuild& rb)
+{
+    __shared__ ListRows lr;
+    const int total = h.off[27];
+    if (total >= kMaxTile) {
+        for (int s = a0 + (int)threadIdx.x; s < a1; s += kTileThreads) {
+            a.ncount[s] = make_int2(a.cap + 1, 0);
+            atomicAdd(&a.stats[2], 1ull);
+            atomicMax(&a.stats[4], (unsigned long long)(a.cap + 1));
         }
-        int n = 0;
-        for (int ub = 0; ub < total; ub += kSweepLen) {
-            double3 pj[kSweep];
-#pragma unroll
-            for (int k = 0; k < kSweep; ++k) {
-                const int u = ub + 64 * k + lane;
-                const int uu = STAGED || u < total ? u : 0;
-                if (STAGED) {
-                    pj[k] = rs.get(uu);
-                } else {
-                    const double4 p = stage_ref(h, xs_ref, uu);
-                    pj[k] = make_double3(p.x, p.y, p.z);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < kSweep; ++k) {
-                const int u = ub + 64 * k + lane;
-                const double dx = pj[k].x - pi.x;
-                const double dy = pj[k].y - pi.y;
-                const double dz = pj[k].z - pi.z;
-                const double d2 = fma(dz, dz, fma(dy, dy, dx * dx));
-                // staged: padding entries past the tile are far, so they miss
-                const bool live = STAGED || u < total;
-                const bool hit = live && ((rl2 - d2) > 1e-4) && (d2 > 1e-4);
-                // the same mask as ballot(hit), formed from the compare masks
-                // directly (no per-lane boolean round trip)
-                const uint64_t mh = __builtin_amdgcn_ballot_w64(live) &
-                                    __builtin_amdgcn_ballot_w64((rl2 - d2) > 1e-4) &
-                                    __builtin_amdgcn_ballot_w64(d2 > 1e-4);
-                const int slot = n + (int)mbcnt64(mh);
-                // tag: LJ range (full list) or the always-kept near band (random batch)
-                const double tag2 = RBL ? rb.near2 : rin2;
-                if (hit && slot < cap) hb[slot] = (uint16_t)(d2 < tag2 ? (u | kInnerFlag) : u);
-                n += __popcll(mh);
+        return;
+    }
+    const ListLds L(lds, stage_cap, a.cap, rows, wv);
+    // candidates [cb, cb + cn) into LDS, padded to whole chunks with points far from
+    // every row
+    auto stage = [&](int cb, int cn) {
+        const int pad = (cn + 15) / 16 * 16;
+        for (int k = opaque(threadIdx.x); k < pad; k += kTileThreads) {
+            if (k < cn) {
+                const double4 p = stage_ref(h, a.xs_ref, cb + k);
+                L.cand[k] = list_pos(a, p.x, p.y, p.z);
+                if (RBL) L.ids[k] = tile_atom_id(h, rb.perm, cb + k);
+            } else {
+                L.cand[k] = make_float4(0.0f, 0.0f, 0.0f, 1.0e30f);
             }
         }
-        uint16_t* __restrict__ row = nlist + (size_t)s * cap;
-        int n_in = n;
-        if (RBL && n < cap) {
-            // random batch list: the near band, and the shell pairs this list build
-            // selects (tagged kRblSel), in sweep order; the pair pass evaluates LJ on
-            // every entry
-            __syncwarp();
-            const int32_t id_i = rb.perm[s];
-            int nk = 0;
-            for (int k0 = 0; k0 < n; k0 += 64) {
-                const int k = k0 + lane;
-                const int e = k < n ? (int)hb[k] : 0;
-                const int u = e & kMaxTile;
-                // every hit draws its selection: a near-band entry kept for being near
-                // counts only if selected should it lie in the shell when evaluated
-                bool sel = false;
-                if (k < n) {
-                    const int32_t id_j = rb.ids ? rb.ids[u] : tile_atom_id(h, rb.perm, u);
-                    sel = rbl_select(rb.seed, rb.epoch, id_i, id_j, rb.pice);
-                }
-                const bool keep = k < n && ((e & kInnerFlag) != 0 || sel);
-                const uint64_t mk = __ballot(keep);
-                if (keep) row[nk + (int)mbcnt64(mk)] = (uint16_t)(sel ? (u | kRblSel) : u);
-                nk += __popcll(mk);
-            }
-            if (lane == 0) row[nk] = (uint16_t)total;
-            __syncwarp();
-            n_in = n = nk;
-        } else if (n < cap) {
-            __syncwarp();  // the hit buffer, written by every lane of this wave
-            n_in = 0;
-            for (int k0 = 0; k0 < n; k0 += 64) {
-                const int k = k0 + lane;
-                n_in += __popcll(__ballot(k < n && (hb[k] & kInnerFlag) != 0));
-            }
-            int ci = 0, co = n_in;
-            for (int k0 = 0; k0 < n; k0 += 64) {
-                const int k = k0 + lane;
-                const int e = k < n ? (int)hb[k] : 0;
-                const bool in = k < n && (e & kInnerFlag) != 0;
-                const bool out = k < n && (e & kInnerFlag) == 0;
-                const uint64_t mi = __ballot(in), mo = __ballot(out);
-                if (in) row[ci + (int)mbcnt64(mi)] = (uint16_t)(e & kMaxTile);
-                if (out) row[co + (int)mbcnt64(mo)] = (uint16_t)e;
-                ci += __popcll(mi);
-                co += __popcll(mo);
-            }
-            if (lane == 0) row[n] = (uint16_t)total;
-            __syncwarp();  // the buffer is reused for the wave's next atom
-        }
-        if (lane == 0) {
-            ncount[s] = n < cap ? make_int2(n_in, n - n_in) : make_int2(n, 0);
-            if (n >= cap) {
-                atomicAdd(&stats[2], 1ull);
-                atomicMax(&stats[4], (unsigned long long)(n + 1));
-            }
+    };
+    const int blk = min(kListBlock, staged ? kListBlock : stage_cap / 16 * 16);
+    if (staged) stage(0, total);
+    const bool narrow = min(blk, total) <= 16 * 16 * kTileWaves;
+    const int group = narrow ? rows : rows / 32 * 16;  // 256 or 512 bytes a row and mask
+    const bool single = total <= blk;
+    const int uh = h.off[kHomeSeg] - h0;
+    for (int s0 = a0; s0 < a1; s0 += group) {
+        const int nrow = min(group, a1 - s0);
+        // the home atoms of the group, when the whole tile is staged
+        const float4* home = staged ? L.cand + s0 + uh : nullptr;
+        for (int cb = 0; cb < total; cb += blk) {
+            const int cn = min(blk, total - cb);
+            if (!staged) stage(cb, cn);
+            if (threadIdx.x == 0) lr.slow = 0ull;
+            __syncthreads();
+            const float4* cand = staged ? L.cand + cb : L.cand;
+            const int32_t* ids = RBL ? (staged ? L.ids + cb : L.ids) : nullptr;
+            const bool last = cb + blk >= total;
+            if (narrow)
+                list_block<RBL, uint32_t>(h, a, L, lr, cand, home, ids, cb, cn, s0, s0 + uh, nrow,
+                                          single, last, wv, lane, rb);
+            else
+                list_block<RBL, uint64_t>(h, a, L, lr, cand, home, ids, cb, cn, s0, s0 + uh, nrow,
+                                          single, last, wv, lane, rb);
         }
     }
 }

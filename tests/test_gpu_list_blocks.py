@@ -1,0 +1,68 @@
+"""Verlet rows across the shapes of the list build: candidate blocks (up to 2048 and up to
+4096 staged candidates, several blocks per tile, tiles beyond the LDS stage), groups of
+home atoms, and pairs at the criterion's small-distance bound.  The rows must equal the
+oracle's neighbour sets, bit for bit."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SEED = 20261202
+
+
+def _dev(a, dtype=torch.float64):
+    return torch.as_tensor(np.ascontiguousarray(a)).to(device="cuda", dtype=dtype)
+
+
+# (cutoff, cells per axis, density): tile candidates about 27 density (cutoff + 0.3)^3
+@pytest.mark.parametrize("rc,cells,rho,stage", [
+    (1.3, 4, 0.3, 0),     # about 35 candidates, a home cell of one or two atoms
+    (2.5, 4, 0.8, 0),     # 470 candidates, 18 home atoms
+    (5.0, 3, 0.3, 0),     # 1,200 candidates, 45 home atoms
+    (6.4, 3, 0.3, 0),     # 2,440: 32-bit masks, five groups of home atoms
+    (7.9, 3, 0.3, 0),     # 4,470: staged in LDS, two blocks
+    (8.4, 3, 0.3, 0),     # 5,300: beyond the LDS stage, blocks staged in turn
+    (5.0, 3, 0.3, 208),   # blocks of 208 candidates
+    (5.0, 2, 0.3, 0),     # two cells per axis: images
+])
+def test_rows_equal_oracle_sets(orc, gpu, rc, cells, rho, stage):
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce, systems
+
+    r_list = rc + 0.3
+    L = 1.013 * cells * r_list
+    n = int(rho * L ** 3)
+    print(f"case: rc {rc}, {cells} cells per axis, {n} ions, stage {stage}", flush=True)
+    sys.stdout.flush()
+    x, y, z, q, Lb_ = systems.random_ions(n, n / L ** 3, 0.8, seed=SEED)
+    # two pairs astride the smallest accepted distance (d^2 > 1e-4), one on the diagonal
+    x[1], y[1], z[1] = x[0] + 0.0099, y[0], z[0]
+    x[3], y[3], z[3] = x[2] + 0.0101, y[2], z[2]
+    x[5], y[5], z[5] = x[4] + 0.0058, y[4] - 0.0058, z[4] + 0.0058
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=(Lb_,) * 3, cut_off=min(rc, 2.5),
+                                         coulomb_cut=rc, alpha=0.5, kspace="NONE", n_max=n,
+                                         tile_stage=stage))
+    f.Init(_dev(q))
+    F = [torch.zeros(n, device="cuda") for _ in range(3)]
+    f.Execute(_dev(x), _dev(y), _dev(z), *F)
+    torch.cuda.synchronize()
+    st = f.stats()
+    assert st["cells"] == cells ** 3 and st["overflow_rows"] == 0
+    assert (st["big_tiles"] > 0) == (st["largest_tile"] >= st["tile_stage"])
+    Lb = np.array([Lb_] * 3)
+    xw, yw, zw = orc.wrap(x, y, z, np.zeros(3), Lb)
+    oo, io = orc.neighbors_images(xw, yw, zw, Lb, r_list)
+    og, ig = f.neighbors()
+    assert og[-1] == oo[-1]
+    for i in range(n):
+        assert np.array_equal(np.sort(ig[og[i]:og[i + 1]]), np.sort(io[oo[i]:oo[i + 1]])), i
+    # rows in their order: the entries within the LJ range come first
+    d = np.stack([xw, yw, zw], 1)
+    j, i = ig, np.repeat(np.arange(n), np.diff(og))
+    dd = d[j] - d[i]
+    dd -= Lb * np.round(dd / Lb)
+    inner = (dd * dd).sum(1) < (min(rc, 2.5) + 0.3) ** 2
+    if cells > 2:
+        assert st["inner_entries"] == int(inner.sum())
