@@ -214,7 +214,7 @@ static void ewald_lattice(const Engine& E, std::vector<int32_t>& m, std::vector<
 static hipError_t reset_tile_order(Engine& E)
 {
     if (!E.tile_order) return hipSuccess;
-    std::vector<int32_t> id((size_t)E.ncell * 4);
+    std::vector<int32_t> id((size_t)E.ncell * E.split_max);
     for (size_t k = 0; k < id.size(); ++k) id[k] = (int32_t)k;
     return hipMemcpy(E.tile_order, id.data(), id.size() * 4, hipMemcpyHostToDevice);
 }
@@ -275,9 +275,14 @@ static void tile_geometry(Engine& E, int64_t n)
     const int lds_wg = E.stage_cap * per + 2048;
     const int per_cu = std::max(1, std::min(4, E.lds_cu / lds_wg));
     const int resident = std::max(E.num_cu, 1) * per_cu;
+    // (more than four only where each part keeps 16 home atoms, a wave's two row times:
+    // boxes of a few cells, whose tiles hold hundreds)
     E.split = 1;
-    if (4 * E.ncell < 3 * resident)
-        E.split = std::min(4, (resident + E.ncell - 1) / E.ncell);
+    if (4 * E.ncell < 3 * resident) {
+        const int want = (resident + E.ncell - 1) / E.ncell;
+        const int parts = (int)std::min<int64_t>(E.split_max, n / ((int64_t)16 * E.ncell));
+        E.split = std::min(want, std::max(4, parts));
+    }
     if (E.tune_split > 0) E.split = std::min(4, E.tune_split);
 }
 
@@ -425,6 +430,7 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
         CR(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev));
         E.lds_cu = v > 0 ? v : E.lds_max;
     }
+    E.split_max = std::max(4, std::min(64, (4 * E.num_cu + E.ncell - 1) / E.ncell));
     tile_geometry(E, n_max);
     CR(dalloc(&E.xr, N * 8));
     CR(dalloc(&E.yr, N * 8));
@@ -437,7 +443,7 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
     CR(dalloc(&E.atom_cell, N * 4));
     CR(dalloc(&E.atom_rank, N * 4));
     CR(dalloc(&E.cell_count, (size_t)E.ncell * 4));
-    CR(dalloc(&E.tile_order, (size_t)E.ncell * 4 * 4));
+    CR(dalloc(&E.tile_order, (size_t)E.ncell * E.split_max * 4));
     CR(reset_tile_order(E));
     {
         // per-cell buckets of the MD step's binning: 4x the mean population
@@ -468,7 +474,7 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
     E.thermo_cnt = (uint32_t*)(E.thermo_st + 4);
     E.thermo_noise = (unsigned long long*)(E.thermo_st + 6);
     CR(dalloc(&E.ev, 16 * 8));
-    E.ev_part_blocks = E.ncell * 4;  // tile workgroups (split <= 4)
+    E.ev_part_blocks = E.ncell * E.split_max;  // tile workgroups
     CR(dalloc(&E.ev_part, (size_t)E.ev_part_blocks * 8 * 8));
     if (E.half) CR(dalloc(&E.planes, (size_t)kHalfSegs * 3 * N * sizeof(float)));
     if (E.rbl) {

@@ -286,7 +286,7 @@ struct KForceDrift {
 
 // ---------------------------------------------------------------- MD cell sort
 // Rebuild-step cell sort from the bins the tile pass made one step earlier
-// (buffer flags[3] & 1): one wave per cell.  The cell's start is the sum of the
+// (buffer flags[3] & 1): one wave per cell, more for cells of hundreds of atoms (sort_parts).  The cell's start is the sum of the
 // counts before it; its atoms come from the bucket (arrival order) ranked by id,
 // or, for a bucket that overflowed, from a scan of every binning slot's cell.  The
 // sorted slot s of atom v receives perm, inv_perm, the binned position as the
@@ -324,12 +324,14 @@ __device__ inline void cellsort_md_emit(const CellSortMDArgs& a, int c, int v, i
     a.ts[s] = a.type ? a.type[v] : 0;
 }
 
-// One wave sorts cell c (c >= ncell: nothing); buf holds kSortWaveBuf ids of
-// this wave's own LDS.  The bucket lists binning slots; atoms are ranked by id.
-__device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int lane, int32_t* buf)
+// One wave sorts entries part * 64 + lane, + 64 parts, ... of cell c (c >= ncell:
+// nothing); buf holds kSortWaveBuf ids of this wave's own LDS.  The bucket lists binning
+// slots; atoms are ranked by id.
+__device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int part, int parts,
+                                        int lane, int32_t* buf)
 {
     const uint32_t req = a.flags[0];
-    if (c == 0 && lane == 0) {
+    if (c == 0 && part == 0 && lane == 0) {
         a.flags[2] = req;
         if (req) {
             a.stats[0] += 1ull;
@@ -348,13 +350,13 @@ __device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int lane
     // chunk before c: at most ncell / kBinChunk + kBinChunk loads per cell (without
     // chunk counts, every earlier cell)
     const int c0 = a.bins.nchunk > 0 ? (c / kBinChunk) * kBinChunk : 0;
-    int part = 0;
+    int before = 0;
     if (a.bins.nchunk > 0)
-        for (int k = lane; k < c / kBinChunk; k += 64) part += chunk[k];
-    for (int k = c0 + lane; k < c; k += 64) part += count[k];
-    const int s0 = wave_sum(part);
+        for (int k = lane; k < c / kBinChunk; k += 64) before += chunk[k];
+    for (int k = c0 + lane; k < c; k += 64) before += count[k];
+    const int s0 = wave_sum(before);
     const int cnt = count[c];
-    if (lane == 0) {
+    if (lane == 0 && part == 0) {
         a.cell_start[c] = s0;
         if (c == a.ncell - 1) a.cell_start[a.ncell] = s0 + cnt;
     }
@@ -364,21 +366,21 @@ __device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int lane
             // ids staged in LDS, each lane ranks its own entries
             for (int k = lane; k < cnt; k += 64) buf[k] = a.bins.vid[bk[k]];
             __syncwarp();
-            for (int k = lane; k < cnt; k += 64) {
+            for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {
                 const int v = buf[k];
                 int r = 0;
                 for (int t = 0; t < cnt; ++t) r += (buf[t] < v) ? 1 : 0;
                 cellsort_md_emit(a, c, v, bk[k], s0 + r);
             }
         } else {
-            for (int k = lane; k < cnt; k += 64) {
+            for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {
                 const int v = a.bins.vid[bk[k]];
                 int r = 0;
                 for (int t = 0; t < cnt; ++t) r += (a.bins.vid[bk[t]] < v) ? 1 : 0;
                 cellsort_md_emit(a, c, v, bk[k], s0 + r);
             }
         }
-    } else {
+    } else if (part == 0) {
         // the bucket overflowed: scan every binning slot (order: by slot)
         int found = 0;
         for (int base = 0; base < a.n; base += 64) {
@@ -391,8 +393,8 @@ __device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int lane
     }
 }
 
-// rho(k) partials (workgroups [0, nrho)) and the MD cell sort (the rest, one
-// cell per wave) in one grid: both read only the step's drifted positions.
+// rho(k) partials (workgroups [0, nrho)) and the MD cell sort (the rest, `parts`
+// waves per cell) in one grid: both read only the step's drifted positions.
 template <typename T>
 struct SortRho {
     static constexpr int kThreads = kRhoBlock;
@@ -407,6 +409,7 @@ struct SortRho {
         int nrho;
         CellSortMDArgs cs;
         int nsort;  // cell-sort workgroups; the one after them orders the tiles
+        int parts;  // waves per cell of the sort
         int3 dims;
         int split, ncu;  // ncu 0: keep the cell order
         int32_t* tile_order;
@@ -430,10 +433,12 @@ struct SortRho {
             return;
         }
         const int wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
-        cellsort_md_cell(A.cs, blk * kWaves + wv, lane, (int32_t*)lds + wv * kSortWaveBuf);
+        const int w = blk * kWaves + wv;
+        cellsort_md_cell(A.cs, w / A.parts, w % A.parts, A.parts, lane,
+                         (int32_t*)lds + wv * kSortWaveBuf);
     }
 };
 
-inline int sortrho_cell_blocks(int ncell) { return (ncell + kRhoBlock / 64 - 1) / (kRhoBlock / 64); }
+inline int sortrho_cell_blocks(int waves) { return (waves + kRhoBlock / 64 - 1) / (kRhoBlock / 64); }
 
 }  // namespace rbmd

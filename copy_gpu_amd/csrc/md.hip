@@ -68,7 +68,8 @@ typename SortRho<T>::Args sortrho_args(Engine& e, const RepState& st, int* block
     else memset(&a.rho, 0, sizeof a.rho);
     a.nrho = nr;
     a.cs = cellsort_md_args(e, st);
-    a.nsort = sortrho_cell_blocks(e.ncell);
+    a.parts = sort_parts(e.n, e.ncell);
+    a.nsort = sortrho_cell_blocks(e.ncell * a.parts);
     a.dims = make_int3(e.dims[0], e.dims[1], e.dims[2]);
     a.split = e.split;
     a.ncu = tile_order_ncu(e.ncell, e.split, e.num_cu);

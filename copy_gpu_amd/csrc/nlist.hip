@@ -150,7 +150,7 @@ struct Scatter {
     static constexpr int kThreads = kBlock;
     struct Args {
         const int32_t *atom_cell, *atom_rank, *start;
-        int32_t* perm;
+        int32_t* order;
         int n;
         const uint32_t* flags;
     };
@@ -159,12 +159,12 @@ struct Scatter {
         if (a.flags[2] == 0u) return;
         const int i = blk * kBlock + threadIdx.x;
         if (i >= a.n) return;
-        a.perm[a.start[a.atom_cell[i]] + a.atom_rank[i]] = i;
+        a.order[a.start[a.atom_cell[i]] + a.atom_rank[i]] = i;
     }
 };
 
 // ---------------------------------------------------------------- per-cell sort
-// One wave per cell: order the cell's atoms by original id (rank sort in LDS)
+// One wave per cell (sort_parts of them in cells of hundreds of atoms): order the cell's atoms by original id (rank sort in LDS)
 // so the layout is deterministic, then write the sorted reference positions
 // (also the current sorted positions: a build happens at the current
 // positions), charges, types, cells and the inverse permutation.
@@ -180,31 +180,33 @@ struct CellSort {
         double4 *xs_ref, *xs;
         int32_t *scell, *ts;
         const uint32_t* flags;
+        const int32_t* order;  // the cells' atoms in arrival order
+        int parts;
     };
     __device__ static void run(const Args& a, int blk, int)
     {
         if (a.flags[2] == 0u) return;
         __shared__ int32_t buf[kCellSortMax];
-        const int c = blk;
+        const int c = blk / a.parts, part = blk % a.parts;
         const int lane = threadIdx.x;
         const int s0 = a.start[c], cnt = a.start[c + 1] - s0;
         const bool sortable = cnt <= kCellSortMax;
         if (sortable) {
-            for (int k = lane; k < cnt; k += 64) buf[k] = a.perm[s0 + k];
+            for (int k = lane; k < cnt; k += 64) buf[k] = a.order[s0 + k];
             __syncthreads();
         }
-        for (int k = lane; k < cnt; k += 64) {
+        for (int k = part * 64 + lane; k < cnt; k += 64 * a.parts) {
             int v, r;
             if (sortable) {
                 v = buf[k];
                 r = 0;
                 for (int t = 0; t < cnt; ++t) r += (buf[t] < v) ? 1 : 0;
             } else {
-                v = a.perm[s0 + k];
+                v = a.order[s0 + k];
                 r = k;
             }
             const int s = s0 + r;
-            if (sortable) a.perm[s] = v;
+            a.perm[s] = v;
             a.inv_perm[v] = s;
             const double4 p = make_double4(a.xr[v], a.yr[v], a.zr[v], a.q[v]);
             a.xs_ref[s] = p;
@@ -407,13 +409,15 @@ Scan::Args scan_args(Engine& e)
 
 Scatter::Args scatter_args(Engine& e)
 {
-    return Scatter::Args{e.atom_cell, e.atom_rank, e.cell_start, e.perm, (int)e.n, e.flags};
+    // the arrival order goes to the MD bins' atom ids, which every MD run fills anew
+    return Scatter::Args{e.atom_cell, e.atom_rank, e.cell_start, e.md_vid, (int)e.n, e.flags};
 }
 
 CellSort::Args cellsort_args(Engine& e)
 {
     return CellSort::Args{e.perm, e.atom_rank /* reused as inverse perm */, e.cell_start, e.xr,
-                          e.yr,   e.zr, e.q, e.type, e.xs_ref, e.xs, e.scell, e.ts, e.flags};
+                          e.yr,   e.zr, e.q, e.type, e.xs_ref, e.xs, e.scell, e.ts, e.flags,
+                          e.md_vid, sort_parts(e.n, e.ncell)};
 }
 
 Gather::Args gather_args(Engine& e, const double* x, const double* y, const double* z)
@@ -460,7 +464,7 @@ void launch_build(Engine& e, const double* x, const double* y, const double* z, 
     }
     {
         ScopedTimer t(e, P_CELLSORT, s);
-        k_one<CellSort><<<e.ncell, 64, 0, s>>>(cellsort_args(e));
+        k_one<CellSort><<<e.ncell * sort_parts(e.n, e.ncell), 64, 0, s>>>(cellsort_args(e));
     }
     // the Verlet rows are built inside the tile pass (pair.hip)
 }
@@ -514,7 +518,7 @@ hipError_t nlist_batch_prepare(Batch& b)
     std::vector<int> nmc(R);
     std::vector<ChunkSum::Args> cks(R);
     std::vector<Gather::Args> ga(R);
-    std::vector<int> nat(R), none(R, 1), ncell(R), nch(R);
+    std::vector<int> nat(R), none(R, 1), nsort(R), nch(R);
     for (size_t r = 0; r < R; ++r) {
         Engine& e = *b.es[r];
         const RepState& st = b.st[r];
@@ -530,14 +534,14 @@ hipError_t nlist_batch_prepare(Batch& b)
         cks[r] = ChunkSum::Args{md_bins(e), e.flags};
         ga[r] = gather_args(e, st.x, st.y, st.z);
         nat[r] = nblk(e.n > 0 ? e.n : 1);
-        ncell[r] = e.ncell;
+        nsort[r] = e.ncell * sort_parts(e.n, e.ncell);
         nch[r] = md_nchunk(e.ncell);
     }
     hipError_t err;
     if ((err = phase_upload(b.ph[BP_BIN], bi, nat, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_SCAN], sc, none, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_SCATTER], sp, nat, 0)) != hipSuccess) return err;
-    if ((err = phase_upload(b.ph[BP_CELLSORT], cs, ncell, 0)) != hipSuccess) return err;
+    if ((err = phase_upload(b.ph[BP_CELLSORT], cs, nsort, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_MDCLEAR], mc, nmc, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_MDBIN], mb, nat, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_CHUNKSUM], cks, nch, 0)) != hipSuccess) return err;

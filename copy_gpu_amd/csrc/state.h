@@ -71,6 +71,7 @@ struct Engine {
     int ncell = 0;
     int cap = 0;        // list row capacity, multiple of 64
     int split = 1;      // workgroups per cell tile
+    int split_max = 4;  // largest split the per-workgroup buffers are sized for
     int stage_cap = 0;  // LDS tile capacity (candidates)
     int stage_override = 0;
     // tile shapes chosen by the autotuner (0 / default: heuristics)
@@ -275,6 +276,15 @@ inline MdBins md_bins(const Engine& e)
     return MdBins{e.md_count, e.md_count + 2 * (size_t)e.ncell, e.md_bucket, e.md_cell,
                   e.md_vid,   e.md_w, e.md_w + n, e.md_w + 2 * n, e.ncell, e.bucket_cap,
                   md_nchunk(e.ncell)};
+}
+
+// Waves that rank one cell's atoms.  The rank of each atom is counted over the whole cell,
+// so one wave takes cnt^2 / 64 steps: a few us at the 20-80 atoms of ordinary cells, 230 us
+// at the 1,000 of a one-cell box.
+inline int sort_parts(int64_t n, int ncell)
+{
+    const int64_t mean = n / ncell;
+    return mean <= 128 ? 1 : (int)std::min<int64_t>(16, (mean + 63) / 64);
 }
 
 // Bytes of the MD bin counts: per-cell and per-chunk, both double-buffered.
