@@ -1,0 +1,73 @@
+// lattice.h -- structure factor on a whole lattice box |m_d| <= M_d in FP64.
+//
+// exp(2 pi i m.s) factors into one phase per axis, so rho(m) of every m of the box is a
+// matrix product over the atoms instead of one sine and cosine per (m, atom).  In real
+// arithmetic, with the per-axis basis e_0 = 1, e_(2m-1) = cos(2 pi m s), e_(2m) =
+// sin(2 pi m s), the sums
+//   T[a, b][c] = sum_j q_j e_a(x_j) e_b(y_j) e_c(z_j),   a <= 2 M_x, b <= 2 M_y, c <= 2 M_z
+// hold rho of (m_x, +-m_y, +-m_z) as combinations of eight of them, with half the products
+// of the complex form.  Rows are (a, b), columns c, and the contraction runs over atoms.
+#pragma once
+#include <stddef.h>
+#include <stdint.h>
+
+#include "engine.h"
+
+namespace rbmd {
+
+constexpr int kLatRows = 256;    // rows of one workgroup: 4 waves x 4 row tiles of 16
+constexpr int kLatStage = 32;    // atoms per LDS stage
+constexpr int kLatStride = 36;   // doubles between rows of a table: 16 rows x 4 atoms of a
+                                 // fragment fall on all 64 banks once
+constexpr int kLatTargetWg = 512;  // two workgroups per CU on the 256 CUs of an MI355X
+constexpr int64_t kLatMaxPart = (int64_t)1 << 26;  // most doubles of the partial sums
+
+// Position of cos / sin of m in an axis basis.
+RBMD_HD inline int lat_cos(int m) { return m ? 2 * m - 1 : 0; }
+RBMD_HD inline int lat_sin(int m) { return 2 * m; }  // m >= 1
+
+struct LatGeom {
+    int M[3];
+    int B, C;              // basis sizes of the y and z axes
+    int64_t R;             // rows (2 M_x + 1) B
+    int nc, rblk, cblk;    // 16-column tiles per workgroup; row and column blocks
+    int nx, ny;            // LDS table rows of the x and y axes
+    int slices, aps;       // atom slices and atoms per slice
+    size_t lds;
+    RBMD_HD int64_t sums() const { return R * (int64_t)C; }
+};
+
+LatGeom lat_geometry(const int M[3], int64_t n);
+
+// T of every slice into part [slices][R][C], then their sum in slice order into part[0].
+void launch_lattice_sums(const LatGeom& g, const Box& box, int64_t n, const double* x,
+                         const double* y, const double* z, const double* q, double* part,
+                         hipStream_t s);
+
+#ifdef __HIPCC__
+// The eight sums of an octant point, axes x, y, z as bits 2, 1, 0 (1: sine).
+struct LatOct {
+    double t[8];
+};
+__device__ inline LatOct lat_octant(const double* __restrict__ T, int B, int C, int mx, int my,
+                                    int mz)
+{
+    LatOct o;
+    for (int k = 0; k < 8; ++k) {
+        const int sx = k >> 2, sy = (k >> 1) & 1, sz = k & 1;
+        const bool ok = (!sx || mx) && (!sy || my) && (!sz || mz);
+        const int a = sx ? lat_sin(mx) : lat_cos(mx), b = sy ? lat_sin(my) : lat_cos(my),
+                  c = sz ? lat_sin(mz) : lat_cos(mz);
+        o.t[k] = ok ? T[((int64_t)a * B + b) * C + c] : 0.0;
+    }
+    return o;
+}
+// rho(mx, gy my, gz mz), gy and gz = +-1.
+__device__ inline void lat_rho(const LatOct& o, double gy, double gz, double* re, double* im)
+{
+    *re = o.t[0] - gy * o.t[6] - gz * o.t[5] - gy * gz * o.t[3];
+    *im = o.t[4] + gy * o.t[2] + gz * o.t[1] - gy * gz * o.t[7];
+}
+#endif
+
+}  // namespace rbmd

@@ -25,7 +25,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .force import ForceConfig, LJCutCoulKspaceForce, RBMDError, _stream
+from .force import LJCutCoulKspaceForce, RBMDError, _ptr, _stream
 
 NPARAM = 4545
 
@@ -181,43 +181,48 @@ def analytic_weight(m: np.ndarray, box_len, alpha: float) -> np.ndarray:
 
 
 # ---------------------------------------------------------------- spectra
+SPECTRUM_MIN_BOX = 1.1  # smallest box edge that spectrum takes
+
+
 def spectrum(snapshots, q: torch.Tensor, box_len, alpha: float, Mg: int,
              box_lo=(0.0, 0.0, 0.0)) -> np.ndarray:
     """Mean |rho(m)|^2 over snapshots on the lattice box |m_d| <= Mg (FP64).
 
     snapshots: iterable of (x, y, z) FP64 device tensors.  rho(m) is the FP64
-    structure factor of the engine's k-space pass over the half space; the
-    other half follows from rho(-m) = conj(rho(m)).  Returns [(2Mg+1)^3], 0 at m = 0.
+    structure factor, formed over the whole box at once (rbmd_lattice_spectrum).
+    Returns [(2Mg+1)^3], 0 at m = 0.
     """
-    m = lattice_grid(Mg)
-    hs = half_space(m)
-    mh = torch.as_tensor(m[hs].ravel(), dtype=torch.int32, device="cuda")
-    Ph = int(hs.sum())
+    lib = L.lib()
+    assert q.is_cuda and q.dtype == torch.float64 and q.is_contiguous()
+    if Mg < 1 or not alpha > 0:
+        raise RBMDError(f"spectrum needs Mg >= 1 and alpha > 0 (Mg {Mg}, alpha {alpha})")
+    if not all(v >= SPECTRUM_MIN_BOX for v in box_len):
+        raise RBMDError(f"box edges must be at least {SPECTRUM_MIN_BOX}: {tuple(box_len)}")
     n = q.numel()
-    cfg = ForceConfig(box_len=tuple(box_len), box_lo=tuple(box_lo), cut_off=1.0,
-                      coulomb_cut=1.0, skin=0.1, alpha=alpha, kspace="RBE",
-                      coulomb_sample_num=Ph, precision=64, n_max=n)
-    f = LJCutCoulKspaceForce(cfg)
-    try:
-        f.Init(q)
-        f.set_kvectors(mh)
-        fx = torch.empty(n, dtype=torch.float64, device="cuda")
-        fy, fz = torch.empty_like(fx), torch.empty_like(fx)
-        acc = np.zeros(Ph)
+    lo = (C.c_double * 3)(*[float(v) for v in box_lo])
+    ln = (C.c_double * 3)(*[float(v) for v in box_len])
+    bytes_ = lib.rbmd_lattice_spectrum_workspace(n, Mg)
+    if bytes_ < 0:
+        raise RBMDError(lib.rbmd_lattice_last_error().decode())
+    with torch.cuda.device(q.device):
+        ws = torch.empty(bytes_ // 8, dtype=torch.float64, device=q.device)
+        s2 = torch.empty((2 * Mg + 1) ** 3, dtype=torch.float64, device=q.device)
         cnt = 0
         for (x, y, z) in snapshots:
-            f.Execute(x, y, z, fx, fy, fz)
-            _, _, re, im = f.kspace()
-            acc += re * re + im * im
+            for t in (x, y, z):
+                assert t.is_cuda and t.dtype == torch.float64 and t.numel() == n
+            rc = lib.rbmd_lattice_spectrum(lo, ln, n, _ptr(x), _ptr(y), _ptr(z), _ptr(q), Mg,
+                                           1 if cnt else 0, _ptr(s2), _ptr(ws), bytes_,
+                                           _stream(None))
+            if rc != 0:
+                raise RBMDError(f"rbmd_lattice_spectrum -> {rc}: "
+                                f"{lib.rbmd_lattice_last_error().decode()}")
             cnt += 1
-    finally:
-        f.close()
-    S2 = np.zeros(len(m))
-    S2[hs] = acc / max(cnt, 1)
-    # rho(-m) = conj(rho(m)): index of -m in x-fastest order is G - 1 - i
-    G = len(m)
-    idx = np.nonzero(hs)[0]
-    S2[G - 1 - idx] = S2[idx]
+        if cnt == 0:
+            s2.zero_()
+        S2 = s2.cpu().numpy()
+    if cnt > 1:
+        S2 /= cnt
     return S2
 
 

@@ -309,6 +309,19 @@ int rbmd_kspace_compute_noalloc(const rbmd_kspace_params* p, int64_t n, const do
 
 const char* rbmd_kspace_last_error(void);
 
+/* |rho(m)|^2 of one configuration on the whole lattice box |m_d| <= Mg (FP64; rho as the
+ * structure factor of rbmd/framework/run/worklet/RunWorklet.cpp:1616-1677), x fastest:
+ * s2[(2Mg+1)^3] on the device, 0 at m = 0; accumulate != 0 adds to s2 instead of writing it
+ * (sums over snapshots).  x, y, z, q: FP64 device arrays (n).  workspace: device memory of
+ * at least rbmd_lattice_spectrum_workspace(n, Mg) bytes (-1: invalid arguments), in use
+ * until the stream has run the call; nothing is allocated or synchronised.  1 <= Mg <= 1024. */
+int64_t rbmd_lattice_spectrum_workspace(int64_t n, int32_t Mg);
+int rbmd_lattice_spectrum(const double* box_lo, const double* box_len, int64_t n,
+                          const double* x, const double* y, const double* z, const double* q,
+                          int32_t Mg, int32_t accumulate, double* s2, void* workspace,
+                          int64_t bytes, void* stream);
+const char* rbmd_lattice_last_error(void);
+
 /* Plain device copy of nbytes (multiple of 16), used to calibrate HBM
  * traffic counters against a kernel of known traffic. */
 int rbmd_util_copy(void* dst, const void* src, int64_t nbytes, void* stream);
