@@ -17,8 +17,8 @@ namespace rbmd {
 
 constexpr int kLatRows = 256;    // rows of one workgroup: 4 waves x 4 row tiles of 16
 constexpr int kLatStage = 32;    // atoms per LDS stage
-constexpr int kLatStride = 36;   // doubles between rows of a table: 16 rows x 4 atoms of a
-                                 // fragment fall on all 64 banks once
+constexpr int kLatStride = 34;   // doubles between rows of a table: the 16 rows x 2 atoms of
+                                 // half a fragment fall on all 64 banks once
 constexpr int kLatTargetWg = 512;  // two workgroups per CU on the 256 CUs of an MI355X
 constexpr int64_t kLatMaxPart = (int64_t)1 << 26;  // most doubles of the partial sums
 

@@ -46,8 +46,17 @@ struct LatSumArgs {
 // the A fragment is the product of an x and a y table value, the B fragment a z value, and
 // the constant column (c = 0) is the running sum of the A fragments.
 //
-// Bound by FP64 matrix issue: 8 x 4 NC matrix instructions of 64 cycles per wave and stage
-// against about 9 sines and cosines per thread.
+// Tables: sines and cosines of m = 1 .. 8 per axis by sincospi, larger m by rotating eight
+// further at a time (one rounding of about 2^-53 each, far below the phase's own).  The
+// positions come through LDS 256 atoms at a time, as exact box fractions.
+//
+// Bound by FP64 issue: 8 x 4 NC matrix instructions of 64 cycles per wave and stage (58% of
+// the cycles) and about three sines and cosines per thread.  100,000 ions, |m_d| <= 32 (5.4e10
+// operations): 1.27 ms, 43 TFLOP/s of the 72 that a large FP64 product reaches here; with a
+// sine and cosine per (m, atom) the sums took 29 ms.
+constexpr int kLatBase = 8;      // m that get a sine and cosine of their own
+constexpr int kLatLoad = 256;    // atoms per load of positions
+
 template <int NC>
 __global__ __launch_bounds__(256, 2) void k_lat_sums(LatSumArgs A)
 {
@@ -64,6 +73,8 @@ __global__ __launch_bounds__(256, 2) void k_lat_sums(LatSumArgs A)
     double* Xt = lat_lds;
     double* Yt = Xt + (size_t)g.nx * kLatStride;
     double* Zt = Yt + (size_t)ny * kLatStride;
+    double* base = Zt + (size_t)16 * NC * kLatStride;  // [y, z][m - 1][cos, sin][atom]
+    double* frac = base + 2 * kLatBase * 2 * kLatStage;  // [x hi, x lo, y .., z .., q][atom]
 
     int xo[4], yo[4];
     for (int i = 0; i < 4; ++i) {
@@ -82,43 +93,86 @@ __global__ __launch_bounds__(256, 2) void k_lat_sums(LatSumArgs A)
 
     const int64_t j0 = (int64_t)blockIdx.z * g.aps;
     const int64_t j1 = j0 + g.aps < A.n ? j0 + g.aps : A.n;
-    const int at = t & (kLatStage - 1);
+    const int at = t & (kLatStage - 1), grp = t / kLatStage;
+    constexpr int kGrp = 256 / kLatStage;
+    static_assert(kGrp == kLatBase, "a thread's multiples of one axis are one rotation apart");
     const int mx0 = (a0 + 1) >> 1, nmx = ((a0 + nx) >> 1) - mx0 + 1;
-    const int items = nmx + g.M[1] + 1 + 8 * NC;
-    for (int64_t base = j0; base < j1; base += kLatStage) {
-        const int64_t j = base + at;
-        Frac s[3] = {{0, 0}, {0, 0}, {0, 0}};
-        double q = 0.0;
-        if (j < j1) {
-            s[0] = lat_frac(A.x[j] - A.box.lo[0], A.box.L[0], A.box.invL[0]);
-            s[1] = lat_frac(A.y[j] - A.box.lo[1], A.box.L[1], A.box.invL[1]);
-            s[2] = lat_frac(A.z[j] - A.box.lo[2], A.box.L[2], A.box.invL[2]);
-            q = A.q[j];
+    const int items = 2 * kLatBase + nmx;
+    for (int64_t j = j0; j < j1; j += kLatStage) {
+        const int fo = (int)((j - j0) & (kLatLoad - 1));
+        if (fo == 0) {
+            const int64_t i = j + t;
+            Frac s[3] = {{0, 0}, {0, 0}, {0, 0}};
+            double q = 0.0;
+            if (i < j1) {
+                s[0] = lat_frac(A.x[i] - A.box.lo[0], A.box.L[0], A.box.invL[0]);
+                s[1] = lat_frac(A.y[i] - A.box.lo[1], A.box.L[1], A.box.invL[1]);
+                s[2] = lat_frac(A.z[i] - A.box.lo[2], A.box.L[2], A.box.invL[2]);
+                q = A.q[i];
+            }
+            for (int d = 0; d < 3; ++d) {
+                frac[(2 * d) * kLatLoad + t] = s[d].hi;
+                frac[(2 * d + 1) * kLatLoad + t] = s[d].lo;
+            }
+            frac[6 * kLatLoad + t] = q;
         }
-        __syncthreads();
-        for (int e = t / kLatStage; e < items; e += 256 / kLatStage) {
+        __syncthreads();  // the fractions are there; the last stage's tables are read
+        for (int e = grp; e < items; e += kGrp) {
+            const int d = e < kLatBase ? 1 : e < 2 * kLatBase ? 2 : 0;
+            const int m = d == 0 ? mx0 + e - 2 * kLatBase : (e & (kLatBase - 1)) + 1;
+            const Frac s{frac[(2 * d) * kLatLoad + fo + at], frac[(2 * d + 1) * kLatLoad + fo + at]};
             double sn, cs;
-            if (e < nmx) {
-                const int m = mx0 + e;
-                lat_sincos(s[0], m, &sn, &cs);
+            lat_sincos(s, m, &sn, &cs);
+            if (d == 0) {
+                const double q = frac[6 * kLatLoad + fo + at];
                 const int ic = lat_cos(m) - a0, is = lat_sin(m) - a0;
                 if (ic >= 0 && ic < nx) Xt[ic * kLatStride + at] = q * cs;
                 if (m && is >= 0 && is < nx) Xt[is * kLatStride + at] = q * sn;
-            } else if (e < nmx + g.M[1] + 1) {
-                const int m = e - nmx;
+            } else {
+                base[(2 * e) * kLatStage + at] = cs;
+                base[(2 * e + 1) * kLatStage + at] = sn;
+            }
+        }
+        __syncthreads();
+        {
+            // y: m = grp, grp + 8, ...
+            const double C8 = base[(2 * kLatBase - 2) * kLatStage + at],
+                         S8 = base[(2 * kLatBase - 1) * kLatStage + at];
+            double cs = grp ? base[(2 * grp - 2) * kLatStage + at] : 1.0,
+                   sn = grp ? base[(2 * grp - 1) * kLatStage + at] : 0.0;
+            for (int m = grp; m <= g.M[1]; m += kGrp) {
                 int ic = lat_cos(m) - b0, is = lat_sin(m) - b0;
                 ic += ic < 0 ? B : 0;
                 is += is < 0 ? B : 0;
-                if (ic >= ny && is >= ny) continue;
-                lat_sincos(s[1], m, &sn, &cs);
                 if (ic < ny) Yt[ic * kLatStride + at] = cs;
                 if (m && is < ny) Yt[is * kLatStride + at] = sn;
+                const double c = fma(cs, C8, -(sn * S8));
+                sn = fma(sn, C8, cs * S8);
+                cs = c;
+            }
+        }
+        {
+            // z: m = c0 / 2 + 1 + grp, .. + 8, ..., columns 2 m - 1 and 2 m
+            const double* zb = base + 2 * kLatBase * kLatStage;
+            const double C8 = zb[(2 * kLatBase - 2) * kLatStage + at],
+                         S8 = zb[(2 * kLatBase - 1) * kLatStage + at];
+            double cs, sn;
+            if (c0 == 0) {
+                cs = zb[(2 * grp) * kLatStage + at];
+                sn = zb[(2 * grp + 1) * kLatStage + at];
             } else {
-                const int i = e - nmx - g.M[1] - 1, m = (c0 >> 1) + 1 + i;
-                sn = cs = 0.0;
-                if (m <= g.M[2]) lat_sincos(s[2], m, &sn, &cs);
-                Zt[(2 * i) * kLatStride + at] = cs;
-                Zt[(2 * i + 1) * kLatStride + at] = sn;
+                lat_sincos({frac[4 * kLatLoad + fo + at], frac[5 * kLatLoad + fo + at]},
+                           (c0 >> 1) + 1 + grp, &sn, &cs);
+            }
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int e = grp + kGrp * i;
+                const bool in = (c0 >> 1) + 1 + e <= g.M[2];
+                Zt[(2 * e) * kLatStride + at] = in ? cs : 0.0;
+                Zt[(2 * e + 1) * kLatStride + at] = in ? sn : 0.0;
+                const double c = fma(cs, C8, -(sn * S8));
+                sn = fma(sn, C8, cs * S8);
+                cs = c;
             }
         }
         __syncthreads();
@@ -209,7 +263,8 @@ LatGeom lat_geometry(const int M[3], int64_t n)
     g.rblk = (int)((g.R + kLatRows - 1) / kLatRows);
     g.ny = std::min(g.B, kLatRows);
     g.nx = std::min(2 * M[0] + 1, (kLatRows - 1) / g.B + 2);
-    g.lds = (size_t)(g.nx + g.ny + 16 * g.nc) * kLatStride * sizeof(double);
+    g.lds = ((size_t)(g.nx + g.ny + 16 * g.nc) * kLatStride +
+             (size_t)4 * kLatBase * kLatStage + (size_t)7 * kLatLoad) * sizeof(double);
     // atom slices: one round of two workgroups per CU (a second, partial round would leave
     // CUs idle), while the partial sums stay bounded and a slice keeps two stages
     int64_t want = std::max<int64_t>(1, kLatTargetWg / ((int64_t)g.rblk * g.cblk));
