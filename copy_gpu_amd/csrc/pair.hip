@@ -1086,39 +1086,33 @@ struct RblMean {
 };
 
 // Deterministic final reduction: pair partials [nb][8] + per-k terms [P][7]
-// + self energy -> ev[10] = {e_lj, e_real, e_self, e_k, W_xx..W_yz}.
-__global__ __launch_bounds__(256) void k_ev_final(const double* __restrict__ ev_part, int nb,
-                                                  const double* __restrict__ kev, int P,
-                                                  double e_self, double* __restrict__ ev)
+// + self energy -> ev[10] = {e_lj, e_real, e_self, e_k, W_xx..W_yz}.  One workgroup per
+// output, a fixed order of strided sums, waves and wave sums.  30,000 ions: 5 us, and 29 us
+// with the 52,800 k-vectors of a full Ewald at 6,000; one workgroup for all fifteen columns
+// took 17 and 206 us.
+constexpr int kEvThreads = 1024;
+__global__ __launch_bounds__(kEvThreads) void k_ev_final(const double* __restrict__ ev_part,
+                                                         int nb, const double* __restrict__ kev,
+                                                         int P, double e_self,
+                                                         double* __restrict__ ev)
 {
-    __shared__ double red[256];
-    const int t = threadIdx.x;
-    double out[10];
-    for (int c = 0; c < 15; ++c) {
-        double v = 0.0;
-        if (c < 8) {
-            for (int b = t; b < nb; b += 256) v += ev_part[(size_t)b * 8 + c];
-        } else {
-            for (int k = t; k < P; k += 256) v += kev[(size_t)k * 7 + (c - 8)];
-        }
-        red[t] = v;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if (t < o) red[t] += red[t + o];
-            __syncthreads();
-        }
-        const double r = red[0];
-        __syncthreads();
-        // c: 0 e_lj, 1 e_real, 2..7 pair virial, 8 e_k, 9..14 k virial
-        if (c == 0) out[0] = r;
-        else if (c == 1) out[1] = r;
-        else if (c < 8) out[4 + (c - 2)] = r;
-        else if (c == 8) out[3] = r;
-        else out[4 + (c - 9)] += r;
-    }
+    __shared__ double red[kEvThreads / 64];
+    const int t = threadIdx.x, o = blockIdx.x;
+    // columns of the pair partials (0 e_lj, 1 e_real, 2..7 virial) and of the per-k terms
+    // (0 e_k, 1..6 virial) that output o sums
+    const int cp = o < 2 ? o : o < 4 ? -1 : o - 2, ck = o < 3 ? -1 : o - 3;
+    double v = 0.0;
+    if (cp >= 0)
+        for (int b = t; b < nb; b += kEvThreads) v += ev_part[(size_t)b * 8 + cp];
+    if (ck >= 0)
+        for (int k = t; k < P; k += kEvThreads) v += kev[(size_t)k * 7 + ck];
+    v = wave_sum(v);
+    if ((t & 63) == 0) red[t >> 6] = v;
+    __syncthreads();
     if (t == 0) {
-        out[2] = e_self;
-        for (int k = 0; k < 10; ++k) ev[k] = out[k];
+        double r = 0.0;
+        for (int w = 0; w < kEvThreads / 64; ++w) r += red[w];
+        ev[o] = o == 2 ? e_self : r;
     }
 }
 
@@ -1384,7 +1378,7 @@ void launch_ev_final(Engine& e, bool with_pair, hipStream_t s)
     const int nb = with_pair ? e.ncell * e.split : 0;  // one partial per tile workgroup
                                                         // (split 1 for half tiles)
     const int P = (e.kspace != 0) ? e.P : 0;
-    k_ev_final<<<1, 256, 0, s>>>(e.ev_part, nb, e.kev, P, e.e_self, e.ev);
+    k_ev_final<<<10, kEvThreads, 0, s>>>(e.ev_part, nb, e.kev, P, e.e_self, e.ev);
 }
 
 hipError_t pair_batch_prepare(Batch& b)
