@@ -122,6 +122,7 @@ static void free_all(Engine& E)
                     E.thermo_st, E.rbl_part, E.rbl_mean, E.planes};
     for (void* p : ptrs)
         if (p) hipFree(p);
+    ewald_free(E);
     if (E.h_stats) hipHostFree(E.h_stats);
     for (auto& G : E.graphs) {
         if (G.exec) hipGraphExecDestroy(G.exec);
@@ -515,6 +516,7 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
         CR(hipMemcpy(E.km, m.data(), m.size() * 4, hipMemcpyHostToDevice));
         CR(hipMemcpy(E.kw, w.data(), w.size() * 8, hipMemcpyHostToDevice));
         E.P = P;
+        if (E.precision == 64) CR(ewald_setup(E, m));
     }
 #undef CR
     *out = h;

@@ -185,7 +185,7 @@ struct RhoFinalArgs {
 };
 
 template <typename T>
-__device__ inline void rho_final_emit(const RhoFinalArgs<T>& A, int k, double re, double im)
+__device__ inline KCoef<T> rho_final_emit(const RhoFinalArgs<T>& A, int k, double re, double im)
 {
     const Box& box = A.box;
     A.rho[2 * k] = re;
@@ -216,6 +216,7 @@ __device__ inline void rho_final_emit(const RhoFinalArgs<T>& A, int k, double re
     o[5] = -e * b * kv[0] * kv[2];
     o[6] = -e * b * kv[1] * kv[2];
     if (k == 0 && A.step_dev) *A.step_dev += 1ull;
+    return kc;
 }
 
 // Beside the tile pass (TileRho): one wave per k, NT / 64 k's per workgroup

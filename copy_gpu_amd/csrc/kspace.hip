@@ -113,6 +113,10 @@ void launch_rho(Engine& e, const double* x, const double* y, const double* z, hi
 {
     int blocks;
     unsigned long long* step_dev = e.capturing ? e.d_step : nullptr;
+    if (e.ew.on) {
+        launch_ewald_rho(e, x, y, z, step_dev, s);
+        return;
+    }
     {
         ScopedTimer t(e, P_RHO, s);
         if (e.precision == 32) {
@@ -137,6 +141,10 @@ void launch_rho(Engine& e, const double* x, const double* y, const double* z, hi
 void launch_kforce(Engine& e, const double* x, const double* y, const double* z, void* fx,
                    void* fy, void* fz, hipStream_t s)
 {
+    if (e.ew.on) {
+        launch_ewald_force(e, x, y, z, (double*)fx, (double*)fy, (double*)fz, s);
+        return;
+    }
     ScopedTimer t(e, P_KFORCE, s);
     if (e.precision == 32)
         k_one<KForce<float, false>><<<kforce_blocks(e), kKfThreads, 0, s>>>(

@@ -33,6 +33,7 @@ struct LatGeom {
     int nc, rblk, cblk;    // 16-column tiles per workgroup; row and column blocks
     int nx, ny;            // LDS table rows of the x and y axes
     int slices, aps;       // atom slices and atoms per slice
+    int max_slices;        // most slices of any atom count up to this one
     size_t lds;
     RBMD_HD int64_t sums() const { return R * (int64_t)C; }
 };
@@ -44,7 +45,48 @@ void launch_lattice_sums(const LatGeom& g, const Box& box, int64_t n, const doub
                          const double* y, const double* z, const double* q, double* part,
                          hipStream_t s);
 
+// Full Ewald of a handle on its lattice box (ewald.hip).
+struct EwaldLat {
+    bool on = false;
+    int M[3] = {0, 0, 0};
+    int ntile = 0;               // 16-row tiles of the (a, b) rows
+    int32_t steps = 0;           // pairs of 4-column steps over all tiles
+    int32_t* idx = nullptr;      // [octant point][4] k-list index or -1
+    int32_t* pairs = nullptr;    // [64-column block][tile] pairs of steps
+    int32_t* before = nullptr;   // [tile] pairs of steps before the tile
+    double* D = nullptr;         // force coefficients in fragment order
+    double* part = nullptr;      // lattice sums
+    double* fpart = nullptr;     // force shares
+};
+
+// Position of D[row][c]: per 64-column block and tile, lane (c % 4) 16 + row % 16 holds its
+// value of step (c % 64) / 4, two steps side by side.
+RBMD_HD inline int64_t ewald_d_pos(const EwaldLat& l, int row, int c)
+{
+    const int s = (c & 63) >> 2, lane = (c & 3) * 16 + (row & 15);
+    return ((int64_t)(c >> 6) * l.ntile + (row >> 4)) * 1024 + (s >> 1) * 128 + lane * 2 + (s & 1);
+}
+
 #ifdef __HIPCC__
+using d4 = double __attribute__((ext_vector_type(4)));
+
+// Fraction s = t / L of a box edge as an unevaluated sum hi + lo, and the sine and cosine of
+// m s turns, the phase reduced exactly up to the rounding of the reduced value.
+struct LatFrac {
+    double hi, lo;
+};
+__device__ inline LatFrac lat_frac(double t, double L, double invL)
+{
+    const double h = t * invL;
+    return {h, fma(-h, L, t) * invL};
+}
+__device__ inline void lat_sincos(const LatFrac& s, int m, double* sn, double* cs)
+{
+    const double md = (double)m, p = md * s.hi;
+    const double f = (p - rint(p)) + (fma(md, s.hi, -p) + md * s.lo);
+    sincospi(2.0 * f, sn, cs);
+}
+
 // The eight sums of an octant point, axes x, y, z as bits 2, 1, 0 (1: sine).
 struct LatOct {
     double t[8];

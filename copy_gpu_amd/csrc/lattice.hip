@@ -13,25 +13,6 @@ namespace rbmd {
 
 namespace {
 
-using d4 = double __attribute__((ext_vector_type(4)));
-
-// Fraction s = t / L of a box edge as an unevaluated sum hi + lo, and the phase of m s
-// reduced to [-1/2, 1/2] turns: exact up to the rounding of the reduced value.
-struct Frac {
-    double hi, lo;
-};
-__device__ inline Frac lat_frac(double t, double L, double invL)
-{
-    const double h = t * invL;
-    return {h, fma(-h, L, t) * invL};
-}
-__device__ inline void lat_sincos(const Frac& s, int m, double* sn, double* cs)
-{
-    const double md = (double)m, p = md * s.hi;
-    const double f = (p - rint(p)) + (fma(md, s.hi, -p) + md * s.lo);
-    sincospi(2.0 * f, sn, cs);
-}
-
 struct LatSumArgs {
     const double *x, *y, *z, *q;
     int64_t n;
@@ -102,7 +83,7 @@ __global__ __launch_bounds__(256, 2) void k_lat_sums(LatSumArgs A)
         const int fo = (int)((j - j0) & (kLatLoad - 1));
         if (fo == 0) {
             const int64_t i = j + t;
-            Frac s[3] = {{0, 0}, {0, 0}, {0, 0}};
+            LatFrac s[3] = {{0, 0}, {0, 0}, {0, 0}};
             double q = 0.0;
             if (i < j1) {
                 s[0] = lat_frac(A.x[i] - A.box.lo[0], A.box.L[0], A.box.invL[0]);
@@ -120,7 +101,7 @@ __global__ __launch_bounds__(256, 2) void k_lat_sums(LatSumArgs A)
         for (int e = grp; e < items; e += kGrp) {
             const int d = e < kLatBase ? 1 : e < 2 * kLatBase ? 2 : 0;
             const int m = d == 0 ? mx0 + e - 2 * kLatBase : (e & (kLatBase - 1)) + 1;
-            const Frac s{frac[(2 * d) * kLatLoad + fo + at], frac[(2 * d + 1) * kLatLoad + fo + at]};
+            const LatFrac s{frac[(2 * d) * kLatLoad + fo + at], frac[(2 * d + 1) * kLatLoad + fo + at]};
             double sn, cs;
             lat_sincos(s, m, &sn, &cs);
             if (d == 0) {
@@ -270,6 +251,7 @@ LatGeom lat_geometry(const int M[3], int64_t n)
     int64_t want = std::max<int64_t>(1, kLatTargetWg / ((int64_t)g.rblk * g.cblk));
     want = std::min(want, std::max<int64_t>(1, kLatMaxPart / g.sums()));
     want = std::min(want, std::max<int64_t>(1, n / (2 * kLatStage)));
+    g.max_slices = (int)want;
     const int64_t per = (n + want - 1) / want;
     g.aps = (int)std::max<int64_t>(kLatStage, (per + kLatStage - 1) / kLatStage * kLatStage);
     g.slices = (int)std::max<int64_t>(1, (n + g.aps - 1) / g.aps);

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "engine.h"
+#include "lattice.h"
 #include "launch.h"
 #include "../../include/rbmd_force.h"
 
@@ -128,6 +129,7 @@ struct Engine {
     double S = 0;             // RBE normaliser H_x H_y H_z - 1
     unsigned long long* d_step = nullptr;  // device step counter for graph replays
     bool kvec_weights_default = true;
+    EwaldLat ew;          // FP64 full Ewald on its lattice box (ewald.hip)
     // learned proposal tables (device), active when gp.cdf != nullptr
     GridProposal gp{};
     double* gp_cdf = nullptr;
@@ -315,6 +317,12 @@ SampleArgs sample_args(const Engine& e, int P, uint64_t seed, const uint64_t* st
 void rho_geometry(const Engine& e, int* atoms_per_block, int* nbx, int* nkt);
 void launch_sample(Engine& e, int P, uint64_t seed, const uint64_t* step_host, hipStream_t s);
 void launch_kweights_default(Engine& e, hipStream_t s);
+hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m);
+void ewald_free(Engine& e);
+void launch_ewald_rho(Engine& e, const double* x, const double* y, const double* z,
+                      unsigned long long* step_dev, hipStream_t s);
+void launch_ewald_force(Engine& e, const double* x, const double* y, const double* z, double* fx,
+                        double* fy, double* fz, hipStream_t s);
 void launch_rho(Engine& e, const double* x, const double* y, const double* z, hipStream_t s);
 void launch_kforce(Engine& e, const double* x, const double* y, const double* z, void* fx,
                    void* fy, void* fz, hipStream_t s);

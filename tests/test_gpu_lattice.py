@@ -61,3 +61,43 @@ def test_spectrum_refuses_what_it_cannot_take():
     with pytest.raises(AssertionError):
         PR.spectrum([(x[:4], x, x)], q, (9.0, 9.0, 9.0), 0.5, 4)
     assert not PR.spectrum([], q, (9.0, 9.0, 9.0), 0.5, 4).any()
+
+
+# full Ewald in FP64 through the lattice box: 64-column blocks (1 to 3), a wide row basis, and
+# atom counts around a wave's 16 and a workgroup's 64
+@pytest.mark.parametrize("L,n", [((6.0, 7.0, 6.5), 2), ((6.0, 7.0, 6.5), 17), ((9.0, 7.0, 25.0), 64),
+                                 ((7.0, 60.0, 9.0), 300), ((7.0, 9.0, 60.0), 257),
+                                 ((31.0, 6.0, 8.0), 65)])
+def test_ewald_against_oracle(L, n):
+    import oracle
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    rng = np.random.default_rng(n)
+    Lb, lo = np.array(L), np.array([0.5, -1.0, 0.0])
+    alpha, tol = 0.5, 1e-12
+    # a jittered lattice: no pair much closer than its spacing
+    g = np.ceil((n / Lb.prod()) ** (1 / 3) * Lb).astype(int) + 1
+    cell = np.stack(np.meshgrid(*[np.arange(k) for k in g], indexing="ij"), -1).reshape(-1, 3)
+    pick = cell[rng.permutation(len(cell))[:n]]
+    pos = lo + (pick + 0.5 + rng.uniform(-0.15, 0.15, (n, 3))) * (Lb / g)
+    x, y, z = (np.ascontiguousarray(pos[:, d]) for d in range(3))
+    q = rng.uniform(-1.0, 1.0, n)
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=L, box_lo=tuple(lo), cut_off=2.5, coulomb_cut=2.9,
+                                         skin=0.3, alpha=alpha, kspace="EWALD", precision=64,
+                                         ewald_tol=tol, n_max=n + 7))
+    dev = lambda a: torch.as_tensor(a).cuda()  # noqa: E731
+    f.Init(dev(q))
+    X, F = [dev(a) for a in (x, y, z)], [torch.zeros(n, device="cuda", dtype=torch.float64)
+                                         for _ in range(3)]
+    for _ in range(2):  # the second evaluation finds the first's sums and coefficients
+        f.Execute(*X, *F, energy_virial=True)
+    m, w, re, im = f.kspace()
+    got = torch.stack(F, 1).cpu().numpy()
+    Fk, evk = oracle.kspace_forces(x - lo[0], y - lo[1], z - lo[2], q, Lb, alpha, m, w)
+    Fp, _ = oracle.pair_forces(x, y, z, q, lo, Lb, 2.5, 2.9, alpha)
+    # the pair part agrees to 1e-12 of itself elsewhere; the k-space part is judged on its own
+    assert np.linalg.norm(got - Fp - Fk) <= 1e-12 * (np.linalg.norm(Fp) + np.linalg.norm(Fk))
+    r, i = _direct(pos.T, q, m, lo, Lb)
+    bound = np.abs(q).sum() * (2 * np.pi * 4 * np.abs(m).max() + 16 + n / 8) * 2.0 ** -53
+    assert np.abs(re - r).max() <= bound and np.abs(im - i).max() <= bound
+    assert abs(f.energy_virial()["e_kspace"] - evk[0]) <= 1e-12 * abs(evk[0])
