@@ -449,9 +449,9 @@ __device__ inline void pair_wave(const PairArgs& a, const TileHdr& h, const Full
 }
 
 // Per-workgroup FP64 energy / virial partial: wave sums, then the 8 waves in order.
-__device__ inline void block_ev(const double* acc, int lane, int wv, double* __restrict__ out)
+__device__ inline void block_ev(const double* acc, int lane, int wv, double (*red)[8],
+                                double* __restrict__ out)
 {
-    __shared__ double red[kTileWaves][8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         const double v = wave_sum_dpp(acc[k]);
@@ -467,9 +467,9 @@ __device__ inline void block_ev(const double* acc, int lane, int wv, double* __r
 
 // Per-workgroup FP64 sums of the near forces (random batch list): wave sums, then
 // the 8 waves in order.
-__device__ inline void block_fsum(const double* fs, int lane, int wv, double* __restrict__ out)
+__device__ inline void block_fsum(const double* fs, int lane, int wv, double (*red)[3],
+                                  double* __restrict__ out)
 {
-    __shared__ double red[kTileWaves][3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const double v = wave_sum_dpp(fs[k]);
@@ -542,6 +542,12 @@ struct TilePass {
         int32_t* ltype = (int32_t*)(lds + A.stage_cap);
         const FullStage fst{(char*)lds, 16u * (uint32_t)A.stage_cap};
         __shared__ TileHdr h;
+        // the build's row counts, then the reductions at the end: one block, as the stage is
+        // sized to leave 2,048 bytes for this and the header
+        constexpr size_t kEvBytes = EV ? kTileWaves * 8 * sizeof(double) : 0;
+        constexpr size_t kRedBytes = kEvBytes + (RBL ? kTileWaves * 3 * sizeof(double) : 0);
+        __shared__ __align__(16) char scratch[std::max(sizeof(ListRows), kRedBytes)];
+        static_assert(sizeof(TileHdr) + sizeof scratch <= 2048, "fits beside the stage");
         const int tb = A.order ? A.order[blk] : blk;
         const int c = tb / A.split, part = tb % A.split;
         const bool rebuild = A.flags[2] != 0u;
@@ -577,7 +583,8 @@ struct TilePass {
                               R.ncount,
                               R.stats};
             const RblBuild rb{R.rbl.seed, epoch, R.rbl.pice, R.a.perm};
-            list_tile<RBL>(h, la, lds, R.stage_cap, R.list_rows, staged, a0, a1, h0, wv, lane, rb);
+            list_tile<RBL>(h, la, lds, *(ListRows*)scratch, R.stage_cap, R.list_rows, staged, a0, a1,
+                           h0, wv, lane, rb);
             __syncthreads();  // rows and LDS are reused below
         }
         if (staged) {
@@ -619,8 +626,10 @@ struct TilePass {
             pair_wave<T, EV, MULTI, false, RBL>(a, h, FullStage{}, nullptr, a0, a1, h0, wv, lane,
                                                 A.ps, A.pp, A.fx, A.fy, A.fz, acc, A.rbl, epoch,
                                                 fsum);
-        if (EV) block_ev(acc, lane, wv, A.ev_part + (size_t)tb * 8);
-        if (RBL) block_fsum(fsum, lane, wv, A.rbl.part + (size_t)tb * 3);
+        if (EV) block_ev(acc, lane, wv, (double(*)[8])scratch, A.ev_part + (size_t)tb * 8);
+        if (RBL)
+            block_fsum(fsum, lane, wv, (double(*)[3])(scratch + kEvBytes),
+                       A.rbl.part + (size_t)tb * 3);
         if (A.md) {
             // bins of the next rebuild: clear this step's buffer (consumed by the
             // cell sort) for this cell, bin the current home atoms into the other
@@ -950,7 +959,10 @@ struct TilePassHalf {
             pl[AH.planes.stride] = (float)J.y[u];
             pl[2 * AH.planes.stride] = (float)J.z[u];
         }
-        if (EV) block_ev(acc, lane, wv, A.ev_part + (size_t)c * 8);
+        if (EV) {
+            __shared__ double red[kTileWaves][8];
+            block_ev(acc, lane, wv, red, A.ev_part + (size_t)c * 8);
+        }
         if (A.md) {
             const int b = (int)(A.flags[3] & 1u);
             if (threadIdx.x == 0) {

@@ -263,9 +263,8 @@ __device__ inline int tile_seg(const TileHdr& h, int u)
 // formed on the matrix cores in FP32, |j|^2 - 2 i.j + (|i|^2 - t) for 16 home atoms x
 // 16 candidates per v_mfma_f32_16x16x4_f32 (positions relative to the home cell's
 // centre): the sign bits are the hits, and those of the same values moved to the
-// LJ range are its entries.  Rows with a value within rounding (list_margin) of a
-// threshold (about 1% of them) are built by the exact criterion instead, so the rows
-// hold exactly the pairs that it accepts.
+// LJ range are its entries.  A value within rounding (list_margin) of a threshold is
+// settled by the exact criterion, so the rows hold exactly the pairs that it accepts.
 //
 // Steps, per block of up to 4096 candidates staged in LDS (float4: position and
 // |j|^2):
@@ -413,19 +412,25 @@ struct MaskRows {
 
 // Masks of NMT x 16 rows against the nch chunks of the staged block.  Word of (row,
 // wave pair, column): the pair's 2T chunks, the first in bit 2T - 1 (W: uint32 for
-// T <= 16, else uint64, built in two halves).  slow: bit per row.  Per 256 pairs 32 cycles
-// of a SIMD's matrix core and 18 VALU instructions (two sign bits, the LJ-range shift
-// and the smallest distances from the thresholds).
+// T <= 16, else uint64, built in two halves).  cb: tile index of the block's first
+// candidate.  Per 256 pairs 32 cycles of a SIMD's matrix core and 18 VALU instructions (two
+// sign bits, the LJ-range shift and the smallest distances from the thresholds).
+//
+// A lane that finds one of its values within rounding of a threshold settles it at once by
+// the exact criterion (about one pair in 130,000).  Building the whole row again by that
+// criterion, 2,000 candidates by one wave, took longer than all the other rows of a
+// workgroup: 7 us of the 23 of a build at 5,775 ions, 12 of 23 at 2,000.
 template <int NMT, typename H>
-__device__ inline void near_masks(const ListArgs& a, const float4* cand, const MaskRows& R,
-                                  const ListLds& L, unsigned long long* slow, int row0, int nch,
+__device__ inline void near_masks(const TileHdr& h, const ListArgs& a, const float4* cand,
+                                  const MaskRows& R, const ListLds& L, int cb, int row0, int nch,
                                   int T, int wv, int lane_in)
 {
     const int lane = opaque(lane_in), col = lane & 15, q = lane >> 4;
     const int tw = min(T, nch - wv * T);
     const float t0 = (float)(a.rl2 - 1e-4);         // d = d2 - t0
     const float tin = (float)(a.rl2 - 1e-4 - a.tag2);  // d + tin = d2 - tag2
-    float av[NMT], near[NMT], dmin = 3.0e38f;
+    const float tiny = 2e-4f - t0 + a.margin;  // x below: d2 within rounding of 1e-4
+    float av[NMT];
     list_f4 c[NMT];
     uint32_t hit[NMT][4], in[NMT][4];
 #pragma unroll
@@ -442,7 +447,6 @@ __device__ inline void near_masks(const ListArgs& a, const float4* cand, const M
         av[m] = q == 3 ? 1.0f : -2.0f * fq;
         // rows past the last: far from everything
         const float w = 16 * m + col < R.nrow ? f.w - t0 : 1.0e30f;
-        near[m] = 3.0e38f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             c[m][r] = __shfl(w, 4 * q + r, 64);
@@ -467,6 +471,7 @@ __device__ inline void near_masks(const ListArgs& a, const float4* cand, const M
                 for (int r = 0; r < 4; ++r)
                     if (uc + col == R.u0 + 16 * m + 4 * q + r) d[m][r] = 1.0e30f;
         }
+        float near = 3.0e38f, dmin = 3.0e38f;
 #pragma unroll
         for (int m = 0; m < NMT; ++m)
 #pragma unroll
@@ -474,12 +479,37 @@ __device__ inline void near_masks(const ListArgs& a, const float4* cand, const M
                 const float x = d[m][r], y = x + tin;
                 hit[m][r] = __builtin_amdgcn_alignbit(hit[m][r], __float_as_uint(x), 31);
                 in[m][r] = __builtin_amdgcn_alignbit(in[m][r], __float_as_uint(y), 31);
-                near[m] = fminf(fminf(near[m], fabsf(x)), fabsf(y));
+                near = fminf(fminf(near, fabsf(x)), fabsf(y));
                 dmin = fminf(dmin, x);
             }
+        if (near < a.margin || dmin < tiny) {
+#pragma clang fp contract(off)
+            // bit e = 4 m + r: the values to settle, then their exact bits
+            uint32_t todo = 0u, eh = 0u, ei = 0u;
+#pragma unroll
+            for (int e = 0; e < 4 * NMT; ++e) {
+                const float x = d[e >> 2][e & 3], y = x + tin;
+                if (fabsf(x) < a.margin || fabsf(y) < a.margin || x < tiny) todo |= 1u << e;
+            }
+            const double4 pj = stage_ref(h, a.xs_ref, cb + uc + col);
+            for (uint32_t w = todo; w != 0u; w &= w - 1u) {
+                const int e = __ffs((int)w) - 1;
+                const double4 pi = a.xs_ref[R.s0 + 16 * (e >> 2) + 4 * q + (e & 3)];
+                const double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+                const double d2 = fma(dz, dz, fma(dy, dy, dx * dx));
+                if ((a.rl2 - d2) > 1e-4 && d2 > 1e-4) eh |= 1u << e;
+                if (d2 < a.tag2) ei |= 1u << e;
+            }
+#pragma unroll
+            for (int e = 0; e < 4 * NMT; ++e) {
+                const uint32_t b = (todo >> e) & 1u;
+                uint32_t &hb = hit[e >> 2][e & 3], &ib = in[e >> 2][e & 3];
+                hb = (hb & ~b) | ((eh >> e) & 1u & b);
+                ib = (ib & ~b) | ((ei >> e) & 1u & b);
+            }
+        }
     }
     const int sh = T - (tw > 0 ? tw : 0);
-    const bool tiny = dmin < 2e-4f - t0 + a.margin;  // d2 within rounding of 1e-4
 #pragma unroll
     for (int m = 0; m < NMT; ++m) {
 #pragma unroll
@@ -489,10 +519,6 @@ __device__ inline void near_masks(const ListArgs& a, const float4* cand, const M
             H* w = (H*)L.mask + (((row * 4 + (wv >> 1)) * 16 + col) * 2 + (1 - (wv & 1)));
             w[0] = tw > 0 ? (H)(hit[m][r] << sh) : (H)0;
             w[L.mask_bytes / (int)sizeof(H)] = tw > 0 ? (H)(in[m][r] << sh) : (H)0;
-        }
-        if (near[m] < a.margin || tiny) {
-            const int row = row0 + 16 * m + 4 * q;
-            atomicOr(slow, 0xfull << row);
         }
     }
 }
@@ -521,9 +547,8 @@ __device__ inline int lead0(uint64_t v) { return __clzll((long long)v); }
 // gave the row.  The last block writes the row.
 template <bool RBL, typename W, bool SINGLE>
 __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListLds& L, int row,
-                                int s, int ui, const float4* cand, const float4* home, int cb,
-                                int cn, const int32_t* ids, int T, int lane_in, bool last,
-                                bool slow, int2 have, const RblBuild& rb)
+                                int s, int cb, const int32_t* ids, int T, int lane_in, bool last,
+                                int2 have, const RblBuild& rb)
 {
     const int lane = opaque(lane_in);
     const int cap = a.cap, total = h.off[27];
@@ -544,7 +569,7 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
         return __popcll(m);
     };
     bool ordered = RBL;  // the others already stand behind the LJ range
-    if (!slow) {
+    {
         constexpr int kBits = 8 * sizeof(W);
         const int wo = (row * 4 + g) * 16 + col;
         W m, mi;
@@ -601,44 +626,6 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
             ci += ni;
             co += no;
         }
-    } else {
-        // some candidate within rounding of a threshold: every candidate's FP32 distance
-        // (as differences, off by at most 13 u R^2) and the exact criterion for those near
-        // a threshold
-        float4 pi;
-        if (home) {
-            pi = home[row];
-        } else {
-            const double4 p = a.xs_ref[s];
-            pi = list_pos(a, p.x, p.y, p.z);
-        }
-        const float thr = (float)(a.rl2 - 1e-4), tag = (float)a.tag2;
-        for (int k0 = 0; k0 < cn; k0 += 64) {
-            const int k = min(k0 + lane, cn - 1), u = cb + k;
-            const float4 pj = cand[k];
-            const float fx = pj.x - pi.x, fy = pj.y - pi.y, fz = pj.z - pi.z;
-            const float f2 = fmaf(fz, fz, fmaf(fy, fy, fx * fx));
-            const bool live = k0 + lane < cn && u != ui;
-            bool hit = live && f2 < thr, in = f2 < tag;
-            const bool near = live && (fabsf(f2 - thr) < a.margin || fabsf(f2 - tag) < a.margin ||
-                                       f2 < 1e-4f + a.margin);
-            if (near) {
-#pragma clang fp contract(off)
-                const double4 e = stage_ref(h, a.xs_ref, u), pd = a.xs_ref[s];
-                const double dx = e.x - pd.x, dy = e.y - pd.y, dz = e.z - pd.z;
-                const double d2 = fma(dz, dz, fma(dy, dy, dx * dx));
-                hit = (a.rl2 - d2) > 1e-4 && d2 > 1e-4;
-                in = d2 < a.tag2;
-            }
-            if (RBL) {
-                bool sel = false;
-                if (hit) sel = rbl_select(rb.seed, rb.epoch, id_i, ids[u - cb], rb.pice);
-                ci += put(hit && (in || sel), true, sel ? (u | kRblSel) : u, ci);
-            } else {
-                ci += put(hit && in, true, u, ci);
-                co += put(hit && !in, false, u, co);
-            }
-        }
     }
     if (!last) return make_int2(ci, co);
     const int n = ci + co;
@@ -673,11 +660,9 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
     return make_int2(ci, co);
 }
 
-// LDS of the build besides the stage: entries per row over the blocks of one tile,
-// and the rows to build by the exact criterion.
+// LDS of the build besides the stage: entries per row over the blocks of one tile.
 struct ListRows {
     int2 cnt[64];
-    unsigned long long slow;
 };
 
 // One block of the build: masks, then rows, for the row group [0, nrow) of home atoms
@@ -690,29 +675,21 @@ __device__ inline void list_block(const TileHdr& h, const ListArgs& a, const Lis
 {
     using H = typename std::conditional<sizeof(W) == 4, uint16_t, uint32_t>::type;
     const int nch = (cn + 15) / 16, T = (nch + kTileWaves - 1) / kTileWaves;
-    // A row or two per wave of a small tile: the wave sweeps the candidates itself.  The
-    // sweep takes about cn / 2 VALU instructions a row; the masks about cn / 3 + 100 a wave,
-    // 185 a row and a barrier.
-    const bool sweep = nrow <= kTileWaves ? cn < 2048 : nrow <= 2 * kTileWaves && cn < 704;
     // 32 rows at a time: more row tiles would take the tile pass past the registers
     // that its LDS stage's occupancy allows
-    for (int r0 = 0; r0 < nrow && !sweep; r0 += 32) {
+    for (int r0 = 0; r0 < nrow; r0 += 32) {
         const MaskRows R{home ? home + r0 : nullptr, s0 + r0, u0 + r0 - cb, min(32, nrow - r0)};
-        if (R.nrow > 16) near_masks<2, H>(a, cand, R, L, &lr.slow, r0, nch, T, wv, lane);
-        else near_masks<1, H>(a, cand, R, L, &lr.slow, r0, nch, T, wv, lane);
+        if (R.nrow > 16) near_masks<2, H>(h, a, cand, R, L, cb, r0, nch, T, wv, lane);
+        else near_masks<1, H>(h, a, cand, R, L, cb, r0, nch, T, wv, lane);
     }
-    if (!sweep) __syncthreads();
-    const uint32_t slow[2] = {sweep ? ~0u : (uint32_t)uniform((int)(uint32_t)lr.slow),
-                              sweep ? ~0u : (uint32_t)uniform((int)(uint32_t)(lr.slow >> 32))};
+    __syncthreads();
     for (int row = wv; row < nrow; row += kTileWaves) {
-        const bool sl = ((row < 32 ? slow[0] : slow[1]) >> (row & 31)) & 1u;
         if (single) {
-            row_hits<RBL, W, true>(h, a, L, row, s0 + row, u0 + row, cand, home, cb, cn, ids, T,
-                                   lane, true, sl, make_int2(0, 0), rb);
+            row_hits<RBL, W, true>(h, a, L, row, s0 + row, cb, ids, T, lane, true,
+                                   make_int2(0, 0), rb);
             continue;
         }
-        const int2 n = row_hits<RBL, W, false>(h, a, L, row, s0 + row, u0 + row, cand, home, cb, cn,
-                                               ids, T, lane, last, sl,
+        const int2 n = row_hits<RBL, W, false>(h, a, L, row, s0 + row, cb, ids, T, lane, last,
                                                cb > 0 ? lr.cnt[row] : make_int2(0, 0), rb);
         if (!last && lane == 0) lr.cnt[row] = n;
     }
@@ -722,11 +699,10 @@ __device__ inline void list_block(const TileHdr& h, const ListArgs& a, const Lis
 // Rows of the home atoms [a0, a1) of a tile (every thread of the workgroup).  staged:
 // the whole tile fits the LDS stage.
 template <bool RBL>
-__device__ inline void list_tile(const TileHdr& h, const ListArgs& a, double4* lds, int stage_cap,
-                                 int rows, bool staged, int a0, int a1, int h0, int wv, int lane,
-                                 const RblBuild& rb)
+__device__ inline void list_tile(const TileHdr& h, const ListArgs& a, double4* lds, ListRows& lr,
+                                 int stage_cap, int rows, bool staged, int a0, int a1, int h0,
+                                 int wv, int lane, const RblBuild& rb)
 {
-    __shared__ ListRows lr;
     const int total = h.off[27];
     if (total >= kMaxTile) {
         for (int s = a0 + (int)threadIdx.x; s < a1; s += kTileThreads) {
@@ -764,7 +740,6 @@ __device__ inline void list_tile(const TileHdr& h, const ListArgs& a, double4* l
         for (int cb = 0; cb < total; cb += blk) {
             const int cn = min(blk, total - cb);
             if (!staged) stage(cb, cn);
-            if (threadIdx.x == 0) lr.slow = 0ull;
             __syncthreads();
             const float4* cand = staged ? L.cand + cb : L.cand;
             const int32_t* ids = RBL ? (staged ? L.ids + cb : L.ids) : nullptr;
