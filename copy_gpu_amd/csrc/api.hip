@@ -113,7 +113,7 @@ static hipError_t dalloc(P** p, size_t bytes)
 static void free_all(Engine& E)
 {
     void* ptrs[] = {E.xr,       E.yr,    E.zr,     E.xs_ref, E.xs,        E.perm,     E.scell,
-                    E.ts,       E.cell_count, E.cell_start, E.atom_cell, E.atom_rank, E.nlist,
+                    E.ts,       E.cell_start, E.atom_rank, E.nlist,
                     E.tile_order,
                     E.md_count, E.md_bucket, E.md_cell, E.md_vid, E.md_w,
                     E.ncount,   E.stats, E.q,      E.type,      E.d_pp,     E.km,
@@ -441,9 +441,7 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
     CR(dalloc(&E.perm, N * 4));
     CR(dalloc(&E.scell, N * 4));
     CR(dalloc(&E.ts, N * 4));
-    CR(dalloc(&E.atom_cell, N * 4));
     CR(dalloc(&E.atom_rank, N * 4));
-    CR(dalloc(&E.cell_count, (size_t)E.ncell * 4));
     CR(dalloc(&E.tile_order, (size_t)E.ncell * E.split_max * 4));
     CR(reset_tile_order(E));
     {
@@ -492,7 +490,6 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
     CR(hipMemset(E.thermo_st, 0, 64));
     CR(hipMemset(E.ev, 0, 16 * 8));
     CR(hipMemset(E.cell_start, 0, ((size_t)E.ncell + 1) * 4));
-    CR(hipMemset(E.cell_count, 0, (size_t)E.ncell * 4));
     CR(hipMemset(E.md_count, 0, md_count_bytes(E.ncell)));
     CR(hipMemset(E.xr, 0, N * 8));
     CR(hipMemset(E.yr, 0, N * 8));
@@ -655,11 +652,8 @@ int rbmd_force_sample_kvectors(rbmd_force_t h, int32_t P, uint64_t seed, uint64_
 static int force_pass(Engine& E, const double* x, const double* y, const double* z, void* fx,
                       void* fy, void* fz, bool ev, hipStream_t s)
 {
-    launch_check(E, x, y, z, s);
     const bool ks = has_kspace(E);
-    launch_build(E, x, y, z, s);
-    launch_gather(E, x, y, z, s);
-    if (ks) launch_rho(E, x, y, z, s);
+    launch_force_lists(E, x, y, z, s);
     launch_pair(E, fx, fy, fz, ev, s);
     // a random batch list's near forces have their mean subtracted by the k-space
     // force kernel (which runs without k-vectors when there is no k-space)
@@ -726,7 +720,8 @@ int rbmd_force_compute(rbmd_force_t h, const double* x, const double* y, const d
     if (rc != RBMD_OK) return rc;
     force_pass(E, x, y, z, fx, fy, fz, (flags & RBMD_EV) != 0, s);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(E.h_stats, E.stats, 64, hipMemcpyDeviceToHost, s));
+    // (full rows that overflow tell the host mirror themselves, ListArgs::host)
+    if (E.half) HIP_TRY(hipMemcpyAsync(E.h_stats, E.stats, 64, hipMemcpyDeviceToHost, s));
     return RBMD_OK;
 }
 
@@ -1275,9 +1270,7 @@ int rbmd_force_autotune(rbmd_force_t h, const double* x, const double* y, const 
     if (!te.ok) return fail(E, RBMD_ERR_HIP, "event creation failed");
     const bool ks = (E.kspace == RBMD_KSPACE_RBE || E.kspace == RBMD_KSPACE_EWALD) && E.P > 0;
     auto pass = [&]() {
-        launch_build(E, x, y, z, s);
-        launch_gather(E, x, y, z, s);
-        if (ks) launch_rho(E, x, y, z, s);
+        launch_force_lists(E, x, y, z, s);
         launch_pair(E, fx, fy, fz, false, s);
         if (ks) launch_kforce(E, x, y, z, fx, fy, fz, s);
     };
@@ -1285,9 +1278,7 @@ int rbmd_force_autotune(rbmd_force_t h, const double* x, const double* y, const 
         apply_policy(E, p);
         double sb = 0, sf = 0;
         for (int r = 0; r <= reps; ++r) {  // the first round warms up
-            // a pass that rebuilds (into a zeroed histogram: the per-step check
-            // kernel clears it in ordinary passes), then one that does not
-            (void)hipMemsetAsync(E.cell_count, 0, (size_t)E.ncell * sizeof(int32_t), s);
+            // a pass that rebuilds, then one that does not
             launch_force_rebuild(E, s);
             (void)hipEventRecord(te.ev[0], s);
             pass();
@@ -1613,25 +1604,23 @@ int rbmd_batch_autotune(rbmd_batch_t b, const rbmd_replica_state* st, int32_t re
         o.img = q.img;
         o.mass = q.mass;
     }
-    const bool ks = B.kspace == RBMD_KSPACE_RBE || B.kspace == RBMD_KSPACE_EWALD;
     auto measure = [&](const TilePolicy& p) -> double {
         for (Engine* E : B.es) apply_policy(*E, p);
         if (nlist_batch_prepare(B) != hipSuccess || pair_batch_prepare(B) != hipSuccess ||
-            md_batch_prepare(B) != hipSuccess || (ks && kspace_batch_prepare(B) != hipSuccess))
+            md_batch_prepare(B) != hipSuccess)
             return -1.0;
         auto pass = [&]() {
-            for (int ph : {BP_BIN, BP_SCAN, BP_SCATTER, BP_CELLSORT}) nlist_batch_launch(B, ph, s);
-            nlist_batch_launch(B, BP_GATHER, s);
-            if (ks) kspace_batch_launch(B, BP_RHO, s);
+            for (int ph : {BP_BIN, BP_CHUNKSUM}) nlist_batch_launch(B, ph, s);
+            md_batch_launch(B, BP_SORT_RHO, s);
             pair_batch_launch(B, BP_PAIR, s);  // rho final + tile pass
             md_batch_launch(B, BP_KFORCE, s);
         };
         double sb = 0, sf = 0;
         for (int r = 0; r <= reps; ++r) {
             for (Engine* E : B.es) {
-                // a rebuild bins into a zeroed histogram (the kick/check kernel
-                // clears it in ordinary steps)
-                (void)hipMemsetAsync(E->cell_count, 0, (size_t)E->ncell * sizeof(int32_t), s);
+                // a rebuild bins into zeroed counts (the tile pass clears them in
+                // ordinary steps)
+                (void)hipMemsetAsync(E->md_count, 0, md_count_bytes(E->ncell), s);
                 launch_force_rebuild(*E, s);
             }
             (void)hipEventRecord(te.ev[0], s);

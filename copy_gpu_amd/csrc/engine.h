@@ -10,7 +10,7 @@
 //                       ("inner") entries, then the rest ("outer"), then one sentinel
 //   ncount[n]    int2   (inner, outer) per row; (n, 0) with n >= C for a row that
 //                       did not fit
-//   cell_count/cell_start  int32 counting-sort histogram and CSR bounds
+//   cell_start   int32  CSR bounds of the cells (counts in the bins, MdBins)
 //   k-space: kvec (m, w), partial structure factors [blocks][P] (FP64), rho[P], per-k
 //   force coefficients, per-k energy/virial terms
 #pragma once

@@ -326,7 +326,7 @@ hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
 }
 
 void launch_ewald_rho(Engine& e, const double* x, const double* y, const double* z,
-                      unsigned long long* step_dev, hipStream_t s)
+                      hipStream_t s)
 {
     const EwaldLat& l = e.ew;
     {
@@ -336,7 +336,7 @@ void launch_ewald_rho(Engine& e, const double* x, const double* y, const double*
     ScopedTimer t(e, P_RHO_FINAL, s);
     const int64_t pts = (int64_t)(l.M[0] + 1) * (l.M[1] + 1) * (l.M[2] + 1);
     k_ewald_final<<<(unsigned)((pts + 255) / 256), 256, 0, s>>>(
-        rho_final_args<double>(e, step_dev), l.part, l);
+        rho_final_args<double>(e, nullptr), l.part, l);
 }
 
 void launch_ewald_force(Engine& e, const double* x, const double* y, const double* z, double* fx,

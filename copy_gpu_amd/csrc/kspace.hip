@@ -64,19 +64,6 @@ __global__ void k_fill(double* __restrict__ a, int n, double v)
     if (i < n) a[i] = v;
 }
 
-template <typename T>
-hipError_t kspace_prepare_t(Batch& b)
-{
-    const size_t R = b.es.size();
-    std::vector<typename RhoPartial<T>::Args> ra(R);
-    std::vector<int> nr(R);
-    for (size_t r = 0; r < R; ++r) {
-        const RepState& st = b.st[r];
-        ra[r] = rho_args<T>(*b.es[r], st.x, st.y, st.z, &nr[r]);
-    }
-    return phase_upload(b.ph[BP_RHO], ra, nr, 0);
-}
-
 }  // namespace
 
 // ================================================================= launchers
@@ -109,35 +96,6 @@ void launch_kweights_default(Engine& e, hipStream_t s)
     k_fill<<<(e.P + 255) / 256, 256, 0, s>>>(e.kw, e.P, e.S / (double)e.P);
 }
 
-void launch_rho(Engine& e, const double* x, const double* y, const double* z, hipStream_t s)
-{
-    int blocks;
-    unsigned long long* step_dev = e.capturing ? e.d_step : nullptr;
-    if (e.ew.on) {
-        launch_ewald_rho(e, x, y, z, step_dev, s);
-        return;
-    }
-    {
-        ScopedTimer t(e, P_RHO, s);
-        if (e.precision == 32) {
-            const auto a = rho_args<float>(e, x, y, z, &blocks);
-            k_one<RhoPartial<float>><<<blocks, kRhoBlock, 0, s>>>(a);
-        } else {
-            const auto a = rho_args<double>(e, x, y, z, &blocks);
-            k_one<RhoPartial<double>><<<blocks, kRhoBlock, 0, s>>>(a);
-        }
-    }
-    {
-        ScopedTimer t(e, P_RHO_FINAL, s);
-        if (e.precision == 32)
-            k_one<RhoFinal<float>><<<e.P, RhoFinal<float>::kThreads, 0, s>>>(
-                rho_final_args<float>(e, step_dev));
-        else
-            k_one<RhoFinal<double>><<<e.P, RhoFinal<double>::kThreads, 0, s>>>(
-                rho_final_args<double>(e, step_dev));
-    }
-}
-
 void launch_kforce(Engine& e, const double* x, const double* y, const double* z, void* fx,
                    void* fy, void* fz, hipStream_t s)
 {
@@ -152,23 +110,6 @@ void launch_kforce(Engine& e, const double* x, const double* y, const double* z,
     else
         k_one<KForce<double, false>><<<kforce_blocks(e), kKfThreads, 0, s>>>(
             kforce_args<double>(e, x, y, z, fx, fy, fz, nullptr, nullptr, nullptr, nullptr, 0.0));
-}
-
-hipError_t kspace_batch_prepare(Batch& b)
-{
-    return b.precision == 32 ? kspace_prepare_t<float>(b) : kspace_prepare_t<double>(b);
-}
-
-void kspace_batch_launch(Batch& b, int phase, hipStream_t s)
-{
-    const bool f32 = b.precision == 32;
-    switch (phase) {
-    case BP_RHO:
-        if (f32) phase_launch<RhoPartial<float>>(b.ph[phase], s);
-        else phase_launch<RhoPartial<double>>(b.ph[phase], s);
-        break;
-    default: break;
-    }
 }
 
 }  // namespace rbmd

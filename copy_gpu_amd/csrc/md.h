@@ -285,7 +285,8 @@ struct KForceDrift {
 };
 
 // ---------------------------------------------------------------- MD cell sort
-// Rebuild-step cell sort from the bins the tile pass made one step earlier
+// Rebuild-step cell sort from the bins the tile pass made one step earlier, or, in the
+// force pass, of the current positions
 // (buffer flags[3] & 1): one wave per cell, more for cells of hundreds of atoms (sort_parts).  The cell's start is the sum of the
 // counts before it; its atoms come from the bucket (arrival order) ranked by id,
 // or, for a bucket that overflowed, from a scan of every binning slot's cell.  The
@@ -438,6 +439,16 @@ struct SortRho {
                          (int32_t*)lds + wv * kSortWaveBuf);
     }
 };
+
+inline CellSortMDArgs cellsort_md_args(Engine& e, const double* x, const double* y,
+                                       const double* z)
+{
+    return CellSortMDArgs{x,       y,       z,        e.q,         e.type,
+                          (int)e.n, e.ncell, e.box,   md_bins(e),  e.cell_start,
+                          e.perm,  e.atom_rank /* inverse perm */, e.scell,
+                          e.ts,    e.xr,    e.yr,     e.zr,        e.xs_ref,
+                          e.xs,    e.flags, e.stats};
+}
 
 inline int sortrho_cell_blocks(int waves) { return (waves + kRhoBlock / 64 - 1) / (kRhoBlock / 64); }
 

@@ -50,15 +50,6 @@ KickDriftArgs<T> kickdrift_args(Engine& e, const RepState& st, double dt, const 
     return a;
 }
 
-CellSortMDArgs cellsort_md_args(Engine& e, const RepState& st)
-{
-    return CellSortMDArgs{st.x,    st.y,    st.z,     e.q,         e.type,
-                          (int)e.n, e.ncell, e.box,   md_bins(e),  e.cell_start,
-                          e.perm,  e.atom_rank /* inverse perm */, e.scell,
-                          e.ts,    e.xr,    e.yr,     e.zr,        e.xs_ref,
-                          e.xs,    e.flags, e.stats};
-}
-
 template <typename T>
 typename SortRho<T>::Args sortrho_args(Engine& e, const RepState& st, int* blocks)
 {
@@ -67,7 +58,7 @@ typename SortRho<T>::Args sortrho_args(Engine& e, const RepState& st, int* block
     if (has_kspace(e)) a.rho = rho_args<T>(e, st.x, st.y, st.z, &nr);
     else memset(&a.rho, 0, sizeof a.rho);
     a.nrho = nr;
-    a.cs = cellsort_md_args(e, st);
+    a.cs = cellsort_md_args(e, st.x, st.y, st.z);
     a.parts = sort_parts(e.n, e.ncell);
     a.nsort = sortrho_cell_blocks(e.ncell * a.parts);
     a.dims = make_int3(e.dims[0], e.dims[1], e.dims[2]);

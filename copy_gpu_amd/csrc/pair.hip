@@ -527,7 +527,7 @@ struct TilePass {
         unsigned long long* stats;
         uint16_t* nlist;
         int2* ncount;
-        int32_t* cell_count;
+        unsigned long long* host;  // ListArgs::host
         int md;        // MD step: bin the home atoms for the next rebuild
         double3 cell;  // cell edge lengths (binning)
         MdBins bins;
@@ -552,10 +552,8 @@ struct TilePass {
         const int c = tb / A.split, part = tb % A.split;
         const bool rebuild = A.flags[2] != 0u;
         if (threadIdx.x == 0) {
-            // the build kernels of this step have read the request and the cell
-            // histogram: clear both for the next step's binning
+            // the build kernels of this step have read the request
             if (blk == 0) A.flags[0] = 0u;
-            if (part == 0) A.cell_count[c] = 0;
         }
         tile_setup(c, A.dims, A.box, A.cell_start, h);
         const int total = h.off[27];
@@ -581,7 +579,8 @@ struct TilePass {
                               R.a.cap,
                               R.nlist,
                               R.ncount,
-                              R.stats};
+                              R.stats,
+                              R.host};
             const RblBuild rb{R.rbl.seed, epoch, R.rbl.pice, R.a.perm};
             list_tile<RBL>(h, la, lds, *(ListRows*)scratch, R.stage_cap, R.list_rows, staged, a0, a1,
                            h0, wv, lane, rb);
@@ -868,7 +867,6 @@ struct TilePassHalf {
         const bool rebuild = A.flags[2] != 0u;
         if (threadIdx.x == 0) {
             if (blk == 0) A.flags[0] = 0u;
-            A.cell_count[c] = 0;
         }
         half_setup(c, A.dims, A.box, A.cell_start, h);
         const int total = h.off[kHalfSegs];
@@ -1172,7 +1170,7 @@ typename TilePass<T, EV, M, RBL>::Args tile_args(Engine& e, void* fx, void* fy, 
         PairArgs{e.xs, e.ts, e.perm, e.nlist, e.ncount, e.cap},
         e.xs_ref, e.cell_start, e.split, make_int3(e.dims[0], e.dims[1], e.dims[2]), e.box,
         e.stage_cap, e.r_list * e.r_list, e.r_in * e.r_in, list_margin(e.cell), pair_list_rows(e), pair_scalars(e), e.d_pp, (T*)fx,
-        (T*)fy, (T*)fz, e.ev_part, e.flags, e.stats, e.nlist, e.ncount, e.cell_count,
+        (T*)fy, (T*)fz, e.ev_part, e.flags, e.stats, e.nlist, e.ncount, e.h_stats,
         md ? 1 : 0, make_double3(e.cell[0], e.cell[1], e.cell[2]), md_bins(e),
         tile_order_ncu(e.ncell, e.split, e.num_cu) > 0 ? e.tile_order : nullptr, rbl};
 }

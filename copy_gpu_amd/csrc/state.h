@@ -92,7 +92,7 @@ struct Engine {
     double *xr = nullptr, *yr = nullptr, *zr = nullptr;
     double4 *xs_ref = nullptr, *xs = nullptr;
     int32_t *perm = nullptr, *scell = nullptr, *ts = nullptr;
-    int32_t *cell_count = nullptr, *cell_start = nullptr, *atom_cell = nullptr,
+    int32_t *cell_start = nullptr,
             *atom_rank = nullptr;
     // tile workgroup -> (cell * split + part): load-balanced when the tiles fit about
     // one dispatch round (rebuilt with the cells; identity until then)
@@ -202,15 +202,10 @@ constexpr int kStatsOutWords = 16;
 // Phases of the batched MD step, one launch each over all replicas.
 enum BatchPh {
     BP_KICKDRIFT = 0,  // segment opening kick/drift (md.hip)
-    BP_BIN,            // force-pass list build (nlist.hip)
-    BP_SCAN,
-    BP_SCATTER,
-    BP_CELLSORT,
+    BP_BIN,            // bins of the current positions, or the gather (nlist.hip)
     BP_MDCLEAR,        // MD bin counts cleared before BP_MDBIN (nlist.hip)
     BP_MDBIN,
     BP_CHUNKSUM,       // chunk counts of the MD bins after BP_MDBIN (nlist.hip)
-    BP_GATHER,
-    BP_RHO,            // rho partials of the force pass (kspace.hip)
     BP_SORT_RHO,       // MD step: rho partials + cell sort (md.hip)
     BP_PAIR,           // rho final + tile pass (pair.hip)
     BP_KFORCE,         // k-space force + closing kick (md.hip)
@@ -250,8 +245,6 @@ hipError_t nlist_batch_prepare(Batch& b);
 void nlist_batch_launch(Batch& b, int phase, hipStream_t s);
 hipError_t pair_batch_prepare(Batch& b);
 void pair_batch_launch(Batch& b, int phase, hipStream_t s);
-hipError_t kspace_batch_prepare(Batch& b);
-void kspace_batch_launch(Batch& b, int phase, hipStream_t s);
 hipError_t md_batch_prepare(Batch& b);
 void md_batch_launch(Batch& b, int phase, hipStream_t s);
 
@@ -296,10 +289,9 @@ inline size_t md_count_bytes(int ncell)
 }
 
 // ---- launchers (nlist.hip)
-void launch_check(Engine& e, const double* x, const double* y, const double* z, hipStream_t s);
 void launch_force_rebuild(Engine& e, hipStream_t s);
-void launch_build(Engine& e, const double* x, const double* y, const double* z, hipStream_t s);
-void launch_gather(Engine& e, const double* x, const double* y, const double* z, hipStream_t s);
+void launch_force_lists(Engine& e, const double* x, const double* y, const double* z,
+                        hipStream_t s);
 void launch_md_bin(Engine& e, const double* x, const double* y, const double* z,
                    unsigned long long step0, hipStream_t s);
 void launch_list_stats(Engine& e, unsigned long long* out, hipStream_t s);
@@ -320,10 +312,9 @@ void launch_kweights_default(Engine& e, hipStream_t s);
 hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m);
 void ewald_free(Engine& e);
 void launch_ewald_rho(Engine& e, const double* x, const double* y, const double* z,
-                      unsigned long long* step_dev, hipStream_t s);
+                      hipStream_t s);
 void launch_ewald_force(Engine& e, const double* x, const double* y, const double* z, double* fx,
                         double* fy, double* fz, hipStream_t s);
-void launch_rho(Engine& e, const double* x, const double* y, const double* z, hipStream_t s);
 void launch_kforce(Engine& e, const double* x, const double* y, const double* z, void* fx,
                    void* fy, void* fz, hipStream_t s);
 

@@ -392,7 +392,17 @@ struct ListArgs {
     uint16_t* nlist;
     int2* ncount;
     unsigned long long* stats;
+    unsigned long long* host;  // pinned mirror of stats: the host reads its word 2 (rows that
+                               // overflowed) before the next evaluation, without a copy each time
 };
+
+// A row of n entries did not fit.
+__device__ inline void list_overflow(const ListArgs& a, int n)
+{
+    atomicAdd(&a.stats[2], 1ull);
+    atomicMax(&a.stats[4], (unsigned long long)n);
+    __hip_atomic_store(&a.host[2], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 typedef float list_f4 __attribute__((ext_vector_type(4)));
 
@@ -652,10 +662,7 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
     }
     if (lane == 0) {
         a.ncount[s] = n < cap ? make_int2(ci, co) : make_int2(n, 0);
-        if (n >= cap) {
-            atomicAdd(&a.stats[2], 1ull);
-            atomicMax(&a.stats[4], (unsigned long long)(n + 1));
-        }
+        if (n >= cap) list_overflow(a, n + 1);
     }
     return make_int2(ci, co);
 }
@@ -707,8 +714,7 @@ __device__ inline void list_tile(const TileHdr& h, const ListArgs& a, double4* l
     if (total >= kMaxTile) {
         for (int s = a0 + (int)threadIdx.x; s < a1; s += kTileThreads) {
             a.ncount[s] = make_int2(a.cap + 1, 0);
-            atomicAdd(&a.stats[2], 1ull);
-            atomicMax(&a.stats[4], (unsigned long long)(a.cap + 1));
+            list_overflow(a, a.cap + 1);
         }
         return;
     }

@@ -249,7 +249,10 @@ int rbmd_force_autotune(rbmd_force_t h, const double* x, const double* y, const 
  * mean milliseconds per launch and the launch count for one pass name:
  * "check", "bin", "scan", "scatter", "cellsort", "gather", "sample", "rho",
  * "rho_final", "pair" (the tile pass: Verlet rows on rebuild steps, then the pair
- * forces), "kforce", "ev_final".  In MD runs: "check" is the kick/drift kernel
+ * forces), "kforce", "ev_final".  In a force evaluation "check" holds the rho(k)
+ * partials, "bin" the gather and "cellsort" the rho(k) final reduction (FP64 full
+ * Ewald: "rho" and "rho_final"); "scan", "scatter", "list" and "gather" have no
+ * launches of their own.  In MD runs: "check" is the kick/drift kernel
  * that opens a run segment, "rho" the rho(k) partials + cell-sort kernel, "pair"
  * the rho(k) final reduction + tile pass, "kforce" the k-space force with the
  * closing kick (and the next step's kick/drift). */

@@ -1,0 +1,84 @@
+"""The force pass's cell bins and sort: chunked prefix sums (more than 16,384 cells), a cell
+beyond its bucket, one atom, atoms outside the box; positions that move with and without a
+rebuild.  The rows must equal the oracle's neighbour sets and the forces a fresh handle's."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a, dtype=torch.float64):
+    return torch.as_tensor(np.ascontiguousarray(a)).to(device="cuda", dtype=dtype)
+
+
+def _system(kind, rng):
+    """positions [3][n], box edge, cutoff"""
+    if kind == "chunked":  # 26^3 cells
+        n, L = 4001, 28.7
+        g = rng.permutation(28 ** 3)[:n]
+        pos = np.stack([g % 28, g // 28 % 28, g // 784]) + 0.5 + rng.uniform(-0.1, 0.1, (3, n))
+        return pos, L, 1.0
+    if kind == "bucket":  # 27 cells, one of them with 700 of 764 atoms
+        L = 9.6
+        g = rng.permutation(9 ** 3)[:700]
+        a = np.stack([g % 9, g // 9 % 9, g // 81]) * 0.35 + 0.1 + rng.uniform(-0.02, 0.02, (3, 700))
+        b = np.stack(np.meshgrid(*[np.arange(4)] * 3)).reshape(3, -1) * 1.4 + 3.6
+        return np.concatenate([a, b], 1), L, 2.9
+    if kind == "one":
+        return np.full((3, 1), 4.2), 9.6, 2.9
+    n = 500  # images outside the box
+    g = rng.permutation(8 ** 3)[:n]
+    pos = (np.stack([g % 8, g // 8 % 8, g // 64]) + 0.5) * 1.3 + rng.uniform(-0.1, 0.1, (3, n))
+    return pos + 10.4 * rng.integers(-1, 2, (3, n)), 10.4, 2.9
+
+
+@pytest.mark.parametrize("kind", ["chunked", "bucket", "one", "outside"])
+def test_bins_and_sort(orc, gpu, kind):
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    rng = np.random.default_rng(11)
+    pos, L, rc = _system(kind, rng)
+    n = pos.shape[1]
+    q = rng.uniform(-1, 1, n)
+    skin = 0.1 if kind == "chunked" else 0.3
+    cfg = ForceConfig(box_len=(L,) * 3, cut_off=rc, coulomb_cut=rc, alpha=0.5, skin=skin,
+                      kspace="RBE", coulomb_sample_num=70, precision=64, n_max=n)
+
+    def evaluate(f, p):
+        f.sample_kvectors(70, 5, 0)
+        F = [torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+        f.Execute(*[_dev(a) for a in p], *F)
+        return torch.stack(F).cpu().numpy()
+
+    f = LJCutCoulKspaceForce(cfg)
+    f.Init(_dev(q))
+    builds = 0
+    # the start, a step within half the skin (no rebuild), one beyond it
+    for step, move in enumerate((0.0, 0.2 * skin, 2.0 * skin)):
+        p = pos + move / np.sqrt(3.0)
+        F = evaluate(f, p)
+        st = f.stats()
+        builds += step != 1
+        assert st["builds"] == builds
+        if st["overflow_rows"]:
+            # the crowded cell's rows are longer than the mean density's: the forces are exact
+            # all the same, and the next evaluation builds longer rows
+            assert kind == "bucket" and step == 0
+            again = evaluate(f, p)
+            assert np.abs(F - again).max() <= 1e-10 * np.abs(again).max()
+            st = f.stats()
+            builds += 1
+            assert st["builds"] == builds and st["overflow_rows"] == 0
+        if step != 1:
+            w = [np.ascontiguousarray(a) for a in orc.wrap(*p, np.zeros(3), np.array([L] * 3))]
+            oo, io = orc.neighbors_images(*w, np.array([L] * 3), rc + skin)
+            og, ig = f.neighbors()
+            assert og[-1] == oo[-1]
+            for i in range(n):
+                assert np.array_equal(np.sort(ig[og[i]:og[i + 1]]), np.sort(io[oo[i]:oo[i + 1]])), i
+        # rounding: positions of about L in steps of 2^-53 L against steep pairs
+        fresh = LJCutCoulKspaceForce(cfg)
+        fresh.Init(_dev(q))
+        G = evaluate(fresh, p)
+        assert np.abs(F - G).max() <= 1e-10 * max(np.abs(G).max(), 1e-300)
