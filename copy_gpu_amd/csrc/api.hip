@@ -118,7 +118,7 @@ static void free_all(Engine& E)
                     E.md_count, E.md_bucket, E.md_cell, E.md_vid, E.md_w,
                     E.ncount,   E.stats, E.q,      E.type,      E.d_pp,     E.km,
                     E.kw,       E.kpart, E.rho,    E.kcoef,  E.kev,       E.kcdf,     E.d_step,
-                    E.ev_part,  E.ev,    E.gp_cdf,  E.gp_ratio, E.gp_guide, E.thermo_part,
+                    E.ev_part,  E.gp_cdf,  E.gp_ratio, E.gp_guide, E.thermo_part,
                     E.thermo_st, E.rbl_part, E.rbl_mean, E.planes};
     for (void* p : ptrs)
         if (p) hipFree(p);
@@ -472,7 +472,6 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
     CR(dalloc(&E.thermo_st, 64));
     E.thermo_cnt = (uint32_t*)(E.thermo_st + 4);
     E.thermo_noise = (unsigned long long*)(E.thermo_st + 6);
-    CR(dalloc(&E.ev, 16 * 8));
     E.ev_part_blocks = E.ncell * E.split_max;  // tile workgroups
     CR(dalloc(&E.ev_part, (size_t)E.ev_part_blocks * 8 * 8));
     if (E.half) CR(dalloc(&E.planes, (size_t)kHalfSegs * 3 * N * sizeof(float)));
@@ -481,21 +480,20 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
         CR(dalloc(&E.rbl_mean, 4 * 8));
         CR(hipMemset(E.rbl_mean, 0, 4 * 8));
     }
-    CR(hipHostMalloc((void**)&E.h_stats, 192, hipHostMallocDefault));
+    CR(hipHostMalloc((void**)&E.h_stats, kHostBytes, hipHostMallocDefault));
     CR(hipStreamCreateWithFlags(&E.own_stream, hipStreamNonBlocking));
     CR(hipEventCreateWithFlags(&E.order_event, hipEventDisableTiming));
     CR(hipMemset(E.flags, 0, 64));
     CR(hipMemset(E.stats, 0, 128));
     CR(hipMemset(E.d_step, 0, 64));
     CR(hipMemset(E.thermo_st, 0, 64));
-    CR(hipMemset(E.ev, 0, 16 * 8));
     CR(hipMemset(E.cell_start, 0, ((size_t)E.ncell + 1) * 4));
     CR(hipMemset(E.md_count, 0, md_count_bytes(E.ncell)));
     CR(hipMemset(E.xr, 0, N * 8));
     CR(hipMemset(E.yr, 0, N * 8));
     CR(hipMemset(E.zr, 0, N * 8));
     CR(hipMemcpy(E.d_pp, &E.pp, sizeof(PairParams), hipMemcpyHostToDevice));
-    memset(E.h_stats, 0, 64);
+    memset(E.h_stats, 0, kHostBytes);
     if ((rc = alloc_list(E, cap)) != RBMD_OK) return bail(rc);
     if (E.kspace == RBMD_KSPACE_RBE) {
         build_kcdf(E.alpha, E.box.L, E.h_kcdf, E.kM);
@@ -764,9 +762,11 @@ int rbmd_force_get_energy_virial(rbmd_force_t h, rbmd_energy_virial* out, void* 
 {
     if (!h || !out) return RBMD_ERR_INVALID;
     Engine& E = h->e;
-    double v[10];
+    // the reduction has written them to host memory; the null stream waits for the other
+    // blocking streams, should the evaluation have run on one of them
     HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
-    HIP_TRY(hipMemcpy(v, E.ev, sizeof v, hipMemcpyDeviceToHost));
+    if (stream) HIP_TRY(hipStreamSynchronize(nullptr));
+    const volatile double* v = (const volatile double*)((const char*)E.h_stats + kHostEv);
     out->e_lj = v[0];
     out->e_real = v[1];
     out->e_self = v[2];

@@ -1,6 +1,6 @@
 // kspace.hip -- Random Batch Ewald (and full Ewald) k-space launches of the
-// force pass: device k-sampler, rho(k) partials and final reduction, and the
-// per-atom k-space force (bodies in kspace.h).
+// force pass: sampler arguments, rho(k) geometry and the per-atom k-space force
+// (bodies in kspace.h; the sampler's in md.h).
 //
 // Reference (paths relative to the reference checkout):
 //   sampler target / normaliser S   rbmd/framework/model/RBEPSample.h:38-61, 87-93, 143-175
@@ -38,26 +38,6 @@ void rho_geometry(const Engine& e, int* atoms_per_block, int* nbx, int* nkt)
 
 namespace {
 
-// ---------------------------------------------------------------- sampler
-struct Sample {
-    static constexpr int kThreads = 256;
-    using Args = SampleArgs;
-    __device__ static void run(const SampleArgs& sa, int blk, int)
-    {
-        const int l = blk * 256 + threadIdx.x;
-        if (l >= sa.P) return;
-        const uint64_t step = sa.step_dev ? (uint64_t)(*sa.step_dev) : sa.step;
-        const int Ms[3] = {sa.M.x, sa.M.y, sa.M.z};
-        int m[3];
-        const double w =
-            draw_kvector(sa.seed, step, (uint32_t)l, sa.cdf, Ms, sa.gp, sa.P, sa.w, sa.w_out, m);
-        sa.km[3 * l] = m[0];
-        sa.km[3 * l + 1] = m[1];
-        sa.km[3 * l + 2] = m[2];
-        sa.kw[l] = w;
-    }
-};
-
 __global__ void k_fill(double* __restrict__ a, int n, double v)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -83,12 +63,6 @@ SampleArgs sample_args(const Engine& e, int P, uint64_t seed, const uint64_t* st
     sa.km = e.km;
     sa.kw = e.kw;
     return sa;
-}
-
-void launch_sample(Engine& e, int P, uint64_t seed, const uint64_t* step_host, hipStream_t s)
-{
-    ScopedTimer t(e, P_SAMPLE, s);
-    k_one<Sample><<<(P + 255) / 256, 256, 0, s>>>(sample_args(e, P, seed, step_host));
 }
 
 void launch_kweights_default(Engine& e, hipStream_t s)

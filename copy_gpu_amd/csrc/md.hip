@@ -13,6 +13,18 @@ namespace {
 
 inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
+// The k-vector draw of a force pass.  Its CDF searches are chains of dependent reads: 6.2 us
+// from global memory, 5.3 us with the tables in LDS.
+struct Sample {
+    static constexpr int kThreads = 256;
+    using Args = SampleArgs;
+    __device__ static void run(const SampleArgs& sa, int blk, int)
+    {
+        __shared__ double cdf[kSamplerLds];
+        sample_block(sa, blk, cdf);
+    }
+};
+
 // Thermostat constants and device state for the closing kick (type none when the
 // handle has no thermostat).
 ThermoArgs thermo_args(const Engine& e, double dt)
@@ -182,6 +194,13 @@ hipError_t md_prepare_t(Batch& b)
 }  // namespace
 
 // ================================================================= launchers
+
+void launch_sample(Engine& e, int P, uint64_t seed, const uint64_t* step_host, hipStream_t s)
+{
+    ScopedTimer t(e, P_SAMPLE, s);
+    k_one<Sample><<<ceil_div(P, Sample::kThreads), Sample::kThreads, 0, s>>>(
+        sample_args(e, P, seed, step_host));
+}
 
 void launch_md_open(Engine& e, const RepState& st, double dt, const SampleArgs& sa,
                     hipStream_t s, bool fuse_thermo)

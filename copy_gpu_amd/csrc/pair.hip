@@ -1096,7 +1096,8 @@ struct RblMean {
 };
 
 // Deterministic final reduction: pair partials [nb][8] + per-k terms [P][7]
-// + self energy -> ev[10] = {e_lj, e_real, e_self, e_k, W_xx..W_yz}.  One workgroup per
+// + self energy -> ev[10] = {e_lj, e_real, e_self, e_k, W_xx..W_yz} in pinned host memory (a
+// readback then waits for the stream and copies nothing).  One workgroup per
 // output, a fixed order of strided sums, waves and wave sums.  30,000 ions: 5 us, and 29 us
 // with the 52,800 k-vectors of a full Ewald at 6,000; one workgroup for all fifteen columns
 // took 17 and 206 us.
@@ -1122,7 +1123,8 @@ __global__ __launch_bounds__(kEvThreads) void k_ev_final(const double* __restric
     if (t == 0) {
         double r = 0.0;
         for (int w = 0; w < kEvThreads / 64; ++w) r += red[w];
-        ev[o] = o == 2 ? e_self : r;
+        if (o == 2) r = e_self;
+        __hip_atomic_store(&ev[o], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1388,7 +1390,8 @@ void launch_ev_final(Engine& e, bool with_pair, hipStream_t s)
     const int nb = with_pair ? e.ncell * e.split : 0;  // one partial per tile workgroup
                                                         // (split 1 for half tiles)
     const int P = (e.kspace != 0) ? e.P : 0;
-    k_ev_final<<<10, kEvThreads, 0, s>>>(e.ev_part, nb, e.kev, P, e.e_self, e.ev);
+    k_ev_final<<<10, kEvThreads, 0, s>>>(e.ev_part, nb, e.kev, P, e.e_self,
+                                           (double*)((char*)e.h_stats + kHostEv));
 }
 
 hipError_t pair_batch_prepare(Batch& b)

@@ -142,7 +142,6 @@ struct Engine {
     // energy / virial
     double* ev_part = nullptr;  // [blocks][8]
     int ev_part_blocks = 0;
-    double* ev = nullptr;       // [10]
 
     // NVT thermostat of rbmd_md_run (rbmd_md_set_thermostat)
     int thermo_type = 0;
@@ -158,7 +157,8 @@ struct Engine {
     int64_t thermo_log_len = 0;
     uint64_t thermo_gen = 0;          // bumped by every thermostat change (keys the MD graph)
 
-    // host pinned mirror of stats
+    // pinned host memory: mirror of stats and flags, and at byte kHostEv the ten energies and
+    // virial components
     unsigned long long* h_stats = nullptr;
 
     hipStream_t own_stream = nullptr;
@@ -185,6 +185,8 @@ struct Engine {
 
     std::string err;
 };
+
+constexpr size_t kHostEv = 192, kHostBytes = kHostEv + 10 * sizeof(double);
 
 // ---- batched replicas: device pointers of one replica's MD state
 struct RepState {
