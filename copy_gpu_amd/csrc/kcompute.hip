@@ -2,7 +2,7 @@
 // handle: structure factor rho(k) = sum_j q_j exp(i k.r_j) (per-workgroup partials,
 // then a fixed-order FP64 reduction per k with the force coefficients and per-k
 // energy / virial terms) and the k-space force scatter, with the kernel bodies of
-// the force pass (kspace.h: RhoPartial, RhoFinal, KForce).
+// the force pass (kspace.h: RhoPartial, RhoFinal, kforce_block).
 //
 // Reference (paths relative to the reference checkout):
 //   ExecutionMD::ComputeRBEEleForce      rbmd/framework/run/ExecutionMD.cpp:389-410
@@ -10,10 +10,12 @@
 //   rho(k) worklet                       rbmd/framework/run/worklet/RunWorklet.cpp:1616-1677
 //   RBE force worklet                    RunWorklet.cpp:1508-1548, ExecForceFunction.h:247-269
 //
-// rbmd_kspace_compute allocates its scratch (partials, rho, per-k coefficients and
-// terms, weights) for the call.  rbmd_kspace_compute_noalloc runs the same kernels
-// on a fixed block of device memory (`scratch` below, 4 MiB per device) and
-// allocates nothing, for callers that cannot call hipMalloc.
+// Calls of at most 4,096 atoms that ask for rho need no scratch: one workgroup per k writes
+// rho, and the force kernel forms coefficients and terms from it (1,000 atoms, 124
+// k-vectors, FP64: 92 -> 44 us a call).  For others rbmd_kspace_compute allocates its scratch (partials,
+// rho, per-k coefficients and terms, weights) for the call.  rbmd_kspace_compute_noalloc
+// runs the same kernels on a fixed block of device memory (`scratch` below, 4 MiB per
+// device) and allocates nothing, for callers that cannot call hipMalloc.
 
 #include <mutex>
 
@@ -75,36 +77,117 @@ KsLayout ks_layout(int64_t n, int P)
 
 namespace {
 
-// The k-space energy and virial: per-k terms [P][7] summed in a fixed order.
-__global__ __launch_bounds__(256) void k_kev_sum(const double* __restrict__ kev, int P,
-                                                 double* __restrict__ out)
+constexpr int kKsSmall = 4096;  // most atoms of the calls without scratch
+
+// rho(k) of at most kKsSmall atoms: one workgroup per k, each thread 16 atoms at most, so no
+// partials go through memory.  (With more atoms the loop would be longer than the reduction
+// it saves: one workgroup takes 4 us for 4,096.)
+template <typename T>
+__global__ __launch_bounds__(256) void k_ks_rho(const double* __restrict__ x,
+                                                const double* __restrict__ y,
+                                                const double* __restrict__ z,
+                                                const double* __restrict__ q, int n, Box box,
+                                                const int32_t* __restrict__ km,
+                                                double* __restrict__ rho)
 {
-    __shared__ double red[256];
-    const int t = threadIdx.x;
-    for (int c = 0; c < 7; ++c) {
-        double v = 0.0;
-        for (int k = t; k < P; k += 256) v += kev[(size_t)k * 7 + c];
-        red[t] = v;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if (t < o) red[t] += red[t + o];
-            __syncthreads();
-        }
-        if (t == 0) out[c] = red[0];
-        __syncthreads();
+#pragma clang fp contract(off)
+    __shared__ double red[4][2];
+    const int k = blockIdx.x, t = threadIdx.x;
+    const double mx = km[3 * (size_t)k], my = km[3 * (size_t)k + 1], mz = km[3 * (size_t)k + 2];
+    T br = 0, bi = 0;
+    for (int i = t; i < n; i += 256) {
+        const double sx = (x[i] - box.lo[0]) * box.invL[0], sy = (y[i] - box.lo[1]) * box.invL[1],
+                     sz = (z[i] - box.lo[2]) * box.invL[2];
+        T sn, cs;
+        sincos2pi<T>(fma(mz, sz, fma(my, sy, mx * sx)), &sn, &cs);
+        const T qa = (T)q[i];
+        br = fma_t(qa, cs, br);
+        bi = fma_t(qa, sn, bi);
     }
+    static_assert(kKsSmall <= 256 * kRhoFlush, "one T-precision block per thread");
+    const double re = wave_sum_dpp((double)br), im = wave_sum_dpp((double)bi);
+    if ((t & 63) == 0) {
+        red[t >> 6][0] = re;
+        red[t >> 6][1] = im;
+    }
+    __syncthreads();
+    if (t < 2) rho[2 * (size_t)k + t] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
 }
+
+// The k-space forces (workgroups [0, nforce)) and, one workgroup each, the seven sums of
+// energy and virial terms in a fixed order.  DIRECT: coefficients and terms from rho, by each
+// workgroup for itself; else those that the rho(k) reduction stored.
+template <typename T, bool DIRECT>
+struct KsForce {
+    static constexpr int kThreads = kKfThreads;
+    struct Args {
+        KForceArgs<T> f;
+        int nforce;
+        double alpha, qqr2e;
+        const int32_t* m;
+        const double* w;  // or null: wdef
+        double wdef;
+        const double* rho;
+        const double* kev;
+        double* ev;
+    };
+    __device__ static KCoef<T> coef(const Args& A, int k, double* ev)
+    {
+        return rho_terms<T>(A.f.box, A.alpha, A.qqr2e, A.m + 3 * (size_t)k, A.w ? A.w[k] : A.wdef,
+                            A.rho[2 * (size_t)k], A.rho[2 * (size_t)k + 1], ev);
+    }
+    __device__ static void run(const Args& A, int blk, int)
+    {
+        __shared__ KForceLds<T> L;
+        if (blk < A.nforce) {
+            kforce_block(
+                A.f, blk, L,
+                [&](int k) {
+                    if constexpr (DIRECT) {
+                        double ev[7];
+                        return coef(A, k, ev);
+                    } else {
+                        return A.f.coef[k];
+                    }
+                },
+                [](int) { return 0; },
+                [&](int i, T f0, T f1, T f2, int) {
+                    A.f.fx[i] = f0;
+                    A.f.fy[i] = f1;
+                    A.f.fz[i] = f2;
+                });
+            return;
+        }
+        double* red = (double*)&L;
+        const int c = blk - A.nforce, t = threadIdx.x;
+        double v = 0.0;
+        for (int k = t; k < A.f.P; k += kThreads) {
+            if constexpr (DIRECT) {
+                double ev[7];
+                coef(A, k, ev);
+                double e = ev[0];
+#pragma unroll
+                for (int d = 1; d < 7; ++d) e = c == d ? ev[d] : e;
+                v += e;
+            } else {
+                v += A.kev[(size_t)k * 7 + c];
+            }
+        }
+        v = wave_sum_dpp(v);
+        if ((t & 63) == 0) red[t >> 6] = v;
+        __syncthreads();
+        if (t == 0) {
+            double s = 0.0;
+            for (int w = 0; w < kThreads / 64; ++w) s += red[w];
+            A.ev[c] = s;
+        }
+    }
+};
 
 __global__ void k_fill_w(double* __restrict__ a, int n, double v)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = v;
-}
-
-__global__ void k_copy_rho(const double* __restrict__ src, int n, double* __restrict__ dst)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
 }
 
 struct KsCall {
@@ -120,24 +203,49 @@ struct KsCall {
     double* ev_out;
 };
 
+// Whether a call runs without scratch memory.
+bool ks_small(const KsCall& c) { return c.rho_out && c.n <= kKsSmall; }
+
 template <typename T>
 void ks_launch(const KsCall& c, char* buf, hipStream_t s)
 {
-    const KsLayout l = ks_layout(c.n, c.P);
-    double* kw = (double*)(buf + l.kw);
-    double* kpart = (double*)(buf + l.kpart);
-    double* rho = (double*)(buf + l.rho);
-    KCoef<T>* coef = (KCoef<T>*)(buf + l.coef);
-    double* kev = (double*)(buf + l.kev);
     Box box;
     for (int d = 0; d < 3; ++d) {
         box.lo[d] = c.lo[d];
         box.L[d] = c.L[d];
         box.invL[d] = 1.0 / c.L[d];
     }
+    KForceArgs<T> ka{};
+    ka.x = c.x;
+    ka.y = c.y;
+    ka.z = c.z;
+    ka.q = c.q;
+    ka.n = (int)c.n;
+    ka.box = box;
+    ka.P = c.P;
+    ka.fx = (T*)c.fx;
+    ka.fy = (T*)c.fy;
+    ka.fz = (T*)c.fz;
+    ka.slices = kf_slices(c.n, c.P);
+    const int nforce = c.n > 0 ? kf_blocks(c.n, ka.slices) : 0, nev = c.ev_out ? 7 : 0;
+    const double wdef = c.w ? 0.0 : rbe_S(c.alpha, c.L) / (double)c.P;
+    if (ks_small(c)) {
+        k_ks_rho<T><<<c.P, 256, 0, s>>>(c.x, c.y, c.z, c.q, (int)c.n, box, c.m, c.rho_out);
+        if (nforce + nev > 0)
+            k_one<KsForce<T, true>><<<nforce + nev, kKfThreads, 0, s>>>(
+                typename KsForce<T, true>::Args{ka, nforce, c.alpha, c.qqr2e, c.m, c.w, wdef,
+                                                c.rho_out, nullptr, c.ev_out});
+        return;
+    }
+    const KsLayout l = ks_layout(c.n, c.P);
+    double* kw = (double*)(buf + l.kw);
+    double* kpart = (double*)(buf + l.kpart);
+    double* rho = c.rho_out ? c.rho_out : (double*)(buf + l.rho);
+    KCoef<T>* coef = (KCoef<T>*)(buf + l.coef);
+    double* kev = (double*)(buf + l.kev);
     const double* w = c.w;
     if (!w) {
-        k_fill_w<<<(c.P + 255) / 256, 256, 0, s>>>(kw, c.P, rbe_S(c.alpha, c.L) / (double)c.P);
+        k_fill_w<<<(c.P + 255) / 256, 256, 0, s>>>(kw, c.P, wdef);
         w = kw;
     }
     int apb, nbx, nkt;
@@ -146,22 +254,10 @@ void ks_launch(const KsCall& c, char* buf, hipStream_t s)
         c.x, c.y, c.z, c.q, (int)c.n, apb, nbx, box, c.m, c.P, kpart});
     k_one<RhoFinal<T>><<<c.P, RhoFinal<T>::kThreads, 0, s>>>(RhoFinalArgs<T>{
         kpart, nbx, c.P, c.m, w, box, c.alpha, c.qqr2e, rho, coef, kev, nullptr});
-    KForceArgs<T> ka{};
-    ka.x = c.x;
-    ka.y = c.y;
-    ka.z = c.z;
-    ka.q = c.q;
-    ka.n = (int)c.n;
-    ka.box = box;
     ka.coef = coef;
-    ka.P = c.P;
-    ka.fx = (T*)c.fx;
-    ka.fy = (T*)c.fy;
-    ka.fz = (T*)c.fz;
-    ka.slices = kf_slices(c.n, c.P);
-    if (c.n > 0) k_one<KForce<T, false>><<<kf_blocks(c.n, ka.slices), kKfThreads, 0, s>>>(ka);
-    if (c.rho_out) k_copy_rho<<<(2 * c.P + 255) / 256, 256, 0, s>>>(rho, 2 * c.P, c.rho_out);
-    if (c.ev_out) k_kev_sum<<<1, 256, 0, s>>>(kev, c.P, c.ev_out);
+    if (nforce + nev > 0)
+        k_one<KsForce<T, false>><<<nforce + nev, kKfThreads, 0, s>>>(typename KsForce<T, false>::Args{
+            ka, nforce, c.alpha, c.qqr2e, c.m, w, wdef, rho, kev, c.ev_out});
 }
 
 thread_local std::string g_ks_err;
@@ -282,12 +378,16 @@ int rbmd_kspace_compute(const rbmd_kspace_params* p, int64_t n, const double* x,
     if (rc != RBMD_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
     char* buf = nullptr;
-    hipError_t st = hipMalloc((void**)&buf, ks_layout(n, P).total);
-    if (st != hipSuccess) return ks_fail(RBMD_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(st));
+    hipError_t st;
+    if (!ks_small(c)) {
+        st = hipMalloc((void**)&buf, ks_layout(n, P).total);
+        if (st != hipSuccess)
+            return ks_fail(RBMD_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(st));
+    }
     ks_dispatch(c, buf, s);
     st = hipGetLastError();
     hipError_t st2 = hipStreamSynchronize(s);
-    (void)hipFree(buf);
+    if (buf) (void)hipFree(buf);
     if (st != hipSuccess) return ks_fail(RBMD_ERR_HIP, std::string("launch: ") + hipGetErrorString(st));
     if (st2 != hipSuccess)
         return ks_fail(RBMD_ERR_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(st2));

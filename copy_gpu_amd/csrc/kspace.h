@@ -184,19 +184,19 @@ struct RhoFinalArgs {
     unsigned long long* step_dev;
 };
 
+// Force coefficients of one k-vector m of weight w with structure factor (re, im), and its
+// energy and virial terms ev[7].
 template <typename T>
-__device__ inline KCoef<T> rho_final_emit(const RhoFinalArgs<T>& A, int k, double re, double im)
+__device__ inline KCoef<T> rho_terms(const Box& box, double alpha, double qqr2e,
+                                     const int32_t* __restrict__ m, double w, double re, double im,
+                                     double ev[7])
 {
-    const Box& box = A.box;
-    A.rho[2 * k] = re;
-    A.rho[2 * k + 1] = im;
-    const double mm[3] = {(double)A.km[3 * k], (double)A.km[3 * k + 1], (double)A.km[3 * k + 2]};
+    const double mm[3] = {(double)m[0], (double)m[1], (double)m[2]};
     double kv[3];
     for (int d = 0; d < 3; ++d) kv[d] = 2.0 * kPi * mm[d] / box.L[d];
     const double k2 = kv[0] * kv[0] + kv[1] * kv[1] + kv[2] * kv[2];
     const double V = box.L[0] * box.L[1] * box.L[2];
-    const double w = A.kw[k];
-    const double c = w * (-4.0 * kPi) / (V * k2) * A.qqr2e;
+    const double c = w * (-4.0 * kPi) / (V * k2) * qqr2e;
     KCoef<T> kc;
     for (int d = 0; d < 3; ++d) {
         kc.m[d] = mm[d];
@@ -204,17 +204,29 @@ __device__ inline KCoef<T> rho_final_emit(const RhoFinalArgs<T>& A, int k, doubl
     }
     kc.A = (T)(c * im);
     kc.B = (T)(c * re);
+    const double e = w * (2.0 * kPi / V) * (re * re + im * im) / k2 * qqr2e;
+    const double b = 2.0 * (1.0 / k2 + 1.0 / (4.0 * alpha));
+    ev[0] = e;
+    ev[1] = e * (1.0 - b * kv[0] * kv[0]);
+    ev[2] = e * (1.0 - b * kv[1] * kv[1]);
+    ev[3] = e * (1.0 - b * kv[2] * kv[2]);
+    ev[4] = -e * b * kv[0] * kv[1];
+    ev[5] = -e * b * kv[0] * kv[2];
+    ev[6] = -e * b * kv[1] * kv[2];
+    return kc;
+}
+
+template <typename T>
+__device__ inline KCoef<T> rho_final_emit(const RhoFinalArgs<T>& A, int k, double re, double im)
+{
+    A.rho[2 * k] = re;
+    A.rho[2 * k + 1] = im;
+    double ev[7];
+    const KCoef<T> kc =
+        rho_terms<T>(A.box, A.alpha, A.qqr2e, A.km + 3 * (size_t)k, A.kw[k], re, im, ev);
     A.coef[k] = kc;
-    const double e = w * (2.0 * kPi / V) * (re * re + im * im) / k2 * A.qqr2e;
-    const double b = 2.0 * (1.0 / k2 + 1.0 / (4.0 * A.alpha));
     double* o = A.kev + (size_t)k * 7;
-    o[0] = e;
-    o[1] = e * (1.0 - b * kv[0] * kv[0]);
-    o[2] = e * (1.0 - b * kv[1] * kv[1]);
-    o[3] = e * (1.0 - b * kv[2] * kv[2]);
-    o[4] = -e * b * kv[0] * kv[1];
-    o[5] = -e * b * kv[0] * kv[2];
-    o[6] = -e * b * kv[1] * kv[2];
+    for (int c = 0; c < 7; ++c) o[c] = ev[c];
     if (k == 0 && A.step_dev) *A.step_dev += 1ull;
     return kc;
 }
@@ -346,9 +358,10 @@ struct KForceLds {
 // overlaps it), then, after the k-sum, fin(i, f0, f1, f2, pre_value) with the
 // complete force (pair force + k-space).
 // fin runs with FP contraction off in the caller's body.
-template <typename T, class Pre, class Fin>
-__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T>& L, Pre pre,
-                                    Fin fin)
+// coef(k) gives the coefficients of k-vector k.
+template <typename T, class Coef, class Pre, class Fin>
+__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T>& L, Coef coef,
+                                    Pre pre, Fin fin)
 {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -384,7 +397,7 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T
     for (int base = 0; base < P; base += kKfStage) {
         __syncthreads();
         for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
-            L.st[k] = A.coef[base + k];
+            L.st[k] = coef(base + k);
         __syncthreads();
         const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
         for (int k = slice; k < cnt; k += slices) {
@@ -425,6 +438,13 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T
         }
         fin(i, f0, f1, f2, pv);
     }
+}
+
+template <typename T, class Pre, class Fin>
+__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T>& L, Pre pre,
+                                    Fin fin)
+{
+    kforce_block(A, blk, L, [&](int k) { return A.coef[k]; }, pre, fin);
 }
 
 // Velocity and mass of atom i for the closing half kick, and the thermostat's

@@ -333,8 +333,8 @@ def kspace_compute(box_len, alpha, x, y, z, q, m, w=None, fx=None, fy=None, fz=N
     dt = torch.float32 if precision == 32 else torch.float64
     if fx is None:
         fx, fy, fz = (torch.zeros(n, device=x.device, dtype=dt) for _ in range(3))
-    rho = torch.zeros(2 * P, device=x.device, dtype=torch.float64)
-    ev = torch.zeros(7, device=x.device, dtype=torch.float64)
+    rho = torch.empty(2 * P, device=x.device, dtype=torch.float64)
+    ev = torch.empty(7, device=x.device, dtype=torch.float64)
     prm = L.KspaceParams((C.c_double * 3)(*[float(v) for v in box_lo]),
                          (C.c_double * 3)(*[float(v) for v in box_len]), float(alpha),
                          float(qqr2e), int(precision))

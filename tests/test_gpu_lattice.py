@@ -101,3 +101,52 @@ def test_ewald_against_oracle(L, n):
     bound = np.abs(q).sum() * (2 * np.pi * 4 * np.abs(m).max() + 16 + n / 8) * 2.0 ** -53
     assert np.abs(re - r).max() <= bound and np.abs(im - i).max() <= bound
     assert abs(f.energy_virial()["e_kspace"] - evk[0]) <= 1e-12 * abs(evk[0])
+
+
+# the handle-free k-space step at most / above 4,096 atoms (no scratch / scratch), one atom,
+# with and without weights, more k-vectors than one LDS stage (512)
+@pytest.mark.parametrize("n,P,weights,precision", [
+    (1, 1, True, 64), (255, 7, False, 64), (257, 600, True, 64), (4096, 124, True, 32),
+    (4097, 124, True, 64), (4097, 65, False, 32)])
+def test_kspace_compute_against_oracle(n, P, weights, precision):
+    import oracle
+    from copy_gpu_amd import force as FM
+    from copy_gpu_amd import systems
+
+    rng = np.random.default_rng(n + P)
+    Lb, alpha = np.array([11.0, 12.5, 10.0]), 0.1
+    pos = rng.uniform(0, 1, (3, n)) * Lb[:, None]
+    q = rng.uniform(-1, 1, n)
+    g = np.stack(np.meshgrid(*[np.arange(-5, 6)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    g = g[(g != 0).any(1)]
+    m = g[rng.permutation(len(g))[:P]].astype(np.int32)
+    w = rng.uniform(0.5, 2.0, P) if weights else None
+    dt = torch.float32 if precision == 32 else torch.float64
+    dev = lambda a, t=torch.float64: torch.as_tensor(np.ascontiguousarray(a)).cuda().to(t)  # noqa: E731
+    F0 = rng.normal(0, 1, (3, n))
+    F = [dev(a, dt) for a in F0]
+    F0 = np.stack([a.double().cpu().numpy() for a in F])
+    rho, ev = FM.kspace_compute(tuple(Lb), alpha, *[dev(a) for a in pos], dev(q),
+                                dev(m.reshape(-1), torch.int32), None if w is None else dev(w),
+                                *F, precision=precision)
+    if w is None:
+        _, S = systems.sample_kvectors_host(alpha, Lb, 1, 1, 0)
+        w = np.full(P, S / P)
+    Fk, evk = oracle.kspace_forces(*pos, q, Lb, alpha, m, w)
+    re, im = oracle.rho(*pos, q, Lb, m)
+    # FP32: sines of 1.3e-7, products and sums of 16 of them; FP64 as the oracle's own
+    tol = 1e-6 if precision == 32 else 1e-12
+    got = rho.cpu().numpy()
+    s = np.abs(q).sum()
+    assert np.abs(got - np.stack([re, im], 1)).max() <= tol * s
+    k = 2 * np.pi * m / Lb
+    k2 = (k * k).sum(1)
+    V = Lb.prod()
+    # each force component is a sum of P terms of at most |q| 4 pi w |k| |rho| / (V k^2), each
+    # with its own sine and structure factor
+    term = np.abs(q).max() * (4 * np.pi * w / (V * np.sqrt(k2)) * (np.hypot(re, im) + s)).sum()
+    out = np.stack([a.double().cpu().numpy() for a in F], 0) - F0
+    eps = 1.2e-7 if precision == 32 else 2.3e-16
+    assert np.abs(out.T - Fk).max() <= tol * term + 2 * eps * np.abs(F0).max()
+    e = (w * 2 * np.pi / V * (np.hypot(re, im) + tol * s) ** 2 / k2 * (4 + k2 / alpha)).sum()
+    assert np.abs(ev.cpu().numpy() - evk).max() <= 4 * tol * (e + (w * s * s / k2).sum() / V * 2 * np.pi)
