@@ -227,6 +227,7 @@ __global__ __launch_bounds__(256) void k_ewald_add(const double* __restrict__ fp
     double* f[3] = {fx, fy, fz};
     for (int d = 0; d < 3; ++d) {
         double v = 0.0;
+#pragma unroll 8
         for (int s = 0; s < split; ++s) v += fpart[((int64_t)s * 3 + d) * n + i];
         double b = f[d][i];
         if (rbl_mean) b -= rbl_mean[d];
@@ -253,9 +254,7 @@ size_t ewald_lds(const EwaldLat& l)
 void ewald_free(Engine& e)
 {
     EwaldLat& l = e.ew;
-    void* ptrs[] = {l.idx, l.pairs, l.before, l.D, l.part, l.fpart};
-    for (void* p : ptrs)
-        if (p) hipFree(p);
+    if (l.idx) hipFree(l.idx);  // the one block
     l = EwaldLat{};
 }
 
@@ -303,19 +302,27 @@ hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
     }
     fp = std::max<int64_t>(fp, e.n_max);
     const LatGeom g = lat_geometry(l.M, e.n_max);
+    // one block: the tables (uploaded together), D, the sums and the force shares
+    std::vector<int32_t> tab(idx);
+    tab.insert(tab.end(), pairs.begin(), pairs.end());
+    tab.insert(tab.end(), before.begin(), before.end());
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t dbytes = (size_t)nkb * l.ntile * 1024 * sizeof(double);
+    const size_t od = up(tab.size() * 4), op = od + dbytes,
+                 of = op + up((size_t)g.max_slices * g.sums() * 8);
+    char* m0 = nullptr;
     hipError_t st;
-    if ((st = hipMalloc((void**)&l.idx, idx.size() * 4)) != hipSuccess ||
-        (st = hipMalloc((void**)&l.pairs, pairs.size() * 4)) != hipSuccess ||
-        (st = hipMalloc((void**)&l.before, before.size() * 4)) != hipSuccess ||
-        (st = hipMalloc((void**)&l.D, dbytes)) != hipSuccess ||
-        (st = hipMalloc((void**)&l.part, (size_t)g.max_slices * g.sums() * 8)) != hipSuccess ||
-        (st = hipMalloc((void**)&l.fpart, (size_t)fp * 3 * 8)) != hipSuccess ||
-        (st = hipMemcpy(l.idx, idx.data(), idx.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
-        (st = hipMemcpy(l.pairs, pairs.data(), pairs.size() * 4, hipMemcpyHostToDevice)) !=
-            hipSuccess ||
-        (st = hipMemcpy(l.before, before.data(), before.size() * 4, hipMemcpyHostToDevice)) !=
-            hipSuccess ||
+    if (hipMalloc((void**)&m0, of + (size_t)fp * 3 * 8) != hipSuccess) {
+        (void)hipGetLastError();  // no memory for it: the sums over single k-vectors need less
+        return hipSuccess;
+    }
+    l.idx = (int32_t*)m0;
+    l.pairs = l.idx + idx.size();
+    l.before = l.pairs + pairs.size();
+    l.D = (double*)(m0 + od);
+    l.part = (double*)(m0 + op);
+    l.fpart = (double*)(m0 + of);
+    if ((st = hipMemcpy(m0, tab.data(), tab.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
         (st = hipMemset(l.D, 0, dbytes)) != hipSuccess ||
         (st = hipFuncSetAttribute((const void*)k_ewald_force,
                                   hipFuncAttributeMaxDynamicSharedMemorySize,

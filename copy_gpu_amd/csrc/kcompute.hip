@@ -30,7 +30,7 @@ namespace {
 
 // Scratch of one call, carved from one block of device memory: weights [P],
 // partial structure factors [nbx][P][2], rho [P][2], coefficients KCoef<T>[P],
-// per-k energy / virial terms [P][7].  Offsets are multiples of 256 bytes.
+// per-k energy / virial terms [7][P].  Offsets are multiples of 256 bytes.
 struct KsLayout {
     size_t kw, kpart, rho, coef, kev, total;
 };
@@ -170,7 +170,7 @@ struct KsForce {
                 for (int d = 1; d < 7; ++d) e = c == d ? ev[d] : e;
                 v += e;
             } else {
-                v += A.kev[(size_t)k * 7 + c];
+                v += A.kev[(size_t)c * A.f.P + k];
             }
         }
         v = wave_sum_dpp(v);

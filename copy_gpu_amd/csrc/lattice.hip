@@ -31,9 +31,9 @@ struct LatSumArgs {
 // further at a time (one rounding of about 2^-53 each, far below the phase's own).  The
 // positions come through LDS 256 atoms at a time, as exact box fractions.
 //
-// Bound by FP64 issue: 8 x 4 NC matrix instructions of 64 cycles per wave and stage (58% of
+// Bound by FP64 issue: 8 x 4 NC matrix instructions of 64 cycles per wave and stage (64% of
 // the cycles) and about three sines and cosines per thread.  100,000 ions, |m_d| <= 32 (5.4e10
-// operations): 1.27 ms, 43 TFLOP/s of the 72 that a large FP64 product reaches here; with a
+// operations): 1.20 ms, 45 TFLOP/s of the 72 that a large FP64 product reaches here; with a
 // sine and cosine per (m, atom) the sums took 29 ms.
 constexpr int kLatBase = 8;      // m that get a sine and cosine of their own
 constexpr int kLatLoad = 256;    // atoms per load of positions
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void k_lat_sums(LatSumArgs A)
             }
         }
         __syncthreads();
-#pragma unroll 2
+#pragma unroll
         for (int k = 0; k < kLatStage; k += 4) {
             double b[NC];
 #pragma unroll

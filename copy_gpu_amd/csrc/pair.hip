@@ -1095,7 +1095,7 @@ struct RblMean {
     }
 };
 
-// Deterministic final reduction: pair partials [nb][8] + per-k terms [P][7]
+// Deterministic final reduction: pair partials [nb][8] + per-k terms [7][P]
 // + self energy -> ev[10] = {e_lj, e_real, e_self, e_k, W_xx..W_yz} in pinned host memory (a
 // readback then waits for the stream and copies nothing).  One workgroup per
 // output, a fixed order of strided sums, waves and wave sums.  30,000 ions: 5 us, and 29 us
@@ -1116,7 +1116,7 @@ __global__ __launch_bounds__(kEvThreads) void k_ev_final(const double* __restric
     if (cp >= 0)
         for (int b = t; b < nb; b += kEvThreads) v += ev_part[(size_t)b * 8 + cp];
     if (ck >= 0)
-        for (int k = t; k < P; k += kEvThreads) v += kev[(size_t)k * 7 + ck];
+        for (int k = t; k < P; k += kEvThreads) v += kev[(size_t)ck * P + k];
     v = wave_sum(v);
     if ((t & 63) == 0) red[t >> 6] = v;
     __syncthreads();

@@ -122,7 +122,7 @@ struct Engine {
     int64_t kpart_cap = 0;    // doubles
     double* rho = nullptr;    // [P][2]
     void* kcoef = nullptr;    // KCoef<T>[P]
-    double* kev = nullptr;    // [P][7] per-k energy / virial terms
+    double* kev = nullptr;    // [7][P] per-k energy / virial terms
     double* kcdf = nullptr;   // sampler CDF tables
     int kM[3] = {0, 0, 0};
     std::vector<double> h_kcdf;
