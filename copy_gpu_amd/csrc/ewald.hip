@@ -100,9 +100,10 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
     const EwaldLat& l = A.l;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, kl = lane >> 4, al = lane & 15;
     const int B = 2 * l.M[1] + 1, C = 2 * l.M[2] + 1;
-    const int R = (2 * l.M[0] + 1) * B;
-    double* Yt = ew_lds;                                   // [2 m + (sin)][atom]
-    double* Xt = Yt + (size_t)2 * (l.M[1] + 1) * kEwStride;  // [2 (m - m0) + (sin)][atom]
+    // rows of basis value a at a + 1, so the cosine and sine of m are at 2 m and 2 m + 1 (each
+    // the other's derivative) and the constant at 1
+    double* Yt = ew_lds;
+    double* Xt = Yt + (size_t)2 * (l.M[1] + 1) * kEwStride;  // from m0 on
     const int t0 = ew_share(l, blockIdx.y, A.split),
               t1 = (int)blockIdx.y + 1 == A.split ? l.ntile : ew_share(l, blockIdx.y + 1, A.split);
     constexpr double kTwoPi = 2.0 * kPi;
@@ -117,8 +118,8 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
         lat_sincos(fy, 4, &s4, &c4);
         lat_sincos(fy, tg, &sn, &cs);
         for (int m = tg; m <= l.M[1]; m += 4) {
-            Yt[(2 * m) * kEwStride + (t & 63)] = cs;
-            Yt[(2 * m + 1) * kEwStride + (t & 63)] = sn;
+            Yt[(2 * m) * kEwStride + (t & 63)] = m ? cs : 0.0;
+            Yt[(2 * m + 1) * kEwStride + (t & 63)] = m ? sn : 1.0;
             const double c = fma(cs, c4, -(sn * s4));
             sn = fma(sn, c4, cs * s4);
             cs = c;
@@ -128,7 +129,6 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
     const int la = wv * 16 + al, ia = blockIdx.x * kEwAtoms + la;
     const int ic = ia < A.n ? ia : A.n - 1;
     const LatFrac fz = lat_frac(A.z[ic] - A.box.lo[2], A.box.L[2], A.box.invL[2]);
-    const double kx = kTwoPi / A.box.L[0], ky = kTwoPi / A.box.L[1], kz = kTwoPi / A.box.L[2];
     double F0 = 0.0, F1 = 0.0, F2 = 0.0;
     for (int kb = 0; kb * 64 < C; ++kb) {
         // columns c = 64 kb + 4 s + kl of the basis, m = (c + 1) / 2: the lane keeps to cosines
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
             lat_sincos(fz, m0, &sn, &cs);
 #pragma unroll
             for (int s = 0; s < 16; ++s) {
-                const double k = kz * (double)(m0 + 2 * s);
+                const double k = (double)(m0 + 2 * s);
                 Z[s] = sine ? (m0 + 2 * s ? sn : 1.0) : cs;
                 Zd[s] = sine ? k * cs : -(k * sn);
                 const double c = fma(cs, c2, -(sn * s2));
@@ -158,8 +158,8 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
             for (int j = tg; j < kEwX; j += 4) {
                 double sn, cs;
                 lat_sincos(fx, m0 + j, &sn, &cs);
-                Xt[(2 * j) * kEwStride + (t & 63)] = cs;
-                Xt[(2 * j + 1) * kEwStride + (t & 63)] = sn;
+                Xt[(2 * j) * kEwStride + (t & 63)] = m0 + j ? cs : 0.0;
+                Xt[(2 * j + 1) * kEwStride + (t & 63)] = m0 + j ? sn : 1.0;
             }
             __syncthreads();
             for (int tl = tb; tl < te; ++tl) {
@@ -167,32 +167,32 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
                 if (np == 0) continue;
                 const double2* Dp =
                     (const double2*)(l.D + ((int64_t)kb * l.ntile + tl) * 1024) + lane;
+                const int4 rw = ((const int4*)l.rows)[tl * 4 + kl];
                 d4 h = {0.0, 0.0, 0.0, 0.0}, hd = {0.0, 0.0, 0.0, 0.0};
+                double2 d[8];  // every load in flight before the first product
+#pragma unroll
+                for (int p = 0; p < 8; ++p)
+                    if (p < np) d[p] = Dp[p * 64];
 #pragma unroll
                 for (int p = 0; p < 8; ++p) {
                     if (p >= np) break;
-                    const double2 d = Dp[p * 64];
-                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(d.x, Z[2 * p], h, 0, 0, 0);
-                    hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d.x, Zd[2 * p], hd, 0, 0, 0);
-                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(d.y, Z[2 * p + 1], h, 0, 0, 0);
-                    hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d.y, Zd[2 * p + 1], hd, 0, 0, 0);
+                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].x, Z[2 * p], h, 0, 0, 0);
+                    hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].x, Zd[2 * p], hd, 0, 0, 0);
+                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].y, Z[2 * p + 1], h, 0, 0, 0);
+                    hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].y, Zd[2 * p + 1], hd, 0, 0, 0);
                 }
+                const int rv[4] = {rw.x, rw.y, rw.z, rw.w};
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    int r = tl * 16 + 4 * v + kl;
-                    r = r < R ? r : R - 1;  // rows beyond hold zeros
-                    const int a = r / B, b = r - a * B;
-                    const int ma = (a + 1) >> 1, mb = (b + 1) >> 1;
-                    const int sa = a > 0 && !(a & 1), sb = b > 0 && !(b & 1);
-                    const double* xp = Xt + (2 * (ma - m0)) * kEwStride + la;
-                    const double* yp = Yt + (2 * mb) * kEwStride + la;
-                    const double X = xp[sa * kEwStride], Y = yp[sb * kEwStride];
-                    const double ka = kx * (double)(sa ? ma : -ma), kb_ = ky * (double)(sb ? mb : -mb);
-                    const double Xd = ka * xp[(1 - sa) * kEwStride],
-                                 Yd = kb_ * yp[(1 - sb) * kEwStride];
-                    const double yh = Y * h[v], xh = X * h[v];
-                    F0 = fma(Xd, yh, F0);
-                    F1 = fma(Yd, xh, F1);
+                    // table rows of the x and y values of row 4 v + kl; derivatives without 2 pi / L
+                    const int ix = rv[v] & 0xffff, iy = rv[v] >> 16;
+                    const double* xp = Xt + la - 2 * m0 * kEwStride;
+                    const double X = xp[ix * kEwStride], Xp = xp[(ix ^ 1) * kEwStride];
+                    const double Y = Yt[iy * kEwStride + la], Yp = Yt[(iy ^ 1) * kEwStride + la];
+                    const double Xd = (double)(ix & 1 ? ix >> 1 : -(ix >> 1)) * Xp,
+                                 Yd = (double)(iy & 1 ? iy >> 1 : -(iy >> 1)) * Yp;
+                    F0 = fma(Xd, Y * h[v], F0);
+                    F1 = fma(Yd, X * h[v], F1);
                     F2 = fma(X * Y, hd[v], F2);
                 }
             }
@@ -208,9 +208,9 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
     F2 += __shfl_xor(F2, 32, 64);
     if (kl == 0 && ia < A.n) {
         double* o = A.fpart + (int64_t)blockIdx.y * 3 * A.n + ia;
-        o[0] = F0;
-        o[(int64_t)A.n] = F1;
-        o[(int64_t)2 * A.n] = F2;
+        o[0] = kTwoPi / A.box.L[0] * F0;
+        o[(int64_t)A.n] = kTwoPi / A.box.L[1] * F1;
+        o[(int64_t)2 * A.n] = kTwoPi / A.box.L[2] * F2;
     }
 }
 
@@ -254,7 +254,7 @@ size_t ewald_lds(const EwaldLat& l)
 void ewald_free(Engine& e)
 {
     EwaldLat& l = e.ew;
-    if (l.idx) hipFree(l.idx);  // the one block
+    if (l.rows) hipFree(l.rows);  // the one block
     l = EwaldLat{};
 }
 
@@ -303,7 +303,15 @@ hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
     fp = std::max<int64_t>(fp, e.n_max);
     const LatGeom g = lat_geometry(l.M, e.n_max);
     // one block: the tables (uploaded together), D, the sums and the force shares
-    std::vector<int32_t> tab(idx);
+    // table rows of every tile row, in the order that lanes hold them
+    std::vector<int32_t> rows((size_t)l.ntile * 16);
+    for (size_t t = 0; t < rows.size() / 16; ++t)
+        for (int k = 0; k < 16; ++k) {
+            const int64_t r = std::min<int64_t>(R - 1, (int64_t)t * 16 + 4 * (k & 3) + (k >> 2));
+            rows[t * 16 + k] = (int32_t)((r / B + 1) | (r % B + 1) << 16);
+        }
+    std::vector<int32_t> tab(rows);
+    tab.insert(tab.end(), idx.begin(), idx.end());
     tab.insert(tab.end(), pairs.begin(), pairs.end());
     tab.insert(tab.end(), before.begin(), before.end());
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -316,7 +324,8 @@ hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
         (void)hipGetLastError();  // no memory for it: the sums over single k-vectors need less
         return hipSuccess;
     }
-    l.idx = (int32_t*)m0;
+    l.rows = (int32_t*)m0;
+    l.idx = l.rows + rows.size();
     l.pairs = l.idx + idx.size();
     l.before = l.pairs + pairs.size();
     l.D = (double*)(m0 + od);

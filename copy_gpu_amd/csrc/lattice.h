@@ -51,7 +51,8 @@ struct EwaldLat {
     int M[3] = {0, 0, 0};
     int ntile = 0;               // 16-row tiles of the (a, b) rows
     int32_t steps = 0;           // pairs of 4-column steps over all tiles
-    // one block of device memory, from idx on
+    // one block of device memory, from rows on
+    int32_t* rows = nullptr;     // [tile][row % 4][row / 4]: a + 1, b + 1 of the row
     int32_t* idx = nullptr;      // [octant point][4] k-list index or -1
     int32_t* pairs = nullptr;    // [64-column block][tile] pairs of steps
     int32_t* before = nullptr;   // [tile] pairs of steps before the tile
