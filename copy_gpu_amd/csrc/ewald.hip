@@ -169,17 +169,23 @@ __global__ __launch_bounds__(256, 3) void k_ewald_force(EwForceArgs A)
                     (const double2*)(l.D + ((int64_t)kb * l.ntile + tl) * 1024) + lane;
                 const int4 rw = ((const int4*)l.rows)[tl * 4 + kl];
                 d4 h = {0.0, 0.0, 0.0, 0.0}, hd = {0.0, 0.0, 0.0, 0.0};
-                double2 d[8];  // every load in flight before the first product
+                // four pairs of steps at a time, their loads in flight together
 #pragma unroll
-                for (int p = 0; p < 8; ++p)
-                    if (p < np) d[p] = Dp[p * 64];
+                for (int p0 = 0; p0 < 8; p0 += 4) {
+                    if (p0 >= np) break;
+                    double2 d[4];
 #pragma unroll
-                for (int p = 0; p < 8; ++p) {
-                    if (p >= np) break;
-                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].x, Z[2 * p], h, 0, 0, 0);
-                    hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].x, Zd[2 * p], hd, 0, 0, 0);
-                    h = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].y, Z[2 * p + 1], h, 0, 0, 0);
-                    hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].y, Zd[2 * p + 1], hd, 0, 0, 0);
+                    for (int p = 0; p < 4; ++p)
+                        if (p0 + p < np) d[p] = Dp[(p0 + p) * 64];
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        if (p0 + p >= np) break;
+                        const int s = 2 * (p0 + p);
+                        h = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].x, Z[s], h, 0, 0, 0);
+                        hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].x, Zd[s], hd, 0, 0, 0);
+                        h = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].y, Z[s + 1], h, 0, 0, 0);
+                        hd = __builtin_amdgcn_mfma_f64_16x16x4f64(d[p].y, Zd[s + 1], hd, 0, 0, 0);
+                    }
                 }
                 const int rv[4] = {rw.x, rw.y, rw.z, rw.w};
 #pragma unroll
