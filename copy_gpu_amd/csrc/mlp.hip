@@ -166,6 +166,14 @@ __device__ inline float mlp_forward(const MlpLds& W, float f, Act1 act1, Act2 ac
     return z + W.b3[0];
 }
 
+// First of a wave's 16-sample tiles (then every grid's worth of waves): consecutive tiles go to
+// different workgroups, so that the last, partial round adds one wave to a workgroup and not
+// eight to some.
+__device__ inline int64_t mlp_first_tile()
+{
+    return (int64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+}
+
 // Bound by the VALU (32 activations per lane and 16 samples, about 2,800 cycles, against 68
 // matrix instructions of 32).  274,625 samples: 46 us; 218 us with one thread per sample.
 __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_mlp_forward(const uint16_t* __restrict__ p16,
@@ -176,8 +184,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_mlp_forward(const uint16_
     mlp_stage(p16, W, nullptr);
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
     const int64_t nt = (B + kMlpTile - 1) / kMlpTile;
-    for (int64_t tl = blockIdx.x * (int64_t)kMlpWaves + (threadIdx.x >> 6); tl < nt;
-         tl += (int64_t)gridDim.x * kMlpWaves) {
+    for (int64_t tl = mlp_first_tile(); tl < nt; tl += (int64_t)gridDim.x * kMlpWaves) {
         const int64_t s = tl * kMlpTile + c;
         const float f = s < B ? feat[4 * s + g] : 0.0f;
         auto act = [](int, int, float p) { return silu(p); };
@@ -203,8 +210,8 @@ __device__ inline void mlp_wave_sync()
 // Per 16 samples 212 matrix instructions of 32 cycles and 32 activations per lane, two waves
 // per SIMD to overlap them; eight waves share one workgroup per CU, so the staging of the
 // weights and the partial gradients (18 KB a workgroup) are paid once per CU.  35,937 samples:
-// 31 us (29 us with 512 workgroups of four waves, but the sum of twice the partials then takes
-// 11 us instead of 7); 352 us with one thread per sample and a scalar loop per parameter.
+// 27 us (with 512 workgroups of four waves the sum of twice the partials takes 11 us instead
+// of 7); 352 us with one thread per sample and a scalar loop per parameter.
 template <bool GRAD>
 __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_mlp_loss_grad(
     const uint16_t* __restrict__ p16, const float* __restrict__ feat, const float* __restrict__ y,
@@ -229,8 +236,7 @@ __global__ __launch_bounds__(64 * kMlpWaves, 2) void k_mlp_loss_grad(
     }
     double loss = 0.0;
     const int64_t nt = (B + kMlpTile - 1) / kMlpTile;
-    for (int64_t tl = blockIdx.x * (int64_t)kMlpWaves + wv; tl < nt;
-         tl += (int64_t)gridDim.x * kMlpWaves) {
+    for (int64_t tl = mlp_first_tile(); tl < nt; tl += (int64_t)gridDim.x * kMlpWaves) {
         const int64_t s = tl * kMlpTile + c;
         const bool ok = s < B;
         const float f = ok ? feat[4 * s + g] : 0.0f;
@@ -539,9 +545,9 @@ int rbmd_mlp_forward(rbmd_mlp_t h, const float* feat, int64_t B, float* out, voi
 {
     if (!h || B < 0 || (B > 0 && (!feat || !out))) return RBMD_ERR_INVALID;
     if (B == 0) return RBMD_OK;
-    // a few workgroups per CU: each stages the weights once
+    // one workgroup per CU, as the registers allow: each stages the weights once
     const int64_t nt = (B + kMlpTile - 1) / kMlpTile;
-    const int blocks = (int)std::min<int64_t>((nt + kMlpWaves - 1) / kMlpWaves, 1024);
+    const int blocks = (int)std::min<int64_t>((nt + kMlpWaves - 1) / kMlpWaves, kGradBlocks);
     k_mlp_forward<<<blocks, 64 * kMlpWaves, 0, (hipStream_t)stream>>>(h->p16, feat, B, out);
     MLP_TRY(hipGetLastError());
     return RBMD_OK;
