@@ -138,24 +138,23 @@ struct KsForce {
     }
     __device__ static void run(const Args& A, int blk, int)
     {
-        __shared__ KForceLds<T> L;
+        __shared__ typename std::conditional<DIRECT, KForceStagedLds<T>, KForceLds<T>>::type L;
         if (blk < A.nforce) {
-            kforce_block(
-                A.f, blk, L,
-                [&](int k) {
-                    if constexpr (DIRECT) {
-                        double ev[7];
-                        return coef(A, k, ev);
-                    } else {
-                        return A.f.coef[k];
-                    }
-                },
-                [](int) { return 0; },
-                [&](int i, T f0, T f1, T f2, int) {
-                    A.f.fx[i] = f0;
-                    A.f.fy[i] = f1;
-                    A.f.fz[i] = f2;
-                });
+            auto pre = [](int) { return 0; };
+            auto fin = [&](int i, T f0, T f1, T f2, int) {
+                A.f.fx[i] = f0;
+                A.f.fy[i] = f1;
+                A.f.fz[i] = f2;
+            };
+            if constexpr (DIRECT) {
+                auto of_rho = [&](int k) {
+                    double ev[7];
+                    return coef(A, k, ev);
+                };
+                kforce_block(A.f, blk, L, of_rho, pre, fin);
+            } else {
+                kforce_block(A.f, blk, L, pre, fin);
+            }
             return;
         }
         double* red = (double*)&L;

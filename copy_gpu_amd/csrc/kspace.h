@@ -17,6 +17,9 @@
 // error grows past one block), and reduces the per-workgroup partials in FP64,
 // deterministically.
 #pragma once
+#include <type_traits>
+
+#include "launch.h"
 #include "state.h"
 
 namespace rbmd {
@@ -301,9 +304,13 @@ struct RhoFinal {
 
 // ---------------------------------------------------------------- k-space force
 // Workgroup = 8 waves = 8 / s atom groups of 64 atoms (lanes, original order) x s
-// k-slices: the waves of a group take k = slice, slice + s, ... of the coefficients
-// staged in LDS (every lane reads the same k: broadcast), then the s partial forces
-// of each atom are summed in a fixed order; slice 0 completes and kicks the atoms.
+// k-slices: the waves of a group take k = slice, slice + s, ... of the coefficients,
+// then the s partial forces of each atom are summed in a fixed order; slice 0 completes
+// and kicks the atoms.  Every lane of a wave takes the same k, so its coefficients come by
+// scalar loads, four k's in flight, and are scalar operands of the arithmetic.  (From an LDS
+// stage they took three 16-byte reads per k and wave and 12 vector registers: 1,048,576 atoms
+// and 500 k-vectors 347 -> 257 us, 14 vector instructions per k and 64 atoms; 32,768 atoms and
+// P = 100 6.9 -> 5.8 us.)
 // s = 8 (64 atoms per workgroup) unless P <= kKfWideP and that would give more
 // than kKfTargetBlocks workgroups: then the fewest slices that still give that many
 // (at 100,000 atoms and P = 50, s = 4), so fewer waves repeat the per-atom work.
@@ -347,10 +354,14 @@ struct KForceArgs {
     int slices = kKfSlices;            // k-slices per atom group (kf_slices)
 };
 
+// LDS: the sums of the slices, and a stage of coefficients for those that are not in memory.
 template <typename T>
 struct KForceLds {
-    KCoef<T> st[kKfStage];
     T red[kKfSlices][3][kKfAtoms];
+};
+template <typename T>
+struct KForceStagedLds : KForceLds<T> {
+    KCoef<T> st[kKfStage];
 };
 
 // The k-space force of the atoms of workgroup blk.  Each lane of an atom-owning
@@ -360,9 +371,9 @@ struct KForceLds {
 // complete force (pair force + k-space).
 // fin runs with FP contraction off in the caller's body.
 // coef(k) gives the coefficients of k-vector k.
-template <typename T, class Coef, class Pre, class Fin>
-__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T>& L, Coef coef,
-                                    Pre pre, Fin fin)
+template <typename T, class Lds, class Coef, class Pre, class Fin>
+__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coef coef, Pre pre,
+                                    Fin fin)
 {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -395,21 +406,38 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T
         pv = pre(i);
     }
     T ax = 0, ay = 0, az = 0;
-    for (int base = 0; base < P; base += kKfStage) {
-        __syncthreads();
-        for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
-            L.st[k] = coef(base + k);
-        __syncthreads();
-        const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
-        for (int k = slice; k < cnt; k += slices) {
-            const KCoef<T>& c = L.st[k];
-            const double phi = fma(c.m[2], sz, fma(c.m[1], sy, c.m[0] * sx));
-            T sn, cs;
-            sincos2pi<T>(phi, &sn, &cs);
-            const T g = fma_t(cs, c.A, -(sn * c.B));
-            ax = fma_t(g, c.k[0], ax);
-            ay = fma_t(g, c.k[1], ay);
-            az = fma_t(g, c.k[2], az);
+    auto add = [&](const KCoef<T>& c) {
+#pragma clang fp contract(off)
+        const double phi = fma(c.m[2], sz, fma(c.m[1], sy, c.m[0] * sx));
+        T sn, cs;
+        sincos2pi<T>(phi, &sn, &cs);
+        const T g = fma_t(cs, c.A, -(sn * c.B));
+        ax = fma_t(g, c.k[0], ax);
+        ay = fma_t(g, c.k[1], ay);
+        az = fma_t(g, c.k[2], az);
+    };
+    if constexpr (std::is_same<Coef, const KCoef<T>*>::value) {
+        int k = uniform(slice);
+        // four k's loads in flight together
+        for (; k + 3 * slices < P; k += 4 * slices) {
+            const KCoef<T> c0 = const_mem(coef + k), c1 = const_mem(coef + k + slices),
+                           c2 = const_mem(coef + k + 2 * slices),
+                           c3 = const_mem(coef + k + 3 * slices);
+            __builtin_amdgcn_sched_barrier(0);
+            add(c0);
+            add(c1);
+            add(c2);
+            add(c3);
+        }
+        for (; k < P; k += slices) add(const_mem(coef + k));
+    } else {
+        for (int base = 0; base < P; base += kKfStage) {
+            __syncthreads();
+            for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
+                L.st[k] = coef(base + k);
+            __syncthreads();
+            const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
+            for (int k = slice; k < cnt; k += slices) add(L.st[k]);
         }
     }
     if (P > 0 && slices > 1) {
@@ -445,7 +473,7 @@ template <typename T, class Pre, class Fin>
 __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T>& L, Pre pre,
                                     Fin fin)
 {
-    kforce_block(A, blk, L, [&](int k) { return A.coef[k]; }, pre, fin);
+    kforce_block(A, blk, L, A.coef, pre, fin);
 }
 
 // Velocity and mass of atom i for the closing half kick, and the thermostat's
