@@ -95,7 +95,13 @@ __global__ __launch_bounds__(256) void k_ks_rho(const double* __restrict__ x,
     const int k = blockIdx.x, t = threadIdx.x;
     const double mx = km[3 * (size_t)k], my = km[3 * (size_t)k + 1], mz = km[3 * (size_t)k + 2];
     T br = 0, bi = 0;
-    for (int i = t; i < n; i += 256) {
+    // FP32: thread (tile, w) sums the 16 atoms 64 tile + w, + 4, ... as wave w of RhoPartial
+    // does, so that rounding is the same for calls of any size; FP64: strided
+    constexpr bool kBlocks = sizeof(T) == 4;
+    static_assert(kRhoFlush == 16 && kKsSmall <= 256 * kRhoFlush, "one block per thread");
+    const int step = kBlocks ? 4 : 256, i0 = kBlocks ? 64 * (t >> 2) + (t & 3) : t;
+    const int i1 = kBlocks ? min(n, 64 * (t >> 2) + 64) : n;
+    for (int i = i0; i < i1; i += step) {
         const double sx = (x[i] - box.lo[0]) * box.invL[0], sy = (y[i] - box.lo[1]) * box.invL[1],
                      sz = (z[i] - box.lo[2]) * box.invL[2];
         T sn, cs;
@@ -104,7 +110,6 @@ __global__ __launch_bounds__(256) void k_ks_rho(const double* __restrict__ x,
         br = fma_t(qa, cs, br);
         bi = fma_t(qa, sn, bi);
     }
-    static_assert(kKsSmall <= 256 * kRhoFlush, "one T-precision block per thread");
     const double re = wave_sum_dpp((double)br), im = wave_sum_dpp((double)bi);
     if ((t & 63) == 0) {
         red[t >> 6][0] = re;
