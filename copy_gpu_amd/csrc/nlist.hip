@@ -239,8 +239,7 @@ struct ChunkSum {
 };
 
 // ---------------------------------------------------------------- Verlet list
-// (row builder list_wave and stage_ref live in tile.h, shared with the fused
-// list + pair pass)
+// (the row builder list_tile lives in tile.h)
 // List statistics on demand: entries, LJ-range entries, longest row.
 __global__ __launch_bounds__(256) void k_list_stats(const int2* __restrict__ ncount, int n,
                                                     unsigned long long* __restrict__ out)
