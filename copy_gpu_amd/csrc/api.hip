@@ -445,14 +445,17 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
     CR(dalloc(&E.tile_order, (size_t)E.ncell * E.split_max * 4));
     CR(reset_tile_order(E));
     {
-        // per-cell buckets of the MD step's binning: 4x the mean population
-        // (a cell beyond it is gathered by a scan instead)
+        // per-cell buckets of the binning: 4x the mean population (an MD run gathers a cell
+        // beyond it by a scan, the force pass by the lists behind the buckets, MdBins)
         const double mean = (double)N / (double)E.ncell;
         E.bucket_cap = std::min(2048, std::max(64, ((int)(4.0 * mean) + 32 + 63) / 64 * 64));
         CR(dalloc(&E.md_count, md_count_bytes(E.ncell)));
-        CR(dalloc(&E.md_bucket, (size_t)2 * E.ncell * E.bucket_cap * 4));
+        const size_t bucket = (size_t)2 * E.ncell * E.bucket_cap * 4,
+                     spill = (size_t)E.ncell * kSpillChains * 4;
+        CR(dalloc(&E.md_bucket, bucket + spill));
+        CR(hipMemset((char*)E.md_bucket + bucket, 0xff, spill));
         CR(dalloc(&E.md_cell, N * 4));
-        CR(dalloc(&E.md_vid, N * 4));
+        CR(dalloc(&E.md_vid, 2 * N * 4));
         CR(dalloc(&E.md_w, N * 3 * 8));
     }
     CR(dalloc(&E.cell_start, ((size_t)E.ncell + 1) * 4));

@@ -68,7 +68,15 @@ struct MdBins {
     int32_t* vid;          // [n] by slot: atom id
     double *xw, *yw, *zw;  // [n] by slot: wrapped positions at the binning
     int ncell, cap, nchunk;
+    // Force pass: the atoms that their cell's bucket has no room for, in kSpillChains linked
+    // lists per cell.  Empty (-1) between evaluations: the cell sort that reads a cell's
+    // lists empties them.
+    int32_t* spill;        // [ncell][kSpillChains] first atom
+    int32_t* spill_next;   // [n] by atom
 };
+// Lists per cell: one lane of the cell sort walks each, so an atom of 1,000 beyond the
+// bucket is at most 32 dependent loads away.
+constexpr int kSpillChains = 32;
 
 // ---------------------------------------------------------------- Philox4x32-10
 // Salmon, Moraes, Dror, Shaw, "Parallel random numbers: as easy as 1, 2, 3",

@@ -284,13 +284,17 @@ struct KForceDrift {
     }
 };
 
-// ---------------------------------------------------------------- MD cell sort
-// Rebuild-step cell sort from the bins the tile pass made one step earlier, or, in the
-// force pass, of the current positions
-// (buffer flags[3] & 1): one wave per cell, more for cells of hundreds of atoms (sort_parts).  The cell's start is the sum of the
-// counts before it; its atoms come from the bucket (arrival order) ranked by id,
-// or, for a bucket that overflowed, from a scan of every binning slot's cell.  The
-// sorted slot s of atom v receives perm, inv_perm, the binned position as the
+// ---------------------------------------------------------------- cell sort
+// Rebuild-step cell sort from the bins (buffer flags[3] & 1) that the tile pass made one
+// step earlier or, in the force pass, of the current positions: one wave per cell, more for
+// cells of hundreds of atoms (sort_parts).  The cell's start is the sum of the counts before
+// it; its atoms come from the bucket (arrival order) ranked by id.  For a bucket that
+// overflowed, the force pass takes the others from the cell's lists (MdBins::spill); an MD
+// run, whose steps bin whether or not a rebuild follows, scans every binning slot's cell, as
+// the force pass does for cells of more than kSortWaveBuf atoms.  With a scan for every such
+// cell the sort of a droplet in a box 27 times its volume (cutoff 6) took 0.52 ms at 100,000
+// ions and 10.3 ms at 1,000,000; with the lists 33 us and 0.33 ms.
+// The sorted slot s of atom v receives perm, inv_perm, the binned position as the
 // new reference, the packed reference and current (unwrapped) positions, its
 // cell and type.  The wave of cell 0 publishes the rebuild decision (flags[2])
 // and resets the build statistics.
@@ -327,7 +331,8 @@ __device__ inline void cellsort_md_emit(const CellSortMDArgs& a, int c, int v, i
 
 // One wave sorts entries part * 64 + lane, + 64 parts, ... of cell c (c >= ncell:
 // nothing); buf holds kSortWaveBuf ids of this wave's own LDS.  The bucket lists binning
-// slots; atoms are ranked by id.
+// slots; atoms are ranked by id.  SPILL: the force pass, whose slots are the atoms.
+template <bool SPILL>
 __device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int part, int parts,
                                         int lane, int32_t* buf)
 {
@@ -361,35 +366,63 @@ __device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int part
         a.cell_start[c] = s0;
         if (c == a.ncell - 1) a.cell_start[a.ncell] = s0 + cnt;
     }
-    if (cnt <= a.bins.cap) {
-        const int32_t* bk = a.bins.bucket + ((size_t)b * a.ncell + c) * a.bins.cap;
-        if (cnt <= kSortWaveBuf) {
-            // ids staged in LDS, each lane ranks its own entries
-            for (int k = lane; k < cnt; k += 64) buf[k] = a.bins.vid[bk[k]];
-            __syncwarp();
-            for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {
-                const int v = buf[k];
-                int r = 0;
-                for (int t = 0; t < cnt; ++t) r += (buf[t] < v) ? 1 : 0;
-                cellsort_md_emit(a, c, v, bk[k], s0 + r);
+    const bool over = cnt > a.bins.cap;
+    const int32_t* bk = a.bins.bucket + ((size_t)b * a.ncell + c) * a.bins.cap;
+    if (SPILL && over) {
+        if (part) return;
+        parts = 1;
+    }
+    // the first atom of list `lane`, which is then empty
+    int u = -1;
+    if (SPILL && over && lane < kSpillChains) {
+        int32_t* head = a.bins.spill + (size_t)c * kSpillChains + lane;
+        u = *head;
+        *head = -1;
+    }
+    if (cnt <= kSortWaveBuf && (SPILL || !over)) {
+        // ids staged in LDS, each lane ranks its own entries
+        int found = min(cnt, a.bins.cap);
+        for (int k = lane; k < found; k += 64) buf[k] = SPILL ? bk[k] : a.bins.vid[bk[k]];
+        if (SPILL)
+            for (uint64_t m; found < cnt && (m = __ballot(u >= 0)) != 0ull; found += __popcll(m)) {
+                const int k = found + (int)mbcnt64(m);
+                if (u >= 0 && k < cnt) buf[k] = u;
+                u = u >= 0 ? a.bins.spill_next[u] : -1;
             }
-        } else {
-            for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {
-                const int v = a.bins.vid[bk[k]];
-                int r = 0;
-                for (int t = 0; t < cnt; ++t) r += (a.bins.vid[bk[t]] < v) ? 1 : 0;
-                cellsort_md_emit(a, c, v, bk[k], s0 + r);
-            }
+        __syncwarp();
+        for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {
+            const int v = buf[k];
+            int r = 0;
+            for (int t = 0; t < cnt; ++t) r += (buf[t] < v) ? 1 : 0;
+            cellsort_md_emit(a, c, v, SPILL ? v : bk[k], s0 + r);
+        }
+    } else if (!over) {
+        for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {
+            const int v = a.bins.vid[bk[k]];
+            int r = 0;
+            for (int t = 0; t < cnt; ++t) r += (a.bins.vid[bk[t]] < v) ? 1 : 0;
+            cellsort_md_emit(a, c, v, bk[k], s0 + r);
         }
     } else if (part == 0) {
-        // the bucket overflowed: scan every binning slot (order: by slot)
+        // scan every binning slot (order: by slot), eight loads in flight
+        constexpr int kScan = 8;
         int found = 0;
-        for (int base = 0; base < a.n; base += 64) {
-            const int i = base + lane;
-            const bool hit = i < a.n && a.bins.cell[i] == c;
-            const uint64_t m = __ballot(hit);
-            if (hit) cellsort_md_emit(a, c, a.bins.vid[i], i, s0 + found + (int)mbcnt64(m));
-            found += __popcll(m);
+        for (int base = lane; base - lane < a.n; base += 64 * kScan) {
+            uint32_t hits = 0u;
+#pragma unroll
+            for (int k = 0; k < kScan; ++k) {
+                const int i = base + 64 * k;
+                hits |= (i < a.n && a.bins.cell[i] == c ? 1u : 0u) << k;
+            }
+            if (__ballot(hits != 0u) == 0ull) continue;
+#pragma unroll 1
+            for (int k = 0; k < kScan; ++k) {
+                const int i = base + 64 * k;
+                const bool hit = ((hits >> k) & 1u) != 0u;
+                const uint64_t m = __ballot(hit);
+                if (hit) cellsort_md_emit(a, c, a.bins.vid[i], i, s0 + found + (int)mbcnt64(m));
+                found += __popcll(m);
+            }
         }
     }
 }
@@ -435,8 +468,8 @@ struct SortRho {
         }
         const int wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
         const int w = blk * kWaves + wv;
-        cellsort_md_cell(A.cs, w / A.parts, w % A.parts, A.parts, lane,
-                         (int32_t*)lds + wv * kSortWaveBuf);
+        cellsort_md_cell<false>(A.cs, w / A.parts, w % A.parts, A.parts, lane,
+                                (int32_t*)lds + wv * kSortWaveBuf);
     }
 };
 

@@ -78,7 +78,9 @@ __global__ void k_set_flag(uint32_t* flags) { flags[0] = 1u; }
 
 // A rebuild bins the current positions; otherwise they go to the sorted packed array,
 // unwrapped against the reference positions (x_ref + min_image(x - x_ref)), so that the
-// image of every list pair stays the one seen at the build.
+// image of every list pair stays the one seen at the build.  SPILL: SortFinal follows, which
+// empties the lists of the atoms beyond their buckets.
+template <bool SPILL>
 struct BinGather {
     static constexpr int kThreads = kBlock;
     struct Args {
@@ -98,7 +100,7 @@ struct BinGather {
         if (i >= a.n) return;
         const double x[3] = {a.x[i], a.y[i], a.z[i]};
         if (a.flags[0] != 0u) {
-            md_bin_atom(a.bins, (int)(a.flags[3] & 1u), i, i, x, a.box, a.dims, a.cell);
+            md_bin_atom<SPILL>(a.bins, (int)(a.flags[3] & 1u), i, i, x, a.box, a.dims, a.cell);
             return;
         }
         const double p = a.xr[i], b = a.yr[i], c = a.zr[i];
@@ -142,8 +144,8 @@ struct SortFinal {
             return;
         }
         const int wv = (int)(threadIdx.x >> 6), w = blk * kWaves + wv;
-        cellsort_md_cell(A.cs, w / A.parts, w % A.parts, A.parts, (int)(threadIdx.x & 63),
-                         lds + wv * kSortWaveBuf);
+        cellsort_md_cell<true>(A.cs, w / A.parts, w % A.parts, A.parts, (int)(threadIdx.x & 63),
+                               lds + wv * kSortWaveBuf);
     }
 };
 
@@ -289,9 +291,11 @@ Check::Args check_args(Engine& e, const double* x, const double* y, const double
     return Check::Args{x, y, z, e.xr, e.yr, e.zr, (int)e.n, e.box, h * h, e.flags, md_bins(e)};
 }
 
-BinGather::Args bin_args(Engine& e, const double* x, const double* y, const double* z)
+template <bool SPILL>
+typename BinGather<SPILL>::Args bin_args(Engine& e, const double* x, const double* y,
+                                         const double* z)
 {
-    return BinGather::Args{x, y, z, e.xr, e.yr, e.zr, e.q, e.atom_rank /* inverse perm */,
+    return typename BinGather<SPILL>::Args{x, y, z, e.xr, e.yr, e.zr, e.q, e.atom_rank /* inverse perm */,
                            (int)e.n, e.box, e.xs, make_int3(e.dims[0], e.dims[1], e.dims[2]),
                            make_double3(e.cell[0], e.cell[1], e.cell[2]), md_bins(e), e.flags};
 }
@@ -352,7 +356,7 @@ void launch_force_lists(Engine& e, const double* x, const double* y, const doubl
     }
     {
         ScopedTimer t(e, P_BIN, s);
-        k_one<BinGather><<<nblk(e.n), kBlock, 0, s>>>(bin_args(e, x, y, z));
+        k_one<BinGather<true>><<<nblk(e.n), kBlock, 0, s>>>(bin_args<true>(e, x, y, z));
         if (md_nchunk(e.ncell) > 0)
             k_one<ChunkSum><<<md_nchunk(e.ncell), ChunkSum::kThreads, 0, s>>>(
                 ChunkSum::Args{md_bins(e), e.flags});
@@ -400,7 +404,7 @@ void launch_copy(void* dst, const void* src, int64_t nbytes, hipStream_t s)
 hipError_t nlist_batch_prepare(Batch& b)
 {
     const size_t R = b.es.size();
-    std::vector<BinGather::Args> bi(R);
+    std::vector<BinGather<false>::Args> bi(R);
     std::vector<MdBin::Args> mb(R);
     std::vector<ClearInts::Args> mc(R);
     std::vector<StatsOut::Args> so(R);
@@ -410,7 +414,7 @@ hipError_t nlist_batch_prepare(Batch& b)
     for (size_t r = 0; r < R; ++r) {
         Engine& e = *b.es[r];
         const RepState& st = b.st[r];
-        bi[r] = bin_args(e, st.x, st.y, st.z);
+        bi[r] = bin_args<false>(e, st.x, st.y, st.z);
         mb[r] = mdbin_args(e, st.x, st.y, st.z, b.step0);
         const int ncount = (int)(md_count_bytes(e.ncell) / sizeof(int32_t));
         mc[r] = ClearInts::Args{e.md_count, ncount};
@@ -433,7 +437,7 @@ hipError_t nlist_batch_prepare(Batch& b)
 void nlist_batch_launch(Batch& b, int phase, hipStream_t s)
 {
     switch (phase) {
-    case BP_BIN: phase_launch<BinGather>(b.ph[phase], s); break;
+    case BP_BIN: phase_launch<BinGather<false>>(b.ph[phase], s); break;
     case BP_MDCLEAR: phase_launch<ClearInts>(b.ph[phase], s); break;
     case BP_MDBIN: phase_launch<MdBin>(b.ph[phase], s); break;
     case BP_STATS_OUT: phase_launch<StatsOut>(b.ph[phase], s); break;

@@ -132,6 +132,9 @@ __device__ inline void md_bin_wave(const MdBins& b, int buf, bool active, int s,
     }
 }
 
+// SPILL: an atom beyond its cell's bucket goes to one of the cell's lists (slot and atom are
+// the same there).
+template <bool SPILL = false>
 __device__ inline void md_bin_atom(const MdBins& b, int buf, int s, int v, const double p[3],
                                    const Box& box, int3 dims, double3 cell)
 {
@@ -145,6 +148,8 @@ __device__ inline void md_bin_atom(const MdBins& b, int buf, int s, int v, const
     const int bc = buf * b.ncell + c;
     const int rank = atomicAdd(&b.count[bc], 1);
     if (rank < b.cap) b.bucket[(size_t)bc * b.cap + rank] = s;
+    else if (SPILL)
+        b.spill_next[v] = atomicExch(&b.spill[(size_t)c * kSpillChains + rank % kSpillChains], v);
 }
 
 // ---------------------------------------------------------------- tile order

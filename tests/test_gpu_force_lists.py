@@ -82,3 +82,80 @@ def test_bins_and_sort(orc, gpu, kind):
         fresh.Init(_dev(q))
         G = evaluate(fresh, p)
         assert np.abs(F - G).max() <= 1e-10 * max(np.abs(G).max(), 1e-300)
+
+
+# cells of exactly their bucket, of up to three atoms in a list beyond it, of as many as the
+# sort ranks at once and of one more; the others hold three
+CROWDED = (64, 65, 96, 97, 129, 1024, 1025)
+
+
+def test_cells_beyond_their_bucket(orc, gpu):
+    """Rows equal the oracle's sets and forces a second handle's bit for bit, at each of
+    several builds (the lists of the atoms beyond a bucket start empty every time)."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    rng = np.random.default_rng(12)
+    edge, cells = 2.2, 9
+    L = 1.0001 * edge * cells
+    crowd = {(1, 1, 1 + k): c for k, c in enumerate(CROWDED)}
+    pos = []
+    for c in np.ndindex(cells, cells, cells):
+        m = crowd.get(c, 3 if min(c) > 0 and max(c) < 8 and c[0] > 3 else 0)
+        g = rng.permutation(12 ** 3)[:m]
+        p = (np.stack([g % 12, g // 12 % 12, g // 144]) + 0.5) * (0.8 * edge / 12) + 0.1 * edge
+        pos.append(p + np.array(c)[:, None] * L / cells)
+    pos = np.concatenate(pos, 1)
+    pos = pos[:, rng.permutation(pos.shape[1])]
+    n = pos.shape[1]
+    q = rng.uniform(-1, 1, n)
+    cfg = ForceConfig(box_len=(L,) * 3, cut_off=2.0, coulomb_cut=2.0, skin=0.2, alpha=0.5,
+                      kspace="NONE", precision=64, n_max=n, list_capacity=2560)
+    assert 4 * n / cells ** 3 + 32 <= 64  # the smallest bucket
+    f = LJCutCoulKspaceForce(cfg)
+    f.Init(_dev(q))
+    for build, move in enumerate((0.0, 0.15, 0.0), 1):
+        p = pos + move
+        F, G = ([torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+                for _ in range(2))
+        f.Execute(*[_dev(a) for a in p], *F)
+        st = f.stats()
+        assert st["builds"] == build and st["overflow_rows"] == 0
+        w = [np.ascontiguousarray(a) for a in orc.wrap(*p, np.zeros(3), np.array([L] * 3))]
+        oo, io = orc.neighbors_images(*w, np.array([L] * 3), 2.2)
+        og, ig = f.neighbors()
+        assert og[-1] == oo[-1]
+        for i in range(n):
+            assert np.array_equal(np.sort(ig[og[i]:og[i + 1]]), np.sort(io[oo[i]:oo[i + 1]])), i
+        h = LJCutCoulKspaceForce(cfg)
+        h.Init(_dev(q))
+        h.Execute(*[_dev(a) for a in p], *G)
+        for a, b in zip(F, G):
+            assert torch.equal(a, b)
+
+
+def test_sort_time_of_a_droplet(gpu):
+    """100,000 ions in a 27th of their box, most cells beyond their bucket: the cell sort of a
+    rebuild takes no more than four times that of the same ions in a box of their own."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    n, m = 100000, 47
+    g = np.random.default_rng(13).permutation(m ** 3)[:n]
+    pos = (np.stack([g % m, g // m % m, g // m ** 2]) + 0.5) * 1.5
+    us = []
+    for L in (1.5 * m, 3 * 1.5 * m):
+        f = LJCutCoulKspaceForce(ForceConfig(box_len=(L,) * 3, cut_off=2.5, coulomb_cut=6.0,
+                                             alpha=0.5, kspace="NONE", n_max=n))
+        f.Init(_dev(np.where(g % 2, 1.0, -1.0)))
+        X = [[_dev(a + d) for a in pos] for d in (0.0, 0.2)]
+        F = [torch.zeros(n, device="cuda") for _ in range(3)]
+        for k in range(4):
+            f.Execute(*X[k % 2], *F)
+        torch.cuda.synchronize()
+        b0 = f.stats()["builds"]
+        f.set_timing(True)
+        for k in range(10):
+            f.Execute(*X[k % 2], *F)
+        us.append(1e3 * f.timing("cellsort")[0])
+        assert f.stats()["builds"] == b0 + 10
+    print(f"cell sort: {us[0]:.1f} us, droplet {us[1]:.1f} us", flush=True)
+    assert us[1] < 4 * us[0]
