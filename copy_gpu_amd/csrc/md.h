@@ -329,15 +329,41 @@ __device__ inline void cellsort_md_emit(const CellSortMDArgs& a, int c, int v, i
     a.ts[s] = a.type ? a.type[v] : 0;
 }
 
-// One wave sorts entries part * 64 + lane, + 64 parts, ... of cell c (c >= ncell:
-// nothing); buf holds kSortWaveBuf ids of this wave's own LDS.  The bucket lists binning
-// slots; atoms are ranked by id.  SPILL: the force pass, whose slots are the atoms.
-template <bool SPILL>
-__device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int part, int parts,
-                                        int lane, int32_t* buf)
+// Sum of the counts of the cells before c, by the whole workgroup: whole chunks, then the
+// cells of c's own chunk (without chunk counts, every earlier cell), eight loads in flight.
+template <int NT>
+__device__ inline int cellsort_before(const int32_t* count, const int32_t* chunk, int nchunk, int c)
+{
+    __shared__ int32_t red[NT / 64];
+    const int t = (int)threadIdx.x, c0 = nchunk > 0 ? (c / kBinChunk) * kBinChunk : 0;
+    int v = 0;
+    if (nchunk > 0) {
+#pragma unroll 8
+        for (int k = t; k < c / kBinChunk; k += NT) v += chunk[k];
+    }
+#pragma unroll 8
+    for (int k = c0 + t; k < c; k += NT) v += count[k];
+    v = wave_sum(v);
+    if ((t & 63) == 0) red[t >> 6] = v;
+    __syncthreads();
+    int s = 0;
+    for (int w = 0; w < NT / 64; ++w) s += red[w];
+    return s;
+}
+
+// Workgroup blk of NT threads sorts the cells of its waves, wave w = blk NT / 64, ..
+// entries (w % parts) 64 + lane, + 64 parts, ... of cell w / parts; lds holds kSortWaveBuf ids
+// per wave.  The bucket lists binning slots; atoms are ranked by id.  SPILL: the force pass,
+// whose slots are the atoms.
+//
+// The starts: the workgroup sums the counts before its first cell together.  (With every wave
+// summing for itself a rebuild's sort read ncell^2 / 2 counts: 66 us at 15,625
+// cells, 16 now, and 46 -> 23 us at 9,826 with 100,000 ions.)
+template <int NT, bool SPILL>
+__device__ inline void cellsort_md(const CellSortMDArgs& a, int blk, int parts, int32_t* lds)
 {
     const uint32_t req = a.flags[0];
-    if (c == 0 && part == 0 && lane == 0) {
+    if (blk == 0 && threadIdx.x == 0) {
         a.flags[2] = req;
         if (req) {
             a.stats[0] += 1ull;
@@ -348,20 +374,19 @@ __device__ inline void cellsort_md_cell(const CellSortMDArgs& a, int c, int part
             a.stats[6] = 0ull;
         }
     }
-    if (req == 0u || c >= a.ncell) return;
+    if (req == 0u) return;
     const int b = (int)(a.flags[3] & 1u);
     const int32_t* count = a.bins.count + (size_t)b * a.ncell;
     const int32_t* chunk = a.bins.chunk + (size_t)b * a.bins.nchunk;
-    // start = the counts of the whole chunks before c, then of the cells of c's own
-    // chunk before c: at most ncell / kBinChunk + kBinChunk loads per cell (without
-    // chunk counts, every earlier cell)
-    const int c0 = a.bins.nchunk > 0 ? (c / kBinChunk) * kBinChunk : 0;
-    int before = 0;
-    if (a.bins.nchunk > 0)
-        for (int k = lane; k < c / kBinChunk; k += 64) before += chunk[k];
-    for (int k = c0 + lane; k < c; k += 64) before += count[k];
-    const int s0 = wave_sum(before);
+    constexpr int kWaves = NT / 64;
+    const int lane = (int)(threadIdx.x & 63), wv = uniform((int)(threadIdx.x >> 6));
+    const int cf = blk * kWaves / parts, c = (blk * kWaves + wv) / parts,
+              part = (blk * kWaves + wv) % parts;
+    int s0 = cellsort_before<NT>(count, chunk, a.bins.nchunk, cf);
+    if (c >= a.ncell) return;
+    for (int k = cf; k < c; ++k) s0 += count[k];
     const int cnt = count[c];
+    int32_t* buf = lds + wv * kSortWaveBuf;
     if (lane == 0 && part == 0) {
         a.cell_start[c] = s0;
         if (c == a.ncell - 1) a.cell_start[a.ncell] = s0 + cnt;
@@ -466,10 +491,7 @@ struct SortRho {
             }
             return;
         }
-        const int wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
-        const int w = blk * kWaves + wv;
-        cellsort_md_cell<false>(A.cs, w / A.parts, w % A.parts, A.parts, lane,
-                                (int32_t*)lds + wv * kSortWaveBuf);
+        cellsort_md<kThreads, false>(A.cs, blk, A.parts, (int32_t*)lds);
     }
 };
 

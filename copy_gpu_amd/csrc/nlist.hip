@@ -143,9 +143,7 @@ struct SortFinal {
                                  A.cs.ncell, A.dims, A.split, A.ncu, A.tile_order, lds);
             return;
         }
-        const int wv = (int)(threadIdx.x >> 6), w = blk * kWaves + wv;
-        cellsort_md_cell<true>(A.cs, w / A.parts, w % A.parts, A.parts, (int)(threadIdx.x & 63),
-                               lds + wv * kSortWaveBuf);
+        cellsort_md<kThreads, true>(A.cs, blk, A.parts, lds);
     }
 };
 

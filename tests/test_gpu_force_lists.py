@@ -159,3 +159,59 @@ def test_sort_time_of_a_droplet(gpu):
         assert f.stats()["builds"] == b0 + 10
     print(f"cell sort: {us[0]:.1f} us, droplet {us[1]:.1f} us", flush=True)
     assert us[1] < 4 * us[0]
+
+
+# every earlier cell counted (no chunk counts) at a number of cells that four does not divide,
+# and three waves per cell: workgroups that begin within a cell
+@pytest.mark.parametrize("cells,n", [((25, 25, 25), 5000), ((1, 1, 5), 850)])
+def test_starts_of_cells(orc, gpu, cells, n):
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    rng = np.random.default_rng(14)
+    rc, skin = 2.0, 0.2
+    L = np.array(cells) * 1.0001 * (rc + skin)
+    m = np.ceil(L / (0.9 * (L.prod() / n) ** (1 / 3))).astype(int)
+    g = rng.permutation(m.prod())[:n]
+    pos = np.stack([g % m[0], g // m[0] % m[1], g // (m[0] * m[1])]) + rng.uniform(0.3, 0.7, (3, n))
+    pos *= (L / m)[:, None]
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=tuple(L), cut_off=rc, coulomb_cut=rc, skin=skin,
+                                         alpha=0.5, kspace="NONE", n_max=n, list_capacity=1024))
+    f.Init(_dev(rng.uniform(-1, 1, n)))
+    F = [torch.zeros(n, device="cuda") for _ in range(3)]
+    f.Execute(*[_dev(a) for a in pos], *F)
+    st = f.stats()
+    assert st["cells"] == np.prod(cells) and st["overflow_rows"] == 0
+    w = [np.ascontiguousarray(a) for a in orc.wrap(*pos, np.zeros(3), L)]
+    oo, io = orc.neighbors_images(*w, L, rc + skin)
+    og, ig = f.neighbors()
+    assert og[-1] == oo[-1]
+    for i in range(n):
+        assert np.array_equal(np.sort(ig[og[i]:og[i + 1]]), np.sort(io[oo[i]:oo[i + 1]])), i
+
+
+def test_sort_time_of_many_cells(gpu):
+    """A thin gas of 4,000 ions: the cell sort of 15,625 cells takes no more than four times
+    that of 512."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    n, m = 4000, 16
+    g = np.random.default_rng(15).permutation(m ** 3)[:n]
+    us = []
+    for cells in (8, 25):
+        L = 5.35 * cells
+        pos = (np.stack([g % m, g // m % m, g // m ** 2]) + 0.5) * (L / m)
+        f = LJCutCoulKspaceForce(ForceConfig(box_len=(L,) * 3, cut_off=2.5, coulomb_cut=5.0,
+                                             alpha=0.5, kspace="NONE", n_max=n))
+        f.Init(_dev(np.where(g % 2, 1.0, -1.0)))
+        X = [[_dev(a + d) for a in pos] for d in (0.0, 0.2)]
+        F = [torch.zeros(n, device="cuda") for _ in range(3)]
+        for k in range(4):
+            f.Execute(*X[k % 2], *F)
+        torch.cuda.synchronize()
+        assert f.stats()["cells"] == cells ** 3
+        f.set_timing(True)
+        for k in range(20):
+            f.Execute(*X[k % 2], *F)
+        us.append(1e3 * f.timing("cellsort")[0])
+    print(f"cell sort: 512 cells {us[0]:.1f} us, 15,625 cells {us[1]:.1f} us", flush=True)
+    assert us[1] < 4 * us[0]
