@@ -716,6 +716,7 @@ __device__ inline void list_tile(const TileHdr& h, const ListArgs& a, double4* l
                                  int wv, int lane, const RblBuild& rb)
 {
     const int total = h.off[27];
+    if (a0 >= a1) return;  // no home atoms
     if (total >= kMaxTile) {
         for (int s = a0 + (int)threadIdx.x; s < a1; s += kTileThreads) {
             a.ncount[s] = make_int2(a.cap + 1, 0);

@@ -215,3 +215,32 @@ def test_sort_time_of_many_cells(gpu):
         us.append(1e3 * f.timing("cellsort")[0])
     print(f"cell sort: 512 cells {us[0]:.1f} us, 15,625 cells {us[1]:.1f} us", flush=True)
     assert us[1] < 4 * us[0]
+
+
+def test_empty_tiles_of_a_rebuild(gpu):
+    """4,000 ions in 64,000 cells: a rebuild costs the tiles without home atoms nothing, so its
+    tile pass takes at most 1.25 times that of an evaluation that keeps its list."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    n, m, L = 4000, 16, 5.35 * 40
+    g = np.random.default_rng(16).permutation(m ** 3)[:n]
+    pos = (np.stack([g % m, g // m % m, g // m ** 2]) + 0.5) * (L / m)
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=(L,) * 3, cut_off=2.5, coulomb_cut=5.0,
+                                         alpha=0.5, kspace="NONE", n_max=n))
+    f.Init(_dev(np.where(g % 2, 1.0, -1.0)))
+    X = [[_dev(a + d) for a in pos] for d in (0.0, 0.2)]
+    F = [torch.zeros(n, device="cuda") for _ in range(3)]
+    us = []
+    for move in (0, 1):
+        for k in range(4):
+            f.Execute(*X[move * (k % 2)], *F)
+        torch.cuda.synchronize()
+        b0 = f.stats()["builds"]
+        f.set_timing(True)
+        for k in range(20):
+            f.Execute(*X[move * (k % 2)], *F)
+        us.append(1e3 * f.timing("pair")[0])
+        f.set_timing(False)
+        assert f.stats()["builds"] == b0 + 20 * move
+    print(f"tile pass: {us[0]:.1f} us, with a rebuild {us[1]:.1f} us", flush=True)
+    assert us[1] < 1.25 * us[0]
