@@ -232,6 +232,7 @@ void ks_launch(const KsCall& c, char* buf, hipStream_t s)
     ka.fz = (T*)c.fz;
     ka.slices = kf_slices(c.n, c.P);
     const int nforce = c.n > 0 ? kf_blocks(c.n, ka.slices) : 0, nev = c.ev_out ? 7 : 0;
+    ka.staged = kf_staged<T>(nforce, c.P);
     const double wdef = c.w ? 0.0 : rbe_S(c.alpha, c.L) / (double)c.P;
     if (ks_small(c)) {
         k_ks_rho<T><<<c.P, 256, 0, s>>>(c.x, c.y, c.z, c.q, (int)c.n, box, c.m, c.rho_out);

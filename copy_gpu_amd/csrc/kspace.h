@@ -313,7 +313,9 @@ struct RhoFinal {
 // scalar loads, four k's in flight, and are scalar operands of the arithmetic.  (From an LDS
 // stage they took three 16-byte reads per k and wave and 12 vector registers: 1,048,576 atoms
 // and 500 k-vectors 347 -> 257 us, 14 vector instructions per k and 64 atoms; 32,768 atoms and
-// P = 100 6.9 -> 5.8 us.)
+// P = 100 6.9 -> 5.8 us.)  That needs other waves to run while a wave waits for its four: FP32
+// launches that leave a CU one workgroup (or none) read the coefficients from the LDS stage
+// when there are many (kf_staged).
 // s = 8 (64 atoms per workgroup) unless P <= kKfWideP and that would give more
 // than kKfTargetBlocks workgroups: then the fewest slices that still give that many
 // (at 100,000 atoms and P = 50, s = 4), so fewer waves repeat the per-atom work.
@@ -340,6 +342,18 @@ inline int kf_blocks(int64_t n, int slices)
     return (int)((n + apb - 1) / apb);
 }
 
+// Whether a launch of `blocks` workgroups stages its coefficients in LDS.  Scalar loads
+// against the stage at 4,000 atoms in FP32 (event times): 6.8 and 6.6 us for 100 k-vectors, 8.6
+// and 7.7 for 200, 22 and 17 for 1,000, 149 and 95 for 8,000; at 16,000 atoms 147 and 98, at
+// 32,768 (two workgroups a CU) 146 and 167.  In FP64 a k-vector takes long enough to hide the
+// loads: 264 and 304 us at 2,000 atoms and 8,000 k-vectors, and no size where the stage wins.
+constexpr int kKfStagedBlocks = 256;  // one per CU of an MI355X
+template <typename T>
+inline bool kf_staged(int64_t blocks, int P)
+{
+    return sizeof(T) == 4 && blocks <= kKfStagedBlocks && P > kKfWideP;
+}
+
 template <typename T>
 struct KForceArgs {
     const double *x, *y, *z, *q;
@@ -355,17 +369,21 @@ struct KForceArgs {
     ThermoArgs th;  // velocity thermostat of the closing kick (KForce<T, true>)
     const double* rbl_mean = nullptr;  // random batch list: mean near force to subtract
     int slices = kKfSlices;            // k-slices per atom group (kf_slices)
+    int staged = 0;                    // kf_staged
 };
 
-// LDS: the sums of the slices, and a stage of coefficients for those that are not in memory.
+// LDS: the sums of the slices, and a stage of coefficients.
 template <typename T>
-struct KForceLds {
+struct KForceSumLds {
     T red[kKfSlices][3][kKfAtoms];
 };
 template <typename T>
-struct KForceStagedLds : KForceLds<T> {
+struct KForceStagedLds : KForceSumLds<T> {
     KCoef<T> st[kKfStage];
 };
+// that of coefficients in memory: FP64 launches stage none
+template <typename T>
+using KForceLds = typename std::conditional<sizeof(T) == 4, KForceStagedLds<T>, KForceSumLds<T>>::type;
 
 // The k-space force of the atoms of workgroup blk.  Each lane of an atom-owning
 // wave (slice 0 of its atom group) first calls pre(i) for its atom i < n (loads
@@ -419,7 +437,24 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coe
         ay = fma_t(g, c.k[1], ay);
         az = fma_t(g, c.k[2], az);
     };
-    if constexpr (std::is_same<Coef, const KCoef<T>*>::value) {
+    constexpr bool kMem = std::is_same<Coef, const KCoef<T>*>::value;
+    auto stage = [&](auto of) {
+        if constexpr (std::is_base_of<KForceStagedLds<T>, Lds>::value) {
+            for (int base = 0; base < P; base += kKfStage) {
+                __syncthreads();
+                for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
+                    L.st[k] = of(base + k);
+                __syncthreads();
+                const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
+                for (int k = slice; k < cnt; k += slices) add(L.st[k]);
+            }
+        }
+    };
+    if constexpr (!kMem) {
+        stage(coef);
+    } else if (sizeof(T) == 4 && A.staged) {
+        stage([&](int k) { return coef[k]; });
+    } else {
         int k = uniform(slice);
         // four k's loads in flight together
         for (; k + 3 * slices < P; k += 4 * slices) {
@@ -433,15 +468,6 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coe
             add(c3);
         }
         for (; k < P; k += slices) add(const_mem(coef + k));
-    } else {
-        for (int base = 0; base < P; base += kKfStage) {
-            __syncthreads();
-            for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
-                L.st[k] = coef(base + k);
-            __syncthreads();
-            const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
-            for (int k = slice; k < cnt; k += slices) add(L.st[k]);
-        }
     }
     if (P > 0 && slices > 1) {
         L.red[wv][0][lane] = ax;
@@ -666,6 +692,7 @@ inline KForceArgs<T> kforce_args(Engine& e, const double* x, const double* y, co
                     e.flags};
     a.rbl_mean = e.rbl ? e.rbl_mean : nullptr;
     a.slices = kf_slices(e.n, a.P);
+    a.staged = kf_staged<T>(kf_blocks(e.n, a.slices), a.P);
     return a;
 }
 

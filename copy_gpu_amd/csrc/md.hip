@@ -164,6 +164,11 @@ hipError_t md_prepare_t(Batch& b)
         nkc[r] = std::max(kforce_blocks(e), 1);
         nko[r] = close_open_blocks(e, b.sa[r]);
     }
+    // one launch holds the workgroups of every replica
+    int64_t blocks = 0;
+    for (int k : nkc) blocks += k;
+    for (size_t r = 0; r < R; ++r)
+        kc[r].staged = ko[r].kf.staged = kf_staged<T>(blocks, kc[r].P);
     hipError_t err;
     if ((err = phase_upload(b.ph[BP_KICKDRIFT], kd, nkd, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_SORT_RHO], sr, nsr, 0)) != hipSuccess) return err;
