@@ -569,21 +569,12 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
     const int cap = a.cap, total = h.off[27];
     const int g = lane >> 4, col = lane & 15;
     uint16_t* __restrict__ rowp = a.nlist + (size_t)s * cap;
-    const int32_t id_i = RBL ? rb.perm[s] : 0;
     int ci = have.x, co = have.y;
     auto put1 = [&](int k, int u) {
         if (SINGLE) L.buf[k] = (uint16_t)u;
         else rowp[k] = (uint16_t)u;
     };
-    // one entry per lane with `keep`: LJ range (and, for a random batch list, every
-    // kept pair) at the front, else at the back
-    auto put = [&](bool keep, bool front, int u, int base) {
-        const uint64_t m = __builtin_amdgcn_ballot_w64(keep);
-        const int k = base + (int)mbcnt64(m);
-        if (keep && k < cap) put1(front ? k : cap - 1 - k, u);
-        return __popcll(m);
-    };
-    bool ordered = RBL;  // the others already stand behind the LJ range
+    bool ordered = false;  // the others already stand behind the LJ range
     {
         constexpr int kBits = 8 * sizeof(W);
         const int wo = (row * 4 + g) * 16 + col;
@@ -600,47 +591,65 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
         mi &= m;
         const int ub = cb + 32 * g * T + col;
         const W top = (W)1 << (kBits - 1);
+        // the row's counts first: a row that fits is written without tests, one that
+        // does not is only counted
+        int pc = sizeof(W) == 4 ? __popc((uint32_t)mi) | (__popc((uint32_t)mo) << 16)
+                                : __popcll(mi) | (__popcll(mo) << 16);
+        pc = wave_sum_int(pc);
+        const int ni = pc & 0xffff, no = pc >> 16;
+        // each trip gives put the next hit of every lane that has one
+        auto expand = [&](W w, int k0, auto put) {
+            while (w != 0) {
+                const uint64_t act = __builtin_amdgcn_ballot_w64(true);
+                const int k = (int)__builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(act >> 32),
+                    __builtin_amdgcn_mbcnt_lo((uint32_t)act, (uint32_t)k0));
+                const int z = lead0(w);
+                put(k, ub + 16 * z);
+                w ^= top >> z;
+                k0 += __popcll(act);
+            }
+        };
         if (RBL) {
-            // every hit draws its selection: a near-band entry kept for being near counts
-            // only if selected should it lie in the shell when evaluated
-            while (__builtin_amdgcn_ballot_w64(m != 0) != 0ull) {
-                const bool act = m != 0;
-                const int z = act ? lead0(m) : 0;
-                const W bit = top >> z;
-                const int u = ub + 16 * z;
-                bool sel = false;
-                if (act) sel = rbl_select(rb.seed, rb.epoch, id_i, ids[u - cb], rb.pice);
-                ci += put(act && ((mi & bit) != 0 || sel), true, sel ? (u | kRblSel) : u, ci);
-                m &= ~bit;
+            // the block's hits to the buffer, the near band first; then each draws its selection,
+            // 64 at a time (a lane drawing for its own column's hits leaves most lanes idle: an
+            // evaluation of 200,000 ions with a rebuild took 568 us so, 453 now).  A near-band
+            // entry kept for being near counts only if selected should it lie in the shell
+            // when evaluated.  co: hits of the blocks so far; rows whose hits do not fit overflow.
+            if (co + ni + no < cap) {
+                auto put = [&](int k, int u) { L.buf[k] = (uint16_t)u; };
+                expand(mi, 0, put);
+                expand(mo, ni, put);
+                __syncwarp();
+                const int32_t id_i = rb.perm[s];
+                for (int k0 = 0; k0 < ni + no; k0 += 64) {
+                    const int k = k0 + lane;
+                    const bool hit = k < ni + no;
+                    const int u = hit ? (int)L.buf[k] : 0;
+                    bool sel = false;
+                    if (hit) sel = rbl_select(rb.seed, rb.epoch, id_i, ids[u - cb], rb.pice);
+                    const bool keep = hit && (k < ni || sel);
+                    const uint64_t mk = __builtin_amdgcn_ballot_w64(keep);
+                    if (keep) rowp[ci + (int)mbcnt64(mk)] = (uint16_t)(sel ? (u | kRblSel) : u);
+                    ci += __popcll(mk);
+                }
+                __syncwarp();  // the buffer is reused for the wave's next row
             }
-        } else {
-            // the row's counts first: a row that fits is written without tests, one that
-            // does not is only counted
-            int pc = sizeof(W) == 4 ? __popc((uint32_t)mi) | (__popc((uint32_t)mo) << 16)
-                                    : __popcll(mi) | (__popcll(mo) << 16);
-            pc = wave_sum_int(pc);
-            const int ni = pc & 0xffff, no = pc >> 16;
-            if (ci + co + ni + no < cap) {
-                // each trip writes the next hit of every lane that has one
-                auto expand = [&](W w, int k0, bool back) {
-                    while (w != 0) {
-                        const uint64_t act = __builtin_amdgcn_ballot_w64(true);
-                        const int k = (int)__builtin_amdgcn_mbcnt_hi(
-                            (uint32_t)(act >> 32),
-                            __builtin_amdgcn_mbcnt_lo((uint32_t)act, (uint32_t)k0));
-                        const int z = lead0(w);
-                        put1(back ? cap - 1 - k : k, ub + 16 * z);
-                        w ^= top >> z;
-                        k0 += __popcll(act);
-                    }
-                };
-                expand(mi, ci, false);
-                expand(mo, SINGLE ? ni : co, !SINGLE);
-                ordered = SINGLE;
+            co += ni + no;
+            if (last && lane == 0) {
+                if (co < cap) rowp[ci] = (uint16_t)total;
+                a.ncount[s] = co < cap ? make_int2(ci, 0) : make_int2(co, 0);
+                if (co >= cap) list_overflow(a, co + 1);
             }
-            ci += ni;
-            co += no;
+            return make_int2(ci, co);
         }
+        if (ci + co + ni + no < cap) {
+            expand(mi, ci, put1);
+            expand(mo, SINGLE ? ni : co, [&](int k, int u) { put1(SINGLE ? k : cap - 1 - k, u); });
+            ordered = SINGLE;
+        }
+        ci += ni;
+        co += no;
     }
     if (!last) return make_int2(ci, co);
     const int n = ci + co;

@@ -66,3 +66,36 @@ def test_rows_equal_oracle_sets(orc, gpu, rc, cells, rho, stage):
     inner = (dd * dd).sum(1) < (min(rc, 2.5) + 0.3) ** 2
     if cells > 2:
         assert st["inner_entries"] == int(inner.sum())
+
+
+# random batch rows: one block, blocks staged in turn (208 candidates), two and more blocks of
+# 4,096; rows whose hits fit, and rows of which only the kept entries would
+@pytest.mark.parametrize("rc,stage,cap,overflow", [
+    (5.0, 0, 0, False), (5.0, 208, 0, False), (7.9, 0, 0, False), (8.4, 0, 0, False),
+    (5.0, 0, 128, True), (5.0, 208, 128, True)])
+def test_random_batch_rows_over_blocks(orc, gpu, rc, stage, cap, overflow):
+    """FP64 forces equal the oracle's for the same draws."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce, systems
+
+    L = 1.013 * 3 * (rc + 0.3)
+    n, pice, seed = int(0.3 * L ** 3), 3, 78
+    print(f"case: random batch rows, rc {rc}, {n} ions, stage {stage}, capacity {cap}", flush=True)
+    x, y, z, q, Lb_ = systems.random_ions(n, n / L ** 3, 0.8, seed=SEED + 1)
+    Lb = np.array([Lb_] * 3)
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=(Lb_,) * 3, cut_off=2.5, coulomb_cut=rc,
+                                         alpha=0.5, kspace="NONE", precision=64, n_max=n,
+                                         tile_stage=stage, list_capacity=cap,
+                                         neighbor_type="RBL", r_core=2.5, rbl_pice=pice,
+                                         rbl_seed=seed))
+    f.Init(_dev(q))
+    F = [torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+    f.Execute(_dev(x), _dev(y), _dev(z), *F)
+    torch.cuda.synchronize()
+    st = f.stats()
+    assert st["builds"] == 1 and (st["overflow_rows"] > 0) == overflow
+    assert (st["big_tiles"] > 0) == (st["largest_tile"] >= st["tile_stage"])
+    xw, yw, zw = orc.wrap(x, y, z, np.zeros(3), Lb)
+    Fo, _ = orc.rbl_forces(xw, yw, zw, q, np.zeros(3), Lb, 2.5, rc, 0.5, 2.5, pice, seed, 1)
+    G = np.stack([t.cpu().numpy() for t in F], 1)
+    assert np.linalg.norm(G - Fo) < 1e-12 * np.linalg.norm(Fo)
+
