@@ -99,3 +99,43 @@ def test_random_batch_rows_over_blocks(orc, gpu, rc, stage, cap, overflow):
     G = np.stack([t.cpu().numpy() for t in F], 1)
     assert np.linalg.norm(G - Fo) < 1e-12 * np.linalg.norm(Fo)
 
+
+# tiles of at most 64 candidates take one wave per row: n atoms in 27 cells make n candidates of
+# every tile, in one cell 27 n, in 2 x 2 x 3 cells 12 cells' atoms up to three times each
+@pytest.mark.parametrize("cells,n", [((3, 3, 3), 2), ((3, 3, 3), 63), ((3, 3, 3), 64),
+                                     ((3, 3, 3), 65), ((1, 1, 1), 2), ((1, 1, 1), 3),
+                                     ((2, 2, 3), 28)])
+@pytest.mark.parametrize("neighbors", ["VERLET-LIST", "RBL"])
+def test_rows_of_few_candidates(orc, gpu, cells, n, neighbors):
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    rng = np.random.default_rng(n)
+    rc, skin = 2.0, 0.3
+    # a grid of 12 points per cell edge of 1.1 list radii, so that pairs at every distance occur
+    Lb = np.array(cells) * 1.1 * (rc + skin)
+    m = 12 * np.array(cells)
+    g = rng.permutation(m.prod())[:n]
+    p = (np.stack([g % m[0], g // m[0] % m[1], g // (m[0] * m[1])]) + 0.5) * (Lb / m)[:, None]
+    if n > 4:  # pairs astride the smallest accepted distance
+        p[:, 1] = p[:, 0] + [0.0099, 0, 0]
+        p[:, 3] = p[:, 2] + [0, 0.0101, 0]
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=tuple(Lb), cut_off=1.0, coulomb_cut=rc, skin=skin,
+                                         alpha=0.5, kspace="NONE", precision=64, n_max=n,
+                                         neighbor_type=neighbors, r_core=1.0, rbl_pice=1))
+    f.Init(_dev(rng.uniform(-1, 1, n)))
+    F = [torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+    f.Execute(*[_dev(a) for a in p], *F)
+    st = f.stats()
+    assert st["cells"] == np.prod(cells) and st["overflow_rows"] == 0
+    assert cells != (3, 3, 3) or st["largest_tile"] == n
+    w = [np.ascontiguousarray(a) for a in orc.wrap(*p, np.zeros(3), Lb)]
+    oo, io = orc.neighbors_images(*w, Lb, rc + skin)
+    og, ig = f.neighbors()
+    assert og[-1] == oo[-1]
+    for i in range(n):
+        assert np.array_equal(np.sort(ig[og[i]:og[i + 1]]), np.sort(io[oo[i]:oo[i + 1]])), i
+    if neighbors == "VERLET-LIST" and min(cells) > 2:
+        d = np.stack(w, 1)
+        dd = d[ig] - d[np.repeat(np.arange(n), np.diff(og))]
+        dd -= Lb * np.round(dd / Lb)
+        assert st["inner_entries"] == int(((dd * dd).sum(1) < (1.0 + skin) ** 2).sum())
