@@ -411,11 +411,14 @@ __device__ inline void list_overflow(const ListArgs& a, int n)
 
 typedef float list_f4 __attribute__((ext_vector_type(4)));
 
-// FP32 position relative to the home cell's centre, its square in w.
+// FP32 position relative to the home cell's centre, its square in w.  One that is not a number
+// stands far from everything, as the exact criterion has it: the masks take the sign bits of
+// the distances, and a NaN has one too.
 __device__ inline float4 list_pos(const ListArgs& A, double x, double y, double z)
 {
     const float a = (float)(x - A.ctr[0]), b = (float)(y - A.ctr[1]), c = (float)(z - A.ctr[2]);
-    return make_float4(a, b, c, fmaf(c, c, fmaf(b, b, a * a)));
+    const float w = fmaf(c, c, fmaf(b, b, a * a));
+    return w < 1.0e30f ? make_float4(a, b, c, w) : make_float4(0.0f, 0.0f, 0.0f, 1.0e30f);
 }
 
 // The home rows of one near_masks call: NMT 16-row tiles, rows [0, nrow) being home

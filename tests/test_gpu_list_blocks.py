@@ -139,3 +139,38 @@ def test_rows_of_few_candidates(orc, gpu, cells, n, neighbors):
         dd = d[ig] - d[np.repeat(np.arange(n), np.diff(og))]
         dd -= Lb * np.round(dd / Lb)
         assert st["inner_entries"] == int(((dd * dd).sum(1) < (1.0 + skin) ** 2).sum())
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("stage", [0, 208])
+def test_position_that_is_not_a_number(gpu, sign, stage):
+    """An atom at NaN (of either sign bit) is nobody's neighbour: it has no row, and the others
+    have the forces of the system without it."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce, systems
+
+    n = 1500
+    x, y, z, q, L = systems.random_ions(n, 0.3, 0.8, seed=SEED + 2)
+    forces = []
+    for bad in (True, False):
+        p = np.stack([x, y, z])
+        keep = np.arange(n) != 700
+        if bad:
+            p[0, 700] = np.copysign(np.nan, sign)
+        else:
+            p = p[:, keep]
+        m = p.shape[1]
+        f = LJCutCoulKspaceForce(ForceConfig(box_len=(L,) * 3, cut_off=2.5, coulomb_cut=5.0,
+                                             alpha=0.5, kspace="NONE", precision=64, n_max=m,
+                                             tile_stage=stage))
+        f.Init(_dev(q if bad else q[keep]))
+        F = [torch.zeros(m, device="cuda", dtype=torch.float64) for _ in range(3)]
+        f.Execute(*[_dev(a) for a in p], *F)
+        st = f.stats()
+        assert st["overflow_rows"] == 0
+        G = np.stack([t.cpu().numpy() for t in F])
+        forces.append(G[:, keep] if bad else G)
+        if bad:
+            og, _ = f.neighbors()
+            assert og[701] == og[700]
+    # the same terms in another order: a few hundred, none above the largest force by much
+    assert np.abs(forces[0] - forces[1]).max() <= 1e-12 * np.abs(forces[1]).max()
