@@ -557,12 +557,11 @@ __device__ inline int wave_sum_int(int v)
 __device__ inline int lead0(uint32_t v) { return __clz((int)v); }
 __device__ inline int lead0(uint64_t v) { return __clzll((long long)v); }
 
-// One wave: the hits of row `row` (home atom s, tile index ui) in the staged block,
-// whose first candidate is tile index cb.  SINGLE: the block is the whole tile and the
-// row collects in the wave's LDS buffer; else over the blocks in its slots in global
-// memory.  It collects from both ends, the LJ-range entries at the front and the others
-// at the back, unless their counts are known first.  have: entries that earlier blocks
-// gave the row.  The last block writes the row.
+// One wave: the hits of row `row` (home atom s) in the staged block, whose first candidate is
+// tile index cb.  SINGLE: the block is the whole tile, and the row collects in the wave's LDS
+// buffer, the LJ range first; else over the blocks in its slots in global memory, the LJ range
+// from the front and the others from the back.  have: entries that earlier blocks gave the row.
+// The last block writes the row.
 template <bool RBL, typename W, bool SINGLE>
 __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListLds& L, int row,
                                 int s, int cb, const int32_t* ids, int T, int lane_in, bool last,
@@ -577,7 +576,6 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
         if (SINGLE) L.buf[k] = (uint16_t)u;
         else rowp[k] = (uint16_t)u;
     };
-    bool ordered = false;  // the others already stand behind the LJ range
     {
         constexpr int kBits = 8 * sizeof(W);
         const int wo = (row * 4 + g) * 16 + col;
@@ -649,7 +647,6 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
         if (ci + co + ni + no < cap) {
             expand(mi, ci, put1);
             expand(mo, SINGLE ? ni : co, [&](int k, int u) { put1(SINGLE ? k : cap - 1 - k, u); });
-            ordered = SINGLE;
         }
         ci += ni;
         co += no;
@@ -662,14 +659,8 @@ __device__ inline int2 row_hits(const TileHdr& h, const ListArgs& a, const ListL
             // the row from global memory into the buffer, in order
             __threadfence_block();
             for (int k = lane; k < n; k += 64)
-                L.buf[k] = rowp[k < ci || ordered ? k : cap - 1 - (k - ci)];
-        } else if (!ordered) {
-            // close the gap between the LJ range and the others: the last of them move
-            // into it (the source starts at or behind the gap's end)
-            const int cnt = min(co, cap - n);
-            for (int k = lane; k < cnt; k += 64) L.buf[ci + k] = L.buf[cap - cnt + k];
+                L.buf[k] = rowp[k < ci ? k : cap - 1 - (k - ci)];
         }
-        __syncwarp();
         // two entries per 32-bit word (rows start at multiples of 64 entries)
         if (lane == 0) L.buf[n] = (uint16_t)total;
         __syncwarp();
