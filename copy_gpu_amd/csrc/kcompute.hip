@@ -10,8 +10,8 @@
 //   rho(k) worklet                       rbmd/framework/run/worklet/RunWorklet.cpp:1616-1677
 //   RBE force worklet                    RunWorklet.cpp:1508-1548, ExecForceFunction.h:247-269
 //
-// Calls of at most 4,096 atoms that ask for rho need no scratch: one workgroup per k writes
-// rho, and the force kernel forms coefficients and terms from it (1,000 atoms, 124
+// Calls of few atoms and k-vectors that ask for rho need no scratch (ks_small): one workgroup
+// per k writes rho, and the force kernel forms coefficients and terms from it (1,000 atoms, 124
 // k-vectors, FP64: 92 -> 44 us a call).  For others rbmd_kspace_compute allocates its scratch (partials,
 // rho, per-k coefficients and terms, weights) for the call.  rbmd_kspace_compute_noalloc
 // runs the same kernels on a fixed block of device memory (`scratch` below, 4 MiB per
@@ -77,7 +77,8 @@ KsLayout ks_layout(int64_t n, int P)
 
 namespace {
 
-constexpr int kKsSmall = 4096;  // most atoms of the calls without scratch
+constexpr int kKsSmall = 4096;    // most atoms of the calls without scratch
+constexpr int kKsSmallP = 16384;  // and most k-vectors
 
 // rho(k) of at most kKsSmall atoms: one workgroup per k, each thread 16 atoms at most, so no
 // partials go through memory.  (With more atoms the loop would be longer than the reduction
@@ -207,9 +208,20 @@ struct KsCall {
     double* ev_out;
 };
 
-// Whether a call runs without scratch memory.
-bool ks_small(const KsCall& c) { return c.rho_out && c.n <= kKsSmall; }
+// Whether a call runs without scratch memory; the same for both entry points, which give the
+// same bits.  Every k reads all positions again and every force workgroup forms all
+// coefficients, so the general path overtakes with P, though it has to allocate (or, in the
+// second figure of each, has the fixed scratch).  Without and with scratch, us: FP32, 4,096
+// atoms 117 / 97 and 127 / 70 for 4,000 k-vectors, 222 / 202 and 185 / 127 for 8,192, 790 and
+// 489 for 30,000; 1,000 atoms 255 and 275 for 16,000.  FP64, 4,096 atoms 210 / 190 and 230 /
+// 175 for 4,000, 573 and 561 for 12,000; 1,000 atoms 665 and 640 for 16,000.
+bool ks_small(const KsCall& c)
+{
+    const int64_t most = (int64_t)1 << (c.precision == 32 ? 24 : 25);
+    return c.rho_out && c.n <= kKsSmall && c.P <= kKsSmallP && c.n * c.P <= most;
+}
 
+// buf: scratch, or null for a call that runs without (ks_small).
 template <typename T>
 void ks_launch(const KsCall& c, char* buf, hipStream_t s)
 {
@@ -234,7 +246,7 @@ void ks_launch(const KsCall& c, char* buf, hipStream_t s)
     const int nforce = c.n > 0 ? kf_blocks(c.n, ka.slices) : 0, nev = c.ev_out ? 7 : 0;
     ka.staged = kf_staged<T>(nforce, c.P);
     const double wdef = c.w ? 0.0 : rbe_S(c.alpha, c.L) / (double)c.P;
-    if (ks_small(c)) {
+    if (!buf) {
         k_ks_rho<T><<<c.P, 256, 0, s>>>(c.x, c.y, c.z, c.q, (int)c.n, box, c.m, c.rho_out);
         if (nforce + nev > 0)
             k_one<KsForce<T, true>><<<nforce + nev, kKfThreads, 0, s>>>(
@@ -415,8 +427,10 @@ int rbmd_kspace_compute_noalloc(const rbmd_kspace_params* p, int64_t n, const do
                            " exceeds the fixed scratch (P <= " +
                            std::to_string(kKsScratchMaxP) + ")");
     char* buf = nullptr;
-    rc = ks_scratch_ptr(&buf);
-    if (rc != RBMD_OK) return rc;
+    if (!ks_small(c)) {
+        rc = ks_scratch_ptr(&buf);
+        if (rc != RBMD_OK) return rc;
+    }
     ks_dispatch(c, buf, (hipStream_t)stream);
     const hipError_t st = hipGetLastError();
     if (st != hipSuccess) return ks_fail(RBMD_ERR_HIP, std::string("launch: ") + hipGetErrorString(st));

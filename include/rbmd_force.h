@@ -291,8 +291,8 @@ typedef struct {
     int32_t precision;  /* 32: FP32 sines and force sums, 64: FP64          */
 } rbmd_kspace_params;
 
-/* Allocates scratch (device memory) for the call unless n <= 4096 and rho is asked for, and
- * synchronises the stream. */
+/* Allocates scratch (device memory) for the call unless rho is asked for and n <= 4096,
+ * P <= 16384 and n P <= 2^24 (FP64: 2^25), and synchronises the stream. */
 int rbmd_kspace_compute(const rbmd_kspace_params* p, int64_t n, const double* x, const double* y,
                         const double* z, const double* q, int32_t P, const int32_t* m,
                         const double* w, void* fx, void* fy, void* fz, double* rho, double* ev,

@@ -150,3 +150,44 @@ def test_kspace_compute_against_oracle(n, P, weights, precision):
     assert np.abs(out.T - Fk).max() <= tol * term + 2 * eps * np.abs(F0).max()
     e = (w * 2 * np.pi / V * (np.hypot(re, im) + tol * s) ** 2 / k2 * (4 + k2 / alpha)).sum()
     assert np.abs(ev.cpu().numpy() - evk).max() <= 4 * tol * (e + (w * s * s / k2).sum() / V * 2 * np.pi)
+
+
+# the last and first calls without and with scratch: 2^24 (FP64: 2^25) atoms times k-vectors,
+# 16,384 k-vectors
+@pytest.mark.parametrize("n,P,precision", [(4096, 4096, 32), (4096, 4097, 32), (4096, 8192, 64),
+                                           (4096, 8193, 64), (60, 16384, 64), (60, 16385, 64)])
+def test_kspace_compute_either_side_of_scratch(n, P, precision):
+    """Both sides against the oracle, with the error model of the test above; the call on the
+    fixed scratch gives the same bits."""
+    import oracle
+    from copy_gpu_amd import force as FM
+
+    rng = np.random.default_rng(n + P)
+    Lb, alpha = np.array([31.0, 42.5, 30.0]), 0.1
+    pos = rng.uniform(0, 1, (3, n)) * Lb[:, None]
+    q = rng.uniform(-1, 1, n)
+    g = np.stack(np.meshgrid(*[np.arange(-13, 14)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    g = g[(g != 0).any(1)]
+    m = g[rng.permutation(len(g))[:P]].astype(np.int32)
+    w = rng.uniform(0.5, 2.0, P)
+    dt = torch.float32 if precision == 32 else torch.float64
+    dev = lambda a, t=torch.float64: torch.as_tensor(np.ascontiguousarray(a)).cuda().to(t)  # noqa: E731
+    args = [tuple(Lb), alpha, *[dev(a) for a in pos], dev(q), dev(m.reshape(-1), torch.int32), dev(w)]
+    F = [torch.zeros(n, device="cuda", dtype=dt) for _ in range(3)]
+    rho, ev = FM.kspace_compute(*args, *F, precision=precision)
+    Fk, _ = oracle.kspace_forces(*pos, q, Lb, alpha, m, w)
+    re, im = oracle.rho(*pos, q, Lb, m)
+    tol = 1e-6 if precision == 32 else 1e-12
+    s = np.abs(q).sum()
+    assert np.abs(rho.cpu().numpy() - np.stack([re, im], 1)).max() <= tol * s
+    k = 2 * np.pi * m / Lb
+    term = np.abs(q).max() * (4 * np.pi * w / (Lb.prod() * np.sqrt((k * k).sum(1))) *
+                              (np.hypot(re, im) + s)).sum()
+    out = np.stack([a.double().cpu().numpy() for a in F])
+    assert np.abs(out.T - Fk).max() <= tol * term
+    if P <= 8192:
+        G = [torch.zeros(n, device="cuda", dtype=dt) for _ in range(3)]
+        rho2, ev2 = FM.kspace_compute(*args, *G, precision=precision, noalloc=True)
+        torch.cuda.synchronize()
+        assert torch.equal(rho, rho2) and torch.equal(ev, ev2)
+        assert all(torch.equal(a, b) for a, b in zip(F, G))
