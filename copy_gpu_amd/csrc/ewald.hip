@@ -72,6 +72,7 @@ __global__ __launch_bounds__(256) void k_ewald_final(RhoFinalArgs<double> A,
 constexpr int kEwAtoms = 64;
 constexpr int kEwStride = 80;  // doubles between table rows: two rows on disjoint banks
 constexpr int kEwX = 8;        // m_x held at a time (a tile of 16 rows spans at most 5)
+constexpr int kEwMaxLds = 140 * 1024;
 
 struct EwForceArgs {
     const double *x, *y, *z;
@@ -270,9 +271,10 @@ hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
     EwaldLat& l = e.ew;
     for (size_t k = 0; k < m.size(); ++k) l.M[k % 3] = std::max(l.M[k % 3], std::abs(m[k]));
     for (int d = 0; d < 3; ++d) l.M[d] = std::max(l.M[d], 1);
-    // the y basis of 64 atoms has to fit the LDS: boxes beyond (|m_y| > 100) keep the sums
+    // the y basis of 64 atoms has to fit the LDS: boxes beyond (|m_y| > 103) keep the sums
     // over single k-vectors
-    if (ewald_lds(l) > (size_t)std::min(e.lds_max, 140 * 1024) || e.n_max < 1) return hipSuccess;
+    const int lds = std::min(e.lds_max, kEwMaxLds);
+    if (ewald_lds(l) > (size_t)lds || e.n_max < 1) return hipSuccess;
     const int B = 2 * l.M[1] + 1, C = 2 * l.M[2] + 1;
     const int64_t R = (int64_t)(2 * l.M[0] + 1) * B;
     const int hy = l.M[1] + 1, hz = l.M[2] + 1;
@@ -339,9 +341,10 @@ hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
     l.fpart = (double*)(m0 + of);
     if ((st = hipMemcpy(m0, tab.data(), tab.size() * 4, hipMemcpyHostToDevice)) != hipSuccess ||
         (st = hipMemset(l.D, 0, dbytes)) != hipSuccess ||
+        (st = lattice_sums_prepare(g)) != hipSuccess ||
+        // (the limit belongs to the kernel, not to this handle: always the bound above)
         (st = hipFuncSetAttribute((const void*)k_ewald_force,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)ewald_lds(l))) != hipSuccess)
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds)) != hipSuccess)
         return st;
     l.on = true;
     return hipSuccess;

@@ -38,7 +38,17 @@ struct LatGeom {
     RBMD_HD int64_t sums() const { return R * (int64_t)C; }
 };
 
+// LDS that a sums kernel may be launched with: 256 rows touch at most 258 rows of the x and y
+// tables together.  The limit is a property of the kernel, shared by every caller, so it is set
+// to this bound and never to one call's need.
+constexpr size_t kLatMaxLds = ((size_t)(kLatRows + 2 + 64) * kLatStride + 4 * 8 * kLatStage +
+                               7 * 256) * sizeof(double);
+
 LatGeom lat_geometry(const int M[3], int64_t n);
+
+// Allows the sums kernel of a geometry its LDS; once per device before launch_lattice_sums (it
+// may be called again at any time).
+hipError_t lattice_sums_prepare(const LatGeom& g);
 
 // T of every slice into part [slices][R][C], then their sum in slice order into part[0].
 void launch_lattice_sums(const LatGeom& g, const Box& box, int64_t n, const double* x,

@@ -246,6 +246,7 @@ LatGeom lat_geometry(const int M[3], int64_t n)
     g.nx = std::min(2 * M[0] + 1, (kLatRows - 1) / g.B + 2);
     g.lds = ((size_t)(g.nx + g.ny + 16 * g.nc) * kLatStride +
              (size_t)4 * kLatBase * kLatStage + (size_t)7 * kLatLoad) * sizeof(double);
+    static_assert(kLatBase == 8 && kLatLoad == 256, "kLatMaxLds");
     // atom slices: one round of two workgroups per CU (a second, partial round would leave
     // CUs idle), while the partial sums stay bounded and a slice keeps two stages
     int64_t want = std::max<int64_t>(1, kLatTargetWg / ((int64_t)g.rblk * g.cblk));
@@ -258,24 +259,34 @@ LatGeom lat_geometry(const int M[3], int64_t n)
     return g;
 }
 
+// f(kernel of the geometry's column tiles)
+template <class F>
+static auto lat_kernel(const LatGeom& g, F f)
+{
+    switch (g.nc) {
+    case 1: return f(k_lat_sums<1>);
+    case 2: return f(k_lat_sums<2>);
+    case 3: return f(k_lat_sums<3>);
+    default: return f(k_lat_sums<4>);
+    }
+}
+
+hipError_t lattice_sums_prepare(const LatGeom& g)
+{
+    if (g.lds <= 65536) return hipSuccess;  // what any kernel may have
+    return lat_kernel(g, [](auto kern) {
+        return hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)kLatMaxLds);
+    });
+}
+
 void launch_lattice_sums(const LatGeom& g, const Box& box, int64_t n, const double* x,
                          const double* y, const double* z, const double* q, double* part,
                          hipStream_t s)
 {
     const LatSumArgs a{x, y, z, q, n, box, g, part};
     const dim3 grid(g.rblk, g.cblk, g.slices);
-    auto go = [&](auto kern) {
-        if (g.lds > 65536)
-            (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)g.lds);
-        kern<<<grid, 256, g.lds, s>>>(a);
-    };
-    switch (g.nc) {
-    case 1: go(k_lat_sums<1>); break;
-    case 2: go(k_lat_sums<2>); break;
-    case 3: go(k_lat_sums<3>); break;
-    default: go(k_lat_sums<4>); break;
-    }
+    lat_kernel(g, [&](auto kern) { kern<<<grid, 256, g.lds, s>>>(a); });
     if (g.slices > 1)
         k_lat_reduce<<<(unsigned)((g.sums() + 255) / 256), 256, 0, s>>>(part, g.sums(), g.slices);
 }
@@ -333,12 +344,15 @@ int rbmd_lattice_spectrum(const double* box_lo, const double* box_len, int64_t n
     const LatGeom g = lat_geometry(M, n);
     if (bytes < (int64_t)g.slices * g.sums() * (int64_t)sizeof(double))
         return lat_fail(RBMD_ERR_CAPACITY, "workspace smaller than rbmd_lattice_spectrum_workspace");
+    hipError_t st = lattice_sums_prepare(g);
+    if (st != hipSuccess)
+        return lat_fail(RBMD_ERR_HIP, std::string("dynamic LDS: ") + hipGetErrorString(st));
     hipStream_t s = (hipStream_t)stream;
     launch_lattice_sums(g, box, n, x, y, z, q, (double*)workspace, s);
     const int64_t pts = (int64_t)(Mg + 1) * (Mg + 1) * (Mg + 1);
     k_lat_spectrum<<<(unsigned)((pts + 255) / 256), 256, 0, s>>>((const double*)workspace, g.B, g.C,
                                                               Mg, accumulate, s2);
-    const hipError_t st = hipGetLastError();
+    st = hipGetLastError();
     if (st != hipSuccess)
         return lat_fail(RBMD_ERR_HIP, std::string("launch: ") + hipGetErrorString(st));
     return RBMD_OK;

@@ -191,3 +191,48 @@ def test_kspace_compute_either_side_of_scratch(n, P, precision):
         torch.cuda.synchronize()
         assert torch.equal(rho, rho2) and torch.equal(ev, ev2)
         assert all(torch.equal(a, b) for a, b in zip(F, G))
+
+
+def test_handles_and_spectra_of_unequal_boxes():
+    """Kernels' limit of dynamic LDS: a full Ewald handle and a spectrum that need more than 64 KiB
+    still run after smaller ones have been made and run."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+    from copy_gpu_amd import proposal as PR
+
+    rng = np.random.default_rng(5)
+    n = 200
+    q = rng.uniform(-1, 1, n)
+    dev = lambda a: torch.as_tensor(np.ascontiguousarray(a)).cuda()  # noqa: E731
+
+    def handle(L):
+        m = np.ceil(np.array(L) / 1.2).astype(int)
+        g = rng.permutation(m.prod())[:n]
+        p = (np.stack([g % m[0], g // m[0] % m[1], g // (m[0] * m[1])]) + 0.5) * (L / m)[:, None]
+        f = LJCutCoulKspaceForce(ForceConfig(box_len=tuple(L), cut_off=2.5, coulomb_cut=3.0,
+                                             alpha=0.5, kspace="EWALD", ewald_tol=1e-10,
+                                             precision=64, n_max=n))
+        f.Init(dev(q))
+        return f, [dev(a) for a in p]
+
+    def evaluate(f, p):
+        F = [torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+        f.Execute(*p, *F)
+        return torch.stack(F)
+
+    big = handle(np.array([8.0, 70.0, 8.0]))
+    mmax = np.abs(big[0].kspace()[0]).max(0)
+    # the y and x tables of 64 atoms, 80 doubles between rows
+    assert (2 * (mmax[1] + 1) + 16) * 80 * 8 > 65536 and mmax[1] <= 103
+    first = evaluate(*big)
+    small = handle(np.array([8.0, 8.0, 9.0]))
+    evaluate(*small)
+    assert torch.equal(evaluate(*big), first)
+
+    X = [dev(rng.uniform(0, 20, n)) for _ in range(3)]
+    spectrum = lambda Mg: PR.spectrum([tuple(X)], dev(q), (20.0,) * 3, 0.5, Mg)  # noqa: E731
+    first = spectrum(60)
+    spectrum(2)
+    assert np.array_equal(spectrum(60), first)
+    c = slice(58, 63)
+    cube = first.reshape(121, 121, 121)[c, c, c].ravel()
+    assert np.abs(cube - spectrum(2)).max() <= 1e-12 * cube.max()
