@@ -73,6 +73,11 @@ constexpr int kEwAtoms = 64;
 constexpr int kEwStride = 80;  // doubles between table rows: two rows on disjoint banks
 constexpr int kEwX = 8;        // m_x held at a time (a tile of 16 rows spans at most 5)
 constexpr int kEwMaxLds = 140 * 1024;
+// Fewest k-vectors that take the lattice: it has two to three launches more, and its sums and
+// forces fill 256-row and 64-column tiles whatever the box.  An evaluation without and with it,
+// us: 4,000 ions 29 and 58 for 46 k-vectors, 45 and 61 for 447, 70 and 67 for 1,051; 100,000
+// ions 334 and 358 for 459, 537 and 381 for 1,051; 64 ions 42 and 43 for 459, 62 and 49 for 1,051.
+constexpr int kEwMinK = 800;
 
 struct EwForceArgs {
     const double *x, *y, *z;
@@ -269,6 +274,7 @@ void ewald_free(Engine& e)
 hipError_t ewald_setup(Engine& e, const std::vector<int32_t>& m)
 {
     EwaldLat& l = e.ew;
+    if (m.size() / 3 < kEwMinK) return hipSuccess;
     for (size_t k = 0; k < m.size(); ++k) l.M[k % 3] = std::max(l.M[k % 3], std::abs(m[k]));
     for (int d = 0; d < 3; ++d) l.M[d] = std::max(l.M[d], 1);
     // the y basis of 64 atoms has to fit the LDS: boxes beyond (|m_y| > 103) keep the sums

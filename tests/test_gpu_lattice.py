@@ -236,3 +236,70 @@ def test_handles_and_spectra_of_unequal_boxes():
     c = slice(58, 63)
     cube = first.reshape(121, 121, 121)[c, c, c].ravel()
     assert np.abs(cube - spectrum(2)).max() <= 1e-12 * cube.max()
+
+
+# 118, 784 and 802 k-vectors: single k-vectors below 800, the lattice box from there
+@pytest.mark.parametrize("tol,P", [(1e-3, 118), (3e-11, 784), (2e-11, 802)])
+def test_ewald_of_few_kvectors(tol, P):
+    import oracle
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    rng = np.random.default_rng(P)
+    n, Lb = 60, np.array([6.0, 7.0, 6.5])
+    m = rng.permutation(125)[:n]
+    pos = (np.stack([m % 5, m // 5 % 5, m // 25]) + 0.5 + rng.uniform(-0.1, 0.1, (3, n))) * Lb[:, None] / 5
+    q = rng.uniform(-1.0, 1.0, n)
+    f = LJCutCoulKspaceForce(ForceConfig(box_len=tuple(Lb), cut_off=2.5, coulomb_cut=2.9, skin=0.3,
+                                         alpha=0.5, kspace="EWALD", precision=64, ewald_tol=tol,
+                                         n_max=n))
+    dev = lambda a: torch.as_tensor(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    f.Init(dev(q))
+    assert f.stats()["ewald_k"] == P
+    F = [torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+    for _ in range(2):
+        f.Execute(*[dev(a) for a in pos], *F, energy_virial=True)
+    mm, w, re, im = f.kspace()
+    Fk, evk = oracle.kspace_forces(*pos, q, Lb, 0.5, mm, w)
+    Fp, _ = oracle.pair_forces(*[np.ascontiguousarray(a) for a in pos], q, np.zeros(3), Lb, 2.5, 2.9, 0.5)
+    got = torch.stack(F, 1).cpu().numpy()
+    assert np.linalg.norm(got - Fp - Fk) <= 1e-12 * (np.linalg.norm(Fp) + np.linalg.norm(Fk))
+    r, i = _direct(pos, q, mm, np.zeros(3), Lb)
+    bound = np.abs(q).sum() * (2 * np.pi * 4 * np.abs(mm).max() + 16 + n / 8) * 2.0 ** -53
+    assert np.abs(re - r).max() <= bound and np.abs(im - i).max() <= bound
+    assert abs(f.energy_virial()["e_kspace"] - evk[0]) <= 1e-12 * abs(evk[0])
+
+
+def test_time_of_few_kvectors():
+    """20,000 ions and 46 k-vectors in FP64: a full Ewald evaluation takes no more than 1.3 times
+    that of as many sampled k-vectors."""
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+
+    n, m = 20000, 28
+    g = np.random.default_rng(1).permutation(m ** 3)[:n]
+    L = 1.5 * m
+    X = [torch.as_tensor(a).cuda() for a in (np.stack([g % m, g // m % m, g // m ** 2]) + 0.5) * 1.5]
+    q = torch.as_tensor(np.where(g % 2, 1.0, -1.0)).cuda()
+    us = {}
+    for kind in ("RBE", "EWALD"):
+        # |m| <= 2.9 at a tolerance of 1e-4
+        alpha = (2 * np.pi * 2.9 / L) ** 2 / (4 * np.log(1e4))
+        f = LJCutCoulKspaceForce(ForceConfig(box_len=(L,) * 3, cut_off=2.5, coulomb_cut=5.0,
+                                             alpha=alpha, kspace=kind, coulomb_sample_num=46,
+                                             ewald_tol=1e-4, precision=64, n_max=n))
+        f.Init(q)
+        if kind == "RBE":
+            f.sample_kvectors(46, 1, 0)
+        else:
+            assert f.stats()["ewald_k"] == 46
+        F = [torch.zeros(n, device="cuda", dtype=torch.float64) for _ in range(3)]
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        for _ in range(5):
+            f.Execute(*X, *F)
+        t[0].record()
+        for _ in range(30):
+            f.Execute(*X, *F)
+        t[1].record()
+        torch.cuda.synchronize()
+        us[kind] = 1e3 * t[0].elapsed_time(t[1]) / 30
+    print(f"evaluation: {us}", flush=True)
+    assert us["EWALD"] < 1.3 * us["RBE"]
