@@ -1524,7 +1524,7 @@ int rbmd_batch_md_run(rbmd_batch_t b, const rbmd_replica_state* st, double dt, i
         };
         for (const BatchPhase& ph : B.ph) key_phase(ph);
         for (const BatchPhase& ph : B.pair_more) key_phase(ph);
-        key.push_back((const void*)(uintptr_t)(B.thermo ? 1 : 0));
+        key.push_back((const void*)(uintptr_t)((B.thermo ? 1 : 0) + (B.kf_staged ? 2 : 0)));
         const int rem = (int)(nsteps % kGraphSteps);
         for (int g : {0, rem}) {
             Engine::StepGraph& G = b->graphs[g];

@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256) void k_ks_rho(const double* __restrict__ x,
 
 // The k-space forces (workgroups [0, nforce)) and, one workgroup each, the seven sums of
 // energy and virial terms in a fixed order.  DIRECT: coefficients and terms from rho, by each
-// workgroup for itself; else those that the rho(k) reduction stored.
-template <typename T, bool DIRECT>
+// workgroup for itself; else those that the rho(k) reduction stored.  STAGED: in LDS.
+template <typename T, bool DIRECT, bool STAGED = DIRECT>
 struct KsForce {
     static constexpr int kThreads = kKfThreads;
     struct Args {
@@ -144,7 +144,7 @@ struct KsForce {
     }
     __device__ static void run(const Args& A, int blk, int)
     {
-        __shared__ typename std::conditional<DIRECT, KForceStagedLds<T>, KForceLds<T>>::type L;
+        __shared__ KForceLds<T, STAGED> L;
         if (blk < A.nforce) {
             auto pre = [](int) { return 0; };
             auto fin = [&](int i, T f0, T f1, T f2, int) {
@@ -244,7 +244,6 @@ void ks_launch(const KsCall& c, char* buf, hipStream_t s)
     ka.fz = (T*)c.fz;
     ka.slices = kf_slices(c.n, c.P);
     const int nforce = c.n > 0 ? kf_blocks(c.n, ka.slices) : 0, nev = c.ev_out ? 7 : 0;
-    ka.staged = kf_staged<T>(nforce, c.P);
     const double wdef = c.w ? 0.0 : rbe_S(c.alpha, c.L) / (double)c.P;
     if (!buf) {
         k_ks_rho<T><<<c.P, 256, 0, s>>>(c.x, c.y, c.z, c.q, (int)c.n, box, c.m, c.rho_out);
@@ -273,8 +272,11 @@ void ks_launch(const KsCall& c, char* buf, hipStream_t s)
         kpart, nbx, c.P, c.m, w, box, c.alpha, c.qqr2e, rho, coef, kev, nullptr});
     ka.coef = coef;
     if (nforce + nev > 0)
-        k_one<KsForce<T, false>><<<nforce + nev, kKfThreads, 0, s>>>(typename KsForce<T, false>::Args{
-            ka, nforce, c.alpha, c.qqr2e, c.m, w, wdef, rho, kev, c.ev_out});
+        kf_dispatch<T>(kf_staged<T>(nforce, c.P), [&](auto sg) {
+            using K = KsForce<T, false, decltype(sg)::value>;
+            k_one<K><<<nforce + nev, kKfThreads, 0, s>>>(typename K::Args{
+                ka, nforce, c.alpha, c.qqr2e, c.m, w, wdef, rho, kev, c.ev_out});
+        });
 }
 
 thread_local std::string g_ks_err;

@@ -369,21 +369,18 @@ struct KForceArgs {
     ThermoArgs th;  // velocity thermostat of the closing kick (KForce<T, true>)
     const double* rbl_mean = nullptr;  // random batch list: mean near force to subtract
     int slices = kKfSlices;            // k-slices per atom group (kf_slices)
-    int staged = 0;                    // kf_staged
 };
 
-// LDS: the sums of the slices, and a stage of coefficients.
-template <typename T>
-struct KForceSumLds {
+// LDS: the sums of the slices, and the stage of coefficients where there is one.  (Kernels of
+// their own with and without: a switch inside cost the launches without 1% of an MD step.)
+template <typename T, bool STAGED = false>
+struct KForceLds {
     T red[kKfSlices][3][kKfAtoms];
 };
 template <typename T>
-struct KForceStagedLds : KForceSumLds<T> {
+struct KForceLds<T, true> : KForceLds<T, false> {
     KCoef<T> st[kKfStage];
 };
-// that of coefficients in memory: FP64 launches stage none
-template <typename T>
-using KForceLds = typename std::conditional<sizeof(T) == 4, KForceStagedLds<T>, KForceSumLds<T>>::type;
 
 // The k-space force of the atoms of workgroup blk.  Each lane of an atom-owning
 // wave (slice 0 of its atom group) first calls pre(i) for its atom i < n (loads
@@ -391,7 +388,8 @@ using KForceLds = typename std::conditional<sizeof(T) == 4, KForceStagedLds<T>, 
 // overlaps it), then, after the k-sum, fin(i, f0, f1, f2, pre_value) with the
 // complete force (pair force + k-space).
 // fin runs with FP contraction off in the caller's body.
-// coef(k) gives the coefficients of k-vector k.
+// coef: the coefficients in memory, by scalar loads; or coef(k) gives those of k-vector k for
+// the stage.
 template <typename T, class Lds, class Coef, class Pre, class Fin>
 __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coef coef, Pre pre,
                                     Fin fin)
@@ -437,24 +435,7 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coe
         ay = fma_t(g, c.k[1], ay);
         az = fma_t(g, c.k[2], az);
     };
-    constexpr bool kMem = std::is_same<Coef, const KCoef<T>*>::value;
-    auto stage = [&](auto of) {
-        if constexpr (std::is_base_of<KForceStagedLds<T>, Lds>::value) {
-            for (int base = 0; base < P; base += kKfStage) {
-                __syncthreads();
-                for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
-                    L.st[k] = of(base + k);
-                __syncthreads();
-                const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
-                for (int k = slice; k < cnt; k += slices) add(L.st[k]);
-            }
-        }
-    };
-    if constexpr (!kMem) {
-        stage(coef);
-    } else if (sizeof(T) == 4 && A.staged) {
-        stage([&](int k) { return coef[k]; });
-    } else {
+    if constexpr (std::is_same<Coef, const KCoef<T>*>::value) {
         int k = uniform(slice);
         // four k's loads in flight together
         for (; k + 3 * slices < P; k += 4 * slices) {
@@ -468,6 +449,17 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coe
             add(c3);
         }
         for (; k < P; k += slices) add(const_mem(coef + k));
+    } else {
+        for (int base = 0; base < P; base += kKfStage) {
+            __syncthreads();
+            for (int k = threadIdx.x; k < kKfStage && base + k < P; k += kKfThreads)
+                L.st[k] = coef(base + k);
+            __syncthreads();
+            const int cnt = (P - base) < kKfStage ? (P - base) : kKfStage;
+            // two k's in flight: 55 -> 50 us for 10,000 atoms and 4,000 k-vectors in a step (four: 54)
+#pragma unroll 2
+            for (int k = slice; k < cnt; k += slices) add(L.st[k]);
+        }
     }
     if (P > 0 && slices > 1) {
         L.red[wv][0][lane] = ax;
@@ -498,11 +490,14 @@ __device__ inline void kforce_block(const KForceArgs<T>& A, int blk, Lds& L, Coe
     }
 }
 
-template <typename T, class Pre, class Fin>
-__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T>& L, Pre pre,
-                                    Fin fin)
+template <typename T, bool STAGED, class Pre, class Fin>
+__device__ inline void kforce_block(const KForceArgs<T>& A, int blk, KForceLds<T, STAGED>& L,
+                                    Pre pre, Fin fin)
 {
-    kforce_block(A, blk, L, A.coef, pre, fin);
+    if constexpr (STAGED)
+        kforce_block(A, blk, L, [&](int k) { return A.coef[k]; }, pre, fin);
+    else
+        kforce_block(A, blk, L, A.coef, pre, fin);
 }
 
 // Velocity and mass of atom i for the closing half kick, and the thermostat's
@@ -584,7 +579,7 @@ struct ThermoReduce {
 // the Nose-Hoover half step v += dt/2 (F/m - xi v) after it
 // (UpdateVelocityNoseHooverWorklet, RunWorklet.cpp:1784-1804), and each
 // workgroup's sum of m |v|^2 of the kicked velocities (reduced by ThermoReduce).
-template <typename T, bool KICK>
+template <typename T, bool KICK, bool STAGED = false>
 struct KForce {
     static constexpr int kThreads = kKfThreads;
     using Args = KForceArgs<T>;
@@ -592,7 +587,7 @@ struct KForce {
     {
 #pragma clang fp contract(off)
         if (KICK && blk == 0 && threadIdx.x == 0) A.flags[3] += 1u;  // MD step epoch
-        __shared__ KForceLds<T> L;
+        __shared__ KForceLds<T, STAGED> L;
         const ThermoArgs& th = A.th;
         double ke = 0;
         kforce_block(
@@ -682,6 +677,19 @@ inline RhoFinalArgs<T> rho_final_args(Engine& e, unsigned long long* step_dev)
 inline int kforce_P(const Engine& e) { return has_kspace(e) ? e.P : 0; }
 inline int kforce_blocks(const Engine& e) { return kf_blocks(e.n, kf_slices(e.n, kforce_P(e))); }
 
+// f(true type) if the launch stages its coefficients, else f(false type).
+template <typename T, class F>
+inline void kf_dispatch(bool staged, F f)
+{
+    if constexpr (sizeof(T) == 4) {
+        if (staged) {
+            f(std::true_type{});
+            return;
+        }
+    }
+    f(std::false_type{});
+}
+
 template <typename T>
 inline KForceArgs<T> kforce_args(Engine& e, const double* x, const double* y, const double* z,
                                  void* fx, void* fy, void* fz, double* vx, double* vy,
@@ -692,7 +700,6 @@ inline KForceArgs<T> kforce_args(Engine& e, const double* x, const double* y, co
                     e.flags};
     a.rbl_mean = e.rbl ? e.rbl_mean : nullptr;
     a.slices = kf_slices(e.n, a.P);
-    a.staged = kf_staged<T>(kf_blocks(e.n, a.slices), a.P);
     return a;
 }
 

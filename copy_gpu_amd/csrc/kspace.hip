@@ -78,12 +78,16 @@ void launch_kforce(Engine& e, const double* x, const double* y, const double* z,
         return;
     }
     ScopedTimer t(e, P_KFORCE, s);
-    if (e.precision == 32)
-        k_one<KForce<float, false>><<<kforce_blocks(e), kKfThreads, 0, s>>>(
-            kforce_args<float>(e, x, y, z, fx, fy, fz, nullptr, nullptr, nullptr, nullptr, 0.0));
-    else
-        k_one<KForce<double, false>><<<kforce_blocks(e), kKfThreads, 0, s>>>(
-            kforce_args<double>(e, x, y, z, fx, fy, fz, nullptr, nullptr, nullptr, nullptr, 0.0));
+    auto go = [&](auto t) {
+        using T = decltype(t);
+        const int blocks = kforce_blocks(e);
+        const auto a = kforce_args<T>(e, x, y, z, fx, fy, fz, nullptr, nullptr, nullptr, nullptr, 0.0);
+        kf_dispatch<T>(kf_staged<T>(blocks, a.P), [&](auto st) {
+            k_one<KForce<T, false, decltype(st)::value>><<<blocks, kKfThreads, 0, s>>>(a);
+        });
+    };
+    if (e.precision == 32) go(0.0f);
+    else go(0.0);
 }
 
 }  // namespace rbmd

@@ -235,7 +235,7 @@ struct VScale {
 // (and its k-vector draw): the lane that completes atom i's force carries its
 // velocity through both half kicks; the atom's other inputs are loaded before
 // the k-space sum.
-template <typename T>
+template <typename T, bool STAGED = false>
 struct KForceDrift {
     static constexpr int kThreads = kKfThreads;
     struct Args {
@@ -250,7 +250,7 @@ struct KForceDrift {
     {
 #pragma clang fp contract(off)
         __shared__ union {
-            KForceLds<T> kf;
+            KForceLds<T, STAGED> kf;
             double cdf[kSamplerLds];
         } lds;
         if (blk == 0 && threadIdx.x == 0) A.kf.flags[3] += 1u;  // MD step epoch

@@ -132,16 +132,22 @@ void md_sort_rho_t(Engine& e, const RepState& st, hipStream_t s)
 template <typename T>
 void md_close_t(Engine& e, const RepState& st, double dt, hipStream_t s)
 {
-    k_one<KForce<T, true>><<<std::max(kforce_blocks(e), 1), kKfThreads, 0, s>>>(
-        close_args<T>(e, st, dt));
+    const int blocks = std::max(kforce_blocks(e), 1);
+    kf_dispatch<T>(kf_staged<T>(blocks, kforce_P(e)), [&](auto sg) {
+        k_one<KForce<T, true, decltype(sg)::value>><<<blocks, kKfThreads, 0, s>>>(
+            close_args<T>(e, st, dt));
+    });
 }
 
 template <typename T>
 void md_close_open_t(Engine& e, const RepState& st, double dt, const SampleArgs& sa,
                      hipStream_t s)
 {
-    k_one<KForceDrift<T>><<<close_open_blocks(e, sa), kKfThreads, 0, s>>>(
-        close_open_args<T>(e, st, dt, sa));
+    const auto a = close_open_args<T>(e, st, dt, sa);
+    kf_dispatch<T>(kf_staged<T>(kforce_blocks(e), kforce_P(e)), [&](auto sg) {
+        using K = KForceDrift<T, decltype(sg)::value>;
+        k_one<K><<<close_open_blocks(e, sa), kKfThreads, 0, s>>>(typename K::Args{a.kf, a.kd});
+    });
 }
 
 template <typename T>
@@ -166,9 +172,12 @@ hipError_t md_prepare_t(Batch& b)
     }
     // one launch holds the workgroups of every replica
     int64_t blocks = 0;
-    for (int k : nkc) blocks += k;
-    for (size_t r = 0; r < R; ++r)
-        kc[r].staged = ko[r].kf.staged = kf_staged<T>(blocks, kc[r].P);
+    int P = 0;
+    for (size_t r = 0; r < R; ++r) {
+        blocks += nkc[r];
+        P = std::max(P, kc[r].P);
+    }
+    b.kf_staged = kf_staged<T>(blocks, P);
     hipError_t err;
     if ((err = phase_upload(b.ph[BP_KICKDRIFT], kd, nkd, 0)) != hipSuccess) return err;
     if ((err = phase_upload(b.ph[BP_SORT_RHO], sr, nsr, 0)) != hipSuccess) return err;
@@ -272,9 +281,13 @@ void md_batch_launch(Batch& b, int phase, hipStream_t s)
     switch (phase) {
     case BP_KICKDRIFT: RBMD_MB(KickDrift); break;
     case BP_SORT_RHO: RBMD_MB(SortRho); break;
-    case BP_KFORCE_DRIFT: RBMD_MB(KForceDrift); break;
+    case BP_KFORCE_DRIFT:
+        if (b.kf_staged) phase_launch<KForceDrift<float, true>>(b.ph[phase], s);
+        else RBMD_MB(KForceDrift);
+        break;
     case BP_KFORCE:
-        if (f32) phase_launch<KForce<float, true>>(b.ph[phase], s);
+        if (b.kf_staged) phase_launch<KForce<float, true, true>>(b.ph[phase], s);
+        else if (f32) phase_launch<KForce<float, true>>(b.ph[phase], s);
         else phase_launch<KForce<double, true>>(b.ph[phase], s);
         break;
     case BP_THERMO_BEGIN: phase_launch<ThermoBegin>(b.ph[phase], s); break;

@@ -228,6 +228,7 @@ struct Batch {
     int kspace = 0;
     bool multi = false;
     bool thermo = false;  // some replica has a thermostat: one segment per step
+    bool kf_staged = false;  // k-space force launches with their coefficients in LDS
     unsigned long long step0 = 0;  // first step of the run (MdBin sets the counters)
     // per replica kStatsOutWords words: the 8 build statistics, then flags[0..4];
     // device block and its pinned host mirror, one copy per run
