@@ -565,7 +565,9 @@ struct TilePass {
         // list build number (the random batch list's selection epoch); the build
         // kernels before this one have counted the current build
         const uint32_t epoch = RBL ? (uint32_t)A.stats[0] : 0u;
-        if (rebuild) {
+        // (out of line: the steps without a rebuild, most of them, run straight on; 17.1 -> 17.0 us a
+        // step at 500 ions, 62.3 -> 62.0 at 100,000)
+        if (__builtin_expect(rebuild, 0)) {
             const Args& R = reload<Args>(self);
             if (!staged && part == 0 && threadIdx.x == 0) atomicAdd(&R.stats[6], 1ull);
             const int cc = opaque(c);  // its divisions stay off the steps without a rebuild
