@@ -312,12 +312,20 @@ constexpr int kMaskRow = 256;     // bytes of a row's mask (64 uint32 words)
 // Staged candidates of a build: whole 16-candidate chunks.
 __host__ __device__ inline int list_len(int stage_cap) { return (stage_cap + 15) / 16 * 16; }
 
+// Row buffers of a build, one per wave.  Rows of more than 8,192 entries leave room for seven
+// beside the smallest stage and its masks (up to the 9,600 entries that handles accept); the
+// last wave then writes no rows.
+__host__ __device__ inline int list_bufs(int cap)
+{
+    return cap <= 8192 ? kTileWaves : kTileWaves - 1;
+}
+
 // Rows of one mask group (a multiple of 16): as many as fit beside the candidates in
 // the LDS that the pair pass's stage takes anyway (pass_bytes), between 32 and 64.
 inline size_t list_fixed_bytes(int stage_cap, int cap, bool rbl)
 {
     return (size_t)(rbl ? 20 : 16) * (size_t)list_len(stage_cap) +
-           (size_t)kTileWaves * (size_t)cap * sizeof(uint16_t);
+           (size_t)list_bufs(cap) * (size_t)cap * sizeof(uint16_t);
 }
 inline int list_rows(int stage_cap, int cap, size_t pass_bytes, bool rbl)
 {
@@ -327,7 +335,7 @@ inline int list_rows(int stage_cap, int cap, size_t pass_bytes, bool rbl)
 }
 
 // LDS bytes of the list build: the candidates (and, for a random batch list, their atom
-// ids), a row buffer of cap entries per wave and two masks of `rows` rows.
+// ids), the row buffers of cap entries and two masks of `rows` rows.
 inline size_t list_lds_bytes(int stage_cap, int cap, int rows = 32, bool rbl = false)
 {
     return list_fixed_bytes(stage_cap, cap, rbl) + 2 * kMaskRow * (size_t)rows;
@@ -337,7 +345,8 @@ struct ListLds {
     float4* cand;    // [list_len]
     char* mask;      // two masks, mask_bytes apart: hits, then their LJ-range ones
     int mask_bytes;
-    uint16_t* buf;   // this wave's row buffer [cap]
+    uint16_t* buf;   // this wave's row buffer [cap], waves below bufs
+    int bufs;
     int32_t* ids;    // random batch list: [list_len] atom ids
     __device__ ListLds(double4* lds, int stage_cap, int cap, int rows, int wv)
     {
@@ -346,7 +355,8 @@ struct ListLds {
         mask_bytes = kMaskRow * rows;
         uint16_t* b = (uint16_t*)(mask + 2 * mask_bytes);
         buf = b + (size_t)wv * cap;
-        ids = (int32_t*)(b + (size_t)kTileWaves * cap);
+        bufs = list_bufs(cap);
+        ids = (int32_t*)(b + (size_t)bufs * cap);
     }
 };
 
@@ -698,7 +708,7 @@ __device__ inline void list_block(const TileHdr& h, const ListArgs& a, const Lis
         else near_masks<1, H>(h, a, cand, R, L, cb, r0, nch, T, wv, lane);
     }
     __syncthreads();
-    for (int row = wv; row < nrow; row += kTileWaves) {
+    for (int row = wv < L.bufs ? wv : nrow; row < nrow; row += L.bufs) {
         if (single) {
             row_hits<RBL, W, true>(h, a, L, row, s0 + row, cb, ids, T, lane, true,
                                    make_int2(0, 0), rb);

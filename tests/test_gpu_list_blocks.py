@@ -174,3 +174,39 @@ def test_position_that_is_not_a_number(gpu, sign, stage):
             assert og[701] == og[700]
     # the same terms in another order: a few hundred, none above the largest force by much
     assert np.abs(forces[0] - forces[1]).max() <= 1e-12 * np.abs(forces[1]).max()
+
+
+# the longest rows of eight row buffers, of seven, and the longest accepted; one more is refused
+@pytest.mark.parametrize("neighbors,cap", [("VERLET-LIST", 8192), ("VERLET-LIST", 8256),
+                                           ("VERLET-LIST", 9600), ("VERLET-LIST", 9664),
+                                           ("RBL", 9472), ("RBL", 9536), ("RBL", 9600)])
+def test_longest_rows(orc, gpu, neighbors, cap):
+    from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce
+    from copy_gpu_amd.force import RBMDError
+
+    rng = np.random.default_rng(cap)
+    n, L = 1200, 2.5  # one cell: 32,400 candidates of 27 images, rows of some 4,190 n / 1000
+    m = 11
+    g = rng.permutation(m ** 3)[:n]
+    p = (np.stack([g % m, g // m % m, g // m ** 2]) + rng.uniform(0.3, 0.7, (3, n))) * (L / m)
+    cfg = ForceConfig(box_len=(L,) * 3, cut_off=2.0, coulomb_cut=2.0, skin=0.45, alpha=0.5,
+                      kspace="NONE", n_max=n, list_capacity=cap, neighbor_type=neighbors,
+                      r_core=1.0, rbl_pice=1)
+    # 159,744 bytes hold 24 (RBL: 28) a candidate for 256 candidates and 16 an entry
+    if cap > (9536 if neighbors == "RBL" else 9600):
+        with pytest.raises(RBMDError):
+            LJCutCoulKspaceForce(cfg)
+        return
+    f = LJCutCoulKspaceForce(cfg)
+    f.Init(_dev(rng.uniform(-1, 1, n)))
+    F = [torch.zeros(n, device="cuda") for _ in range(3)]
+    f.Execute(*[_dev(a) for a in p], *F)
+    st = f.stats()
+    assert st["cap"] == cap and st["overflow_rows"] == 0 and st["cells"] == 1
+    Lb = np.array([L] * 3)
+    w = [np.ascontiguousarray(a) for a in orc.wrap(*p, np.zeros(3), Lb)]
+    oo, io = orc.neighbors_images(*w, Lb, 2.45)
+    og, ig = f.neighbors()
+    assert og[-1] == oo[-1] and np.diff(og).max() > 4096
+    for i in range(n):
+        assert np.array_equal(np.sort(ig[og[i]:og[i + 1]]), np.sort(io[oo[i]:oo[i + 1]])), i
