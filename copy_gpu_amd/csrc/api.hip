@@ -455,7 +455,7 @@ int rbmd_force_create(const rbmd_force_params* p, int64_t n_max, rbmd_force_t* o
         CR(dalloc(&E.md_bucket, bucket + spill));
         CR(hipMemset((char*)E.md_bucket + bucket, 0xff, spill));
         CR(dalloc(&E.md_cell, N * 4));
-        CR(dalloc(&E.md_vid, 2 * N * 4));
+        CR(dalloc(&E.md_vid, N * 4));
         CR(dalloc(&E.md_w, N * 3 * 8));
     }
     CR(dalloc(&E.cell_start, ((size_t)E.ncell + 1) * 4));

@@ -72,7 +72,8 @@ struct MdBins {
     // lists per cell.  Empty (-1) between evaluations: the cell sort that reads a cell's
     // lists empties them.
     int32_t* spill;        // [ncell][kSpillChains] first atom
-    int32_t* spill_next;   // [n] by atom
+    int2* spill_next;      // [n] by atom, x: the next one.  The reference positions' memory, which
+                           // the cell sort writes after an atom's list has been read
 };
 // Lists per cell: one lane of the cell sort walks each, so an atom of 1,000 beyond the
 // bucket is at most 32 dependent loads away.

@@ -412,7 +412,7 @@ __device__ inline void cellsort_md(const CellSortMDArgs& a, int blk, int parts, 
             for (uint64_t m; found < cnt && (m = __ballot(u >= 0)) != 0ull; found += __popcll(m)) {
                 const int k = found + (int)mbcnt64(m);
                 if (u >= 0 && k < cnt) buf[k] = u;
-                u = u >= 0 ? a.bins.spill_next[u] : -1;
+                u = u >= 0 ? a.bins.spill_next[u].x : -1;
             }
         __syncwarp();
         for (int k = part * 64 + lane; k < cnt; k += 64 * parts) {

@@ -274,7 +274,7 @@ inline MdBins md_bins(const Engine& e)
     return MdBins{e.md_count, e.md_count + 2 * (size_t)e.ncell, e.md_bucket, e.md_cell,
                   e.md_vid,   e.md_w, e.md_w + n, e.md_w + 2 * n, e.ncell, e.bucket_cap,
                   md_nchunk(e.ncell),
-                  e.md_bucket + 2 * (size_t)e.ncell * (size_t)e.bucket_cap, e.md_vid + n};
+                  e.md_bucket + 2 * (size_t)e.ncell * (size_t)e.bucket_cap, (int2*)e.xr};
 }
 
 // Waves that rank one cell's atoms.  The rank of each atom is counted over the whole cell,

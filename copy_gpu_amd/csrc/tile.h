@@ -149,7 +149,7 @@ __device__ inline void md_bin_atom(const MdBins& b, int buf, int s, int v, const
     const int rank = atomicAdd(&b.count[bc], 1);
     if (rank < b.cap) b.bucket[(size_t)bc * b.cap + rank] = s;
     else if (SPILL)
-        b.spill_next[v] = atomicExch(&b.spill[(size_t)c * kSpillChains + rank % kSpillChains], v);
+        b.spill_next[v].x = atomicExch(&b.spill[(size_t)c * kSpillChains + rank % kSpillChains], v);
 }
 
 // ---------------------------------------------------------------- tile order
