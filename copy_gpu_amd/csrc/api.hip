@@ -3,11 +3,10 @@
 // Host orchestration of one force evaluation (the work of Force::Execute,
 // rbmd-gpu src/force/src/lj_cut_coul_kspace_force.cpp:73-78, and of
 // ExecutionNVT::ComputeAllForce, rbmd/framework/run/ExecutionNVT.cpp:185-222):
-//   check -> [bin, scan, scatter, cellsort, list]* -> gather -> [rho, rho_final]
-//   -> pair -> [kforce] -> [ev_final]
-// (* the build kernels run every call but exit at once unless the displacement
-// check or the host asked for a rebuild, so a step needs no host round trip and
-// can be captured in a HIP graph).
+//   check and rho(k) partials -> [bin]* or gather -> [cell sort]* and rho(k) final
+//   -> [list]* and pair -> [kforce] -> [ev_final]
+// (* only if the displacement check or the host asked for a rebuild: the kernels decide on
+// the device, so a step needs no host round trip and can be captured in a HIP graph).
 #include <math.h>
 #include <string.h>
 

@@ -31,7 +31,7 @@ struct LatSumArgs {
 // further at a time (one rounding of about 2^-53 each, far below the phase's own).  The
 // positions come through LDS 256 atoms at a time, as exact box fractions.
 //
-// Bound by FP64 issue: 8 x 4 NC matrix instructions of 64 cycles per wave and stage (64% of
+// Bound by FP64 issue: 8 x 4 NC matrix instructions of 64 cycles per wave and stage (67% of
 // the cycles) and about three sines and cosines per thread.  100,000 ions, |m_d| <= 32 (5.4e10
 // operations): 1.20 ms, 45 TFLOP/s of the 72 that a large FP64 product reaches here; with a
 // sine and cosine per (m, atom) the sums took 29 ms.

@@ -29,7 +29,7 @@ constexpr int min_waves(long)
 
 // The pointee as constant memory (address space 4): uniform reads of it are scalar loads
 // for the whole kernel.  Through a plain pointer the reads that follow a store become
-// vector loads, and the arguments then fill vector registers (109 against 76 in the FP32
+// vector loads, and the arguments then fill vector registers (101 against 78 in the FP32
 // tile pass of a batch, past the occupancy that its LDS stage allows).
 template <class T>
 __device__ inline const T& const_mem(const T* p)

@@ -1100,7 +1100,7 @@ struct RblMean {
 // Deterministic final reduction: pair partials [nb][8] + per-k terms [7][P]
 // + self energy -> ev[10] = {e_lj, e_real, e_self, e_k, W_xx..W_yz} in pinned host memory (a
 // readback then waits for the stream and copies nothing).  One workgroup per
-// output, a fixed order of strided sums, waves and wave sums.  30,000 ions: 5 us, and 29 us
+// output, a fixed order of strided sums, waves and wave sums.  30,000 ions: 4 us, and 17 us
 // with the 52,800 k-vectors of a full Ewald at 6,000; one workgroup for all fifteen columns
 // took 17 and 206 us.
 constexpr int kEvThreads = 1024;

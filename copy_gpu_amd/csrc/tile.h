@@ -284,10 +284,11 @@ __device__ inline int tile_seg(const TileHdr& h, int u)
 // index range mark their rows overflowed.
 //
 // Bound by VALU issue: at 100,000 ions (1,229 candidates a tile, 45 rows) staging takes
-// 6 us, the masks 28 us and the rows about 40 us of a rebuild's tile pass.  Against one wave
-// per row testing every candidate in FP64: 150 -> 125 us (the whole pass, the pair part 48 of
-// it), 26 -> 22 us at 2,000 ions, and 6.6 -> 2.0 ms where the tile is staged in blocks (1,000
-// ions in a box of one cell, 27,000 candidates).
+// 6 us, the masks 28 us and the rows about 40 us of a rebuild's tile pass, at 0.89 vector
+// instructions per CU cycle.  Against one wave per row testing every candidate in FP64: 163 ->
+// 132 us (the whole pass, the pair part 47 of it), 27 -> 21 us at 2,000 ions; where the tile is
+// staged in blocks (1,000 ions in a box of one cell, 27,000 candidates) 6.6 ms -> 135 us,
+// with the tile split among 62 workgroups instead of four.
 //
 // Row layout (uint16 tile-local indices, cap slots per home atom): the LJ-range
 // entries (d2 < r_in^2) first, then the others, then one sentinel slot holding
