@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void k_ewald_final(RhoFinalArgs<double> A,
         const double gy = cl & 2 ? -1.0 : 1.0, gz = cl & 1 ? -1.0 : 1.0;
         double re, im;
         lat_rho(t, gy, gz, &re, &im);
-        const KCoef<double> kc = rho_final_emit(A, k, re, im);
+        const KCoef<double> kc = rho_final_emit<double, false>(A, k, re, im);
         D[0] += kc.B;
         D[6] -= gy * kc.B;
         D[5] -= gz * kc.B;

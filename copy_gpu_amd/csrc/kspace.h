@@ -222,7 +222,8 @@ __device__ inline KCoef<T> rho_terms(const Box& box, double alpha, double qqr2e,
     return kc;
 }
 
-template <typename T>
+// STORE: the coefficients too, for the k-space force of single k-vectors.
+template <typename T, bool STORE = true>
 __device__ inline KCoef<T> rho_final_emit(const RhoFinalArgs<T>& A, int k, double re, double im)
 {
     A.rho[2 * k] = re;
@@ -230,7 +231,7 @@ __device__ inline KCoef<T> rho_final_emit(const RhoFinalArgs<T>& A, int k, doubl
     double ev[7];
     const KCoef<T> kc =
         rho_terms<T>(A.box, A.alpha, A.qqr2e, A.km + 3 * (size_t)k, A.kw[k], re, im, ev);
-    A.coef[k] = kc;
+    if (STORE) A.coef[k] = kc;
     // one column per term: a reduction reads its column alone (rows of seven cost each of the
     // seven sums the whole array through one CU, 29 us for 52,800 k-vectors)
     for (int c = 0; c < 7; ++c) A.kev[(size_t)c * A.P + k] = ev[c];
