@@ -43,13 +43,14 @@ def test_forces_against_oracle(n, P):
     assert np.abs(out.T - Fk).max() <= 1e-6 * term + 2.4e-7 * np.abs(F0).max()
 
 
-def test_batch_and_single_run_same_bits(gpu):
-    """Six replicas of 3,000 ions fill more than one workgroup per CU (scalar loads); one alone
-    does not (LDS stage)."""
+@pytest.mark.parametrize("R", [2, 6])
+def test_batch_and_single_run_same_bits(gpu, R):
+    """Six replicas of 3,000 ions fill more than one workgroup per CU (scalar loads); two, or one
+    alone, do not (LDS stage).  First with 100 k-vectors, which none stages, then with 200."""
     from copy_gpu_amd import ForceConfig, LJCutCoulKspaceForce, systems
     from copy_gpu_amd.batch import ReplicaBatch
 
-    n, P, R = 3000, 200, 6
+    n, P = 3000, 200
     x, y, z, q, L = systems.random_ions(n, 0.3, 0.8, seed=21)
     v = systems.velocities(n, 1.0, seed=21)
     cfg = ForceConfig(box_len=(L,) * 3, cut_off=2.5, coulomb_cut=5.0, alpha=0.5, skin=0.3,
@@ -62,12 +63,14 @@ def test_batch_and_single_run_same_bits(gpu):
         st = [_dev(a) for a in (x, y, z, *v)] + \
             [torch.zeros(n, device="cuda") for _ in range(3)] + \
             [torch.zeros(3 * n, device="cuda", dtype=torch.int32)]
-        f.sample_kvectors(P, 5, 0)
-        f.Execute(*st[:3], *st[6:9])
         states.append(st)
-    b.md_run([tuple(st) for st in states[:R]], dt=0.002, nsteps=6, seeds=[5] * R, step0=1)
-    st = states[R]
-    single.md_run(*st[:9], dt=0.002, nsteps=6, seed=5, step0=1, img=st[9])
+    for P, step0 in ((100, 1), (200, 7)):
+        for f, st in zip([*b.replicas, single], states):
+            f.sample_kvectors(P, 5, 0)
+            f.Execute(*st[:3], *st[6:9])
+        b.md_run([tuple(st) for st in states[:R]], dt=0.002, nsteps=6, seeds=[5] * R, step0=step0)
+        st = states[R]
+        single.md_run(*st[:9], dt=0.002, nsteps=6, seed=5, step0=step0, img=st[9])
     torch.cuda.synchronize()
     for s in states[:R]:
         for a, c in zip(s, st):
