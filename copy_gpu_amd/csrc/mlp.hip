@@ -49,20 +49,19 @@ __device__ inline uint16_t f2bf(float f)
 
 // silu(x) = x / (1 + e^-x) and its derivative from one reciprocal: v_rcp_f32 with a Newton
 // step, and the quotient corrected by its residual, 8 instructions for the 22 of two IEEE
-// divisions.  e^-x is 2^(p + r), p = -x log2 e and r the rest of that product, with |x| bounded
-// by 87 so that neither it nor the denominator leaves the normal range: above, the quotient is
-// x, and below -87 both values are set to 0, which they are to 1.5e-36 (x / (1 + e^87) would
-// grow with x again).
+// divisions.  e^-x is 2^(p + r), p = -x log2 e and r the rest of that product, with x held to
+// -88.5 .. 87 there so that neither it nor the denominator leaves the finite range: above 87 the
+// quotient is x, and where e^-x passes 2^126 (x < -87.3) v_rcp_f32 gives 0, as it does for every
+// reciprocal below the normal range, so silu and its derivative are 0, which they are to 1e-36.
 __device__ inline float silu_d(float x, float* d)
 {
     constexpr float kLog2e = 1.44269504f, kLog2eLo = 1.92596299e-8f, kLn2 = 0.693147181f;
-    const float n = __builtin_amdgcn_fmed3f(-x, -87.0f, 87.0f);
+    const float n = __builtin_amdgcn_fmed3f(-x, -87.0f, 88.5f);
     const float p = n * kLog2e, r = fmaf(n, kLog2eLo, fmaf(n, kLog2e, -p));
     const float q = __builtin_amdgcn_exp2f(p);
     const float e = 1.0f + fmaf(q, r * kLn2, q);
     float s = __builtin_amdgcn_rcpf(e);
     s = fmaf(fmaf(-e, s, 1.0f), s, s);
-    s = x < -87.0f ? 0.0f : s;
     const float a = x * s;
     *d = s * (1.0f + x * (1.0f - s));
     return fabsf(x) < 1e30f ? fmaf(fmaf(-e, a, x), s, a) : a;
